@@ -19,6 +19,13 @@
 // Every row is summed in an order fixed by the matrix alone, so results are
 // identical from run to run.  Replaces csr_spmv_* (SpMV_kernel.cu:81-403) for
 // the tuned solution.
+//
+// A PageRank iteration over the plain in-CSR is the same reduction without
+// values (k_pr_merge): the tile's row sums go to LDS, the epilogue of its rows
+// runs coalesced, and the last workgroup finishes the rows that cross tiles
+// and applies the stop rule, so an iteration is one launch.  It replaces
+// pagerank_* (pagerank_kernel.cu:95-601) on graphs below the binned layout's
+// size.
 
 #include <algorithm>
 #include <vector>
@@ -29,17 +36,13 @@ namespace smdp {
 namespace {
 
 constexpr int kMpNT = 256;                // threads per workgroup
-#ifndef SMDP_MERGE_ITEMS
-#define SMDP_MERGE_ITEMS 16
-#endif
-constexpr int kMpT = SMDP_MERGE_ITEMS;    // merge items per thread
-constexpr int kMpItems = kMpNT * kMpT;    // merge items per tile
-
-#ifndef SMDP_MERGE_RELABEL
-#define SMDP_MERGE_RELABEL 1
-#endif
+// Merge items per thread: kMpBig where the tiles fill the device many times
+// over, kMpSmall where they would not (see items_per_thread).
+constexpr int kMpBig = 16;
+constexpr int kMpSmall = 4;
 
 struct MergePlan {
+  int32_t items = 0;             // merge items per tile
   int32_t* tstart = nullptr;     // ntiles + 1: row ends before each tile's first item
   int32_t* pcol = nullptr;       // m: the columns renumbered by falling in-degree (ties by id)
   int32_t* perm = nullptr;       // n: renumbered column -> original column
@@ -49,6 +52,7 @@ struct MergePlan {
   int32_t* carry_row = nullptr;  // per tile: that row
   float2* head = nullptr;        // per tile: its part of a row begun in an earlier tile and ended in it
   int32_t* head_row = nullptr;   // per tile: that row, or -1
+  double2* part = nullptr;       // PageRank, per tile: (residual, dangling)
   int32_t ntiles = 0;
   int32_t n = -1;
   int32_t m = -1;
@@ -69,6 +73,16 @@ struct MArgs {
   int32_t n, m, ntiles;
 };
 
+// Items per thread of a matrix with `total` = n + m merge items.  A tile of
+// kMpSmall * 256 items has a quarter of the serial work of a kMpBig one but
+// pays the tile's fixed steps four times as often: SpMV on 900K items (220 or
+// 880 tiles on 256 CUs) took 87.8 us a call with kMpBig and 83.7 with kMpSmall;
+// on 17.8M items kMpBig is the faster (0.102 against 0.136 ms).  The line is
+// two kMpBig tiles per CU.
+int items_per_thread(int64_t total, int cus) {
+  return total <= (int64_t)cus * kMpNT * kMpBig * 2 ? kMpSmall : kMpBig;
+}
+
 // Number of row ends among the first d merge items: the smallest i with
 // end(i) > d - i - 1, searched in [max(0, d - nz), min(d, nr)].
 template <typename End>
@@ -84,15 +98,83 @@ __device__ __forceinline__ int64_t merge_search(End end, int64_t d, int64_t nr, 
 }
 
 __global__ void k_merge_starts(const int32_t* __restrict__ row, int32_t n, int32_t m, int32_t ntiles,
-                               int32_t* tstart) {
+                               int32_t items, int32_t* tstart) {
   const int64_t total = (int64_t)n + m;
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t <= ntiles; t += gridDim.x * blockDim.x) {
-    const int64_t d = (int64_t)t * kMpItems < total ? (int64_t)t * kMpItems : total;
+    const int64_t d = (int64_t)t * items < total ? (int64_t)t * items : total;
     tstart[t] = (int32_t)merge_search([&](int64_t i) { return (int64_t)row[i + 1]; }, d, n, m);
   }
 }
 
+// Inclusive segmented scan of the threads' open sums: every thread gets the
+// sum of its row's partials (rows are the keys, which do not decrease from
+// thread to thread, so the threads ending inside one row are consecutive)
+// from the first of those threads up to itself: six shuffle steps in the
+// wave, then the tails of at most three earlier waves.  The combination order
+// is fixed.  All threads; the three arrays hold one entry per wave.
+__device__ __forceinline__ CSum open_row_scan(int key, CSum sc, int32_t* s_hk, int32_t* s_tk, float2* s_tv) {
+  const int lane = lane_id(), wave = threadIdx.x / SMDP_WAVE;
+#pragma unroll
+  for (int d = 1; d < SMDP_WAVE; d <<= 1) {
+    const int k2 = __shfl_up(key, d);
+    CSum o;
+    o.s = __shfl_up(sc.s, d);
+    o.c = __shfl_up(sc.c, d);
+    if (lane >= d && k2 == key) {
+      o.merge(sc);
+      sc = o;
+    }
+  }
+  if (lane == 0) s_hk[wave] = key;
+  if (lane == SMDP_WAVE - 1) {
+    s_tk[wave] = key;
+    s_tv[wave] = make_float2(sc.s, sc.c);
+  }
+  __syncthreads();
+  if (key == s_hk[wave]) {
+    int v = wave;
+    while (v > 0 && s_tk[v - 1] == key) {
+      --v;
+      if (s_hk[v] != key) break;
+    }
+    if (v < wave) {
+      CSum pre;
+      for (int u = v; u < wave; ++u) {
+        CSum o;
+        o.s = s_tv[u].x;
+        o.c = s_tv[u].y;
+        pre.merge(o);
+      }
+      pre.merge(sc);
+      sc = pre;
+    }
+  }
+  return sc;
+}
+
+// Sum of a row that began before tile t and ends in it: the partials of the
+// tiles it crosses, merged in tile order, then tile t's part.
+__device__ __forceinline__ CSum crossing_row(const float2* carry, const int32_t* carry_row, const float2* head, int t,
+                                             int r) {
+  int k = t;
+  while (k > 0 && carry_row[k - 1] == r) --k;
+  CSum tot;
+  for (int q = k; q < t; ++q) {
+    CSum o;
+    o.s = carry[q].x;
+    o.c = carry[q].y;
+    tot.merge(o);
+  }
+  CSum h;
+  h.s = head[t].x;
+  h.c = head[t].y;
+  tot.merge(h);
+  return tot;
+}
+
+template <int kMpT>
 __global__ __launch_bounds__(kMpNT) void k_spmv_merge(MArgs a) {
+  constexpr int kMpItems = kMpNT * kMpT;
   // The tile's nr row ends and nz nonzeros fill its kMpItems merge items, so
   // one array holds both: slot k < nr the end of row i0 + k (in tile nonzero
   // positions, as int bits in .x), slot nr + j the product of nonzero j and
@@ -197,49 +279,7 @@ __global__ __launch_bounds__(kMpNT) void k_spmv_merge(MArgs a) {
       ++zi;
     }
   }
-  // The open rows (keys) do not decrease from thread to thread, so the
-  // threads ending inside one row are consecutive.  An inclusive segmented
-  // scan gives every thread the sum of its row's partials from the first of
-  // those threads up to itself: six shuffle steps in the wave, then the tails
-  // of at most three earlier waves.  The combination order is fixed.
-  const int key = ri;
-  const int lane = lane_id(), wave = tid / SMDP_WAVE;
-  CSum sc = acc;
-#pragma unroll
-  for (int d = 1; d < SMDP_WAVE; d <<= 1) {
-    const int k2 = __shfl_up(key, d);
-    CSum o;
-    o.s = __shfl_up(sc.s, d);
-    o.c = __shfl_up(sc.c, d);
-    if (lane >= d && k2 == key) {
-      o.merge(sc);
-      sc = o;
-    }
-  }
-  if (lane == 0) s_hk[wave] = key;
-  if (lane == SMDP_WAVE - 1) {
-    s_tk[wave] = key;
-    s_tv[wave] = make_float2(sc.s, sc.c);
-  }
-  __syncthreads();
-  if (key == s_hk[wave]) {
-    int v = wave;
-    while (v > 0 && s_tk[v - 1] == key) {
-      --v;
-      if (s_hk[v] != key) break;
-    }
-    if (v < wave) {
-      CSum pre;
-      for (int u = v; u < wave; ++u) {
-        CSum o;
-        o.s = s_tv[u].x;
-        o.c = s_tv[u].y;
-        pre.merge(o);
-      }
-      pre.merge(sc);
-      sc = pre;
-    }
-  }
+  const CSum sc = open_row_scan(ri, acc, s_hk, s_tk, s_tv);
   s_cs[tid] = make_float2(sc.s, sc.c);
   __syncthreads();
 
@@ -278,32 +318,168 @@ __global__ void k_renumber_cols(const int32_t* __restrict__ col, int64_t m, cons
     pcol[e] = inv[col[e]];
 }
 
-// xp[i] = x[perm[i]] for the ncols columns that occur.
+// xp[i] = x[perm[i]] for the ncols columns that occur; workgroup 0 also clears
+// the counters that the product adds to.
 __global__ void k_permute_x(const float* __restrict__ x, const int32_t* __restrict__ perm, int32_t ncols,
-                            float* __restrict__ xp) {
+                            float* __restrict__ xp, Counters* cnt) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ncols; i += gridDim.x * blockDim.x) xp[i] = x[perm[i]];
+  if (blockIdx.x == 0) {
+    unsigned long long* c = reinterpret_cast<unsigned long long*>(cnt);
+    for (int i = threadIdx.x; i < (int)(kCntParts * sizeof(Counters) / 8); i += blockDim.x) c[i] = 0;
+  }
 }
 
-// Rows that began in an earlier tile: the partials of the tiles they cross,
-// merged in tile order, then the part of the tile where they end.
+// Rows that began in an earlier tile.
 __global__ void k_merge_fixup(MArgs a) {
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.ntiles; t += gridDim.x * blockDim.x) {
     const int r = a.head_row[t];
-    if (r < 0) continue;
-    int k = t;
-    while (k > 0 && a.carry_row[k - 1] == r) --k;
-    CSum tot;
-    for (int q = k; q < t; ++q) {
-      CSum o;
-      o.s = a.carry[q].x;
-      o.c = a.carry[q].y;
-      tot.merge(o);
+    if (r >= 0) a.y[r] = crossing_row(a.carry, a.carry_row, a.head, t, r).value();
+  }
+}
+
+// One PageRank iteration: tiles of the merged sequence of the in-CSR's row
+// ends and arcs, grid-stride over the launch (the ticket that ends an
+// iteration is one address, so the launch is held to a few workgroups per
+// CU).  The tile's arcs gather their sources' contributions; rows' sums are
+// collected in LDS and their epilogue (rank, contribution, FP64 residual and
+// dangling mass) runs one row per thread with the old ranks and degrees
+// loaded at the tile's start.
+//
+// What bounds it below 2^20 arcs is the chain of one tile (row ends, columns,
+// gathers, walk, scan, epilogue) and the launch, not bytes: 262K arcs and 16K
+// rows take about 10 us an iteration.  The row-tile kernel it replaces took
+// 157 us there: 64 tiles of 256 rows on 64 of the 256 CUs, with each row of
+// 64 or more arcs summed by one wave after another.  A drop-in PageRank of
+// RMAT-14 went from 2.55 to 0.47 ms.
+template <int kMpT>
+__global__ __launch_bounds__(kMpNT) void k_pr_merge(RArgs a, MArgs p, int k) {
+  if (a.st->done) return;
+  constexpr int kMpItems = kMpNT * kMpT;
+  __shared__ int32_t s_item[kMpItems];  // slots < nr: row ends; then the arcs' contributions (float bits)
+  __shared__ float s_sum[kMpItems];     // row sums of the tile
+  __shared__ float2 s_cs[kMpNT];
+  __shared__ int32_t s_hk[kMpNT / SMDP_WAVE], s_tk[kMpNT / SMDP_WAVE];
+  __shared__ float2 s_tv[kMpNT / SMDP_WAVE];
+  __shared__ double2 s_red2[kMpNT / SMDP_WAVE];
+  __shared__ int s_last;
+  const float base = iteration_base(a, k);
+  const int tid = threadIdx.x;
+  const int64_t dn = (int64_t)p.n + p.m;
+  unsigned long long edges = 0, rows = 0;
+  for (int t = blockIdx.x; t < p.ntiles; t += gridDim.x) {
+    const int64_t d0 = (int64_t)t * kMpItems;
+    const int64_t d1 = d0 + kMpItems < dn ? d0 + kMpItems : dn;
+    const int i0 = p.tstart[t], i1 = p.tstart[t + 1];
+    const int j0 = (int)(d0 - i0), j1 = (int)(d1 - i1);
+    const int nr = i1 - i0, nz = j1 - j0;
+    const bool mid_row = i0 < p.n && a.row[i0] < j0;
+    edges += nz;
+    rows += nr;
+    if (tid == 0) p.head_row[t] = (mid_row && nr > 0) ? i0 : -1;
+    float rold[kMpT];
+    int od[kMpT];
+    // every load at a clamped position, issued before the first use
+    if (nr > 0) {
+      int re[kMpT];
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) {
+        const int q = i0 + min(tid + u * kMpNT, nr - 1);
+        re[u] = a.row[q + 1];
+        rold[u] = a.rold[q];
+        od[u] = a.outdeg[q];
+      }
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) {
+        const int q = tid + u * kMpNT;
+        if (q < nr) s_item[q] = re[u] - j0;
+      }
     }
-    CSum h;
-    h.s = a.head[t].x;
-    h.c = a.head[t].y;
-    tot.merge(h);
-    a.y[r] = tot.value();
+    if (nz > 0) {
+      int c[kMpT];
+      float xv[kMpT];
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) c[u] = a.col[j0 + min(tid + u * kMpNT, nz - 1)];
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) xv[u] = a.x[c[u]];
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) {
+        const int q = tid + u * kMpNT;
+        if (q < nz) s_item[nr + q] = __float_as_int(xv[u]);
+      }
+    }
+    __syncthreads();
+
+    const int dl = min(tid * kMpT, nr + nz), dr = min(dl + kMpT, nr + nz);
+    int ri;
+    {
+      int lo = max(0, dl - nz), hi = min(dl, nr);
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (s_item[mid] <= dl - mid - 1) lo = mid + 1;
+        else hi = mid;
+      }
+      ri = lo;
+    }
+    int zi = dl - ri;
+    const int rfirst = ri;
+    CSum acc, fpart;
+    bool fdone = false;
+    for (int q = dl; q < dr; ++q) {
+      if (ri < nr && s_item[ri] <= zi) {
+        if (ri == rfirst) {
+          fpart = acc;
+          fdone = true;
+        } else {
+          s_sum[ri] = acc.value();
+        }
+        acc = CSum();
+        ++ri;
+      } else {
+        acc.add(__int_as_float(s_item[nr + zi]));
+        ++zi;
+      }
+    }
+    const CSum sc = open_row_scan(ri, acc, s_hk, s_tk, s_tv);
+    s_cs[tid] = make_float2(sc.s, sc.c);
+    __syncthreads();
+    if (fdone) {
+      CSum tot;
+      if (tid > 0) {
+        tot.s = s_cs[tid - 1].x;
+        tot.c = s_cs[tid - 1].y;
+      }
+      tot.merge(fpart);
+      if (rfirst == 0 && mid_row) p.head[t] = make_float2(tot.s, tot.c);
+      else s_sum[rfirst] = tot.value();
+    }
+    if (tid == kMpNT - 1) {
+      p.carry[t] = make_float2(sc.s, sc.c);
+      p.carry_row[t] = i1;
+    }
+    __syncthreads();
+    double res = 0.0, dang = 0.0;
+    if (nr > 0) {
+#pragma unroll
+      for (int u = 0; u < kMpT; ++u) {
+        const int q = tid + u * kMpNT;
+        if (q < nr && !(q == 0 && mid_row)) pr_epilogue(a, i0 + q, s_sum[q], base, rold[u], od[u], res, dang);
+      }
+    }
+    const double2 part = wg_sum2<kMpNT>(make_double2(res, dang), s_red2);
+    if (tid == 0) a.tile_part[t] = part;
+  }
+  if (tid == 0) {
+    Counters* c = cnt_of(a.cnt);
+    if (edges) atomicAdd(&c->edges, edges);
+    if (rows) atomicAdd(&c->verts, rows);
+  }
+  if (arrive_last(a.st, &s_last)) {
+    double res = 0.0, dang = 0.0;
+    for (int t = tid; t < p.ntiles; t += kMpNT) {
+      const int r = p.head_row[t];
+      if (r >= 0) epilogue<true>(a, r, crossing_row(p.carry, p.carry_row, p.head, t, r).value(), base, res, dang);
+    }
+    finish_pass<true>(a, k, make_double2(res, dang), s_red2);
   }
 }
 
@@ -312,7 +488,7 @@ __global__ void k_merge_fixup(MArgs a) {
 void merge_free(void* p) {
   MergePlan* mp = static_cast<MergePlan*>(p);
   if (!mp) return;
-  void* ptrs[] = {mp->tstart, mp->carry, mp->carry_row, mp->head, mp->head_row, mp->pcol, mp->perm, mp->xp};
+  void* ptrs[] = {mp->tstart, mp->carry, mp->carry_row, mp->head, mp->head_row, mp->pcol, mp->perm, mp->xp, mp->part};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   delete mp;
@@ -359,30 +535,40 @@ static int renumber_columns(smdp_graph* g, MergePlan* mp, hipStream_t s) {
   return SMDP_OK;
 }
 
-int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches) {
-  const int64_t total = (int64_t)g->n + g->m;
-  if (g->n <= 0 || total > (int64_t)INT32_MAX - kMpItems) return SMDP_ERR_ARG;
+// The plan of g's CSR in *slot, built on first use; `spmv` adds the column
+// renumbering, else the per-tile partials of PageRank.
+static int ensure_merge(smdp_graph* g, void** slot, bool spmv, hipStream_t s, MergePlan** out) {
   MergePlan* mp = static_cast<MergePlan*>(*slot);
-  if (!mp || mp->n != g->n || mp->m != g->m) {
-    merge_free(mp);
-    *slot = nullptr;
-    mp = new MergePlan();
-    *slot = mp;
-    mp->ntiles = (int32_t)((total + kMpItems - 1) / kMpItems);
-    const int64_t nt = std::max<int64_t>(1, mp->ntiles);
-    SMDP_CHECK(alloc_once(&mp->tstart, nt + 1));
-    SMDP_CHECK(alloc_once(&mp->carry, nt));
-    SMDP_CHECK(alloc_once(&mp->carry_row, nt));
-    SMDP_CHECK(alloc_once(&mp->head, nt));
-    SMDP_CHECK(alloc_once(&mp->head_row, nt));
-    hipLaunchKernelGGL(k_merge_starts, dim3((mp->ntiles + 256) / 256), dim3(256), 0, s, g->row, g->n, g->m,
-                       mp->ntiles, mp->tstart);
-    SMDP_HIP(hipGetLastError());
-    if (SMDP_MERGE_RELABEL && g->m > 0) SMDP_CHECK(renumber_columns(g, mp, s));
-    mp->n = g->n;
-    mp->m = g->m;
+  if (mp && mp->n == g->n && mp->m == g->m) {
+    *out = mp;
+    return SMDP_OK;
   }
-  MArgs a;
+  merge_free(mp);
+  *slot = nullptr;
+  mp = new MergePlan();
+  *slot = mp;
+  const int64_t total = (int64_t)g->n + g->m;
+  mp->items = kMpNT * items_per_thread(total, g->ctx->cus);
+  mp->ntiles = (int32_t)((total + mp->items - 1) / mp->items);
+  const int64_t nt = std::max<int64_t>(1, mp->ntiles);
+  SMDP_CHECK(alloc_once(&mp->tstart, nt + 1));
+  SMDP_CHECK(alloc_once(&mp->carry, nt));
+  SMDP_CHECK(alloc_once(&mp->carry_row, nt));
+  SMDP_CHECK(alloc_once(&mp->head, nt));
+  SMDP_CHECK(alloc_once(&mp->head_row, nt));
+  if (!spmv) SMDP_CHECK(alloc_once(&mp->part, nt));
+  hipLaunchKernelGGL(k_merge_starts, dim3((mp->ntiles + 256) / 256), dim3(256), 0, s, g->row, g->n, g->m, mp->ntiles,
+                     mp->items, mp->tstart);
+  SMDP_HIP(hipGetLastError());
+  if (spmv && g->m > 0) SMDP_CHECK(renumber_columns(g, mp, s));
+  mp->n = g->n;
+  mp->m = g->m;
+  *out = mp;
+  return SMDP_OK;
+}
+
+static MArgs merge_args(smdp_graph* g, const MergePlan* mp) {
+  MArgs a{};
   a.row = g->row;
   a.col = g->col;
   a.val = g->val;
@@ -397,24 +583,55 @@ int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches) {
   a.n = g->n;
   a.m = g->m;
   a.ntiles = mp->ntiles;
-  if (mp->ntiles == 0) return SMDP_OK;
+  return a;
+}
+
+int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches) {
+  if (g->n <= 0 || (int64_t)g->n + g->m > (int64_t)INT32_MAX - kMpNT * kMpBig) return SMDP_ERR_ARG;
+  MergePlan* mp = nullptr;
+  SMDP_CHECK(ensure_merge(g, slot, true, s, &mp));
+  MArgs a = merge_args(g, mp);
   prof_mark(g->ctx, 0);
+  // x in the renumbered order (part of the timed product); without arcs only
+  // the counters are cleared
+  hipLaunchKernelGGL(k_permute_x, dim3(std::max(1, std::min((mp->ncols + 255) / 256, g->ctx->cus * 8))), dim3(256), 0,
+                     s, g->x, mp->perm, mp->ncols, mp->xp, g->cnt);
   if (mp->pcol) {
-    // x in the renumbered order (part of the timed product)
-    hipLaunchKernelGGL(k_permute_x, dim3(std::max(1, std::min((mp->ncols + 255) / 256, g->ctx->cus * 8))), dim3(256),
-                       0, s, g->x, mp->perm, mp->ncols, mp->xp);
     a.col = mp->pcol;
     a.x = mp->xp;
-    ++*launches;
   }
-  hipLaunchKernelGGL(k_spmv_merge, dim3(mp->ntiles), dim3(kMpNT), 0, s, a);
+  if (mp->items == kMpNT * kMpSmall)
+    hipLaunchKernelGGL(k_spmv_merge<kMpSmall>, dim3(mp->ntiles), dim3(kMpNT), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_spmv_merge<kMpBig>, dim3(mp->ntiles), dim3(kMpNT), 0, s, a);
   prof_mark(g->ctx, 0);
   prof_mark(g->ctx, 1);
   hipLaunchKernelGGL(k_merge_fixup, dim3((mp->ntiles + 255) / 256), dim3(256), 0, s, a);
   prof_mark(g->ctx, 1);
-  *launches += 2;
+  *launches += 3;
   SMDP_HIP(hipGetLastError());
   return SMDP_OK;
+}
+
+int merge_pagerank_ensure(smdp_graph* g, void** slot, RArgs* a) {
+  MergePlan* mp = nullptr;
+  SMDP_CHECK(ensure_merge(g, slot, false, g->ctx->stream, &mp));
+  a->tile_part = mp->part;
+  a->ntiles = mp->ntiles;
+  return SMDP_OK;
+}
+
+void merge_pagerank_pass(smdp_graph* g, void* slot, int grid, const RArgs& a, int k, int* launches) {
+  const MergePlan* mp = static_cast<const MergePlan*>(slot);
+  const MArgs p = merge_args(g, mp);
+  const dim3 gd(std::max(1, std::min(grid, mp->ntiles)));
+  prof_mark(g->ctx, 0);
+  if (mp->items == kMpNT * kMpSmall)
+    hipLaunchKernelGGL(k_pr_merge<kMpSmall>, gd, dim3(kMpNT), 0, g->ctx->stream, a, p, k);
+  else
+    hipLaunchKernelGGL(k_pr_merge<kMpBig>, gd, dim3(kMpNT), 0, g->ctx->stream, a, p, k);
+  prof_mark(g->ctx, 0);
+  ++*launches;
 }
 
 }  // namespace smdp

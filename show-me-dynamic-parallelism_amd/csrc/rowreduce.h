@@ -40,16 +40,9 @@ struct RArgs {
   double2* tile_part;              // per tile: (residual, dangling)
   double2* heavy_part;             // grid solution: per heavy-queue entry
   int32_t* hq;                     // grid solution: heavy rows
-  const int32_t* __restrict__ mrows;   // tuned: rows cut into chunks, ascending
-  const int32_t* __restrict__ mfirst;  // tuned: first chunk of each such row (nm+1)
-  float2* mpart;                       // tuned: per chunk (sum, error)
   int32_t n;
   int32_t ntiles;
-  int32_t nm;        // tuned: rows cut into chunks
-  int32_t nchunks;   // tuned: chunks
   int32_t heavy;
-  int32_t split;
-  int32_t chunk;
   float damping;
   float base_rw;     // (1-d) T / N
   double tol_abs;    // stop when residual < tol_abs
@@ -282,6 +275,11 @@ void binned_pass(smdp_ctx* ctx, hipStream_t s, const RArgs& a, const BArgs& b, i
 // Merge-path SpMV (merge.hip): y = A x over g's CSR, values and x, with the
 // per-graph plan kept in *slot (built on first use).
 int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches);
+// PageRank iterations over g's in-CSR by merge-path tiles: the plan in *slot
+// (built on first use; sets the partials of *a that a pass fills), and one
+// iteration on at most `grid` workgroups.
+int merge_pagerank_ensure(smdp_graph* g, void** slot, RArgs* a);
+void merge_pagerank_pass(smdp_graph* g, void* slot, int grid, const RArgs& a, int k, int* launches);
 void merge_free(void* plan);
 
 }  // namespace smdp

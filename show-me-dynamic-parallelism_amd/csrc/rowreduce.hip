@@ -24,9 +24,8 @@
 //    in float every iteration, and reads a "changed" flag back every
 //    iteration (pagerank_wrapper.cu:212-233).
 //  * Heavy rows go to wave / workgroup LDS queues or a grid queue as the
-//    solution says; in the tuned solution rows of at least `split` arcs are
-//    cut into chunks that any workgroup can take, and light rows are summed
-//    from coalesced LDS windows of products.
+//    solution says; the tuned solution works on merge-path tiles (merge.hip)
+//    or, for PageRank on large graphs, on the binned layout (binned.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -167,158 +166,6 @@ __global__ __launch_bounds__(SMDP_WG) void k_rows_grid(RArgs a, int k) {
         extra.y += a.heavy_part[t].y;
       }
     finish_pass<PR>(a, k, extra, s_red2);
-  }
-}
-
-// Tuned solution, one kernel per pass.  Work items, taken from a shared
-// counter: first the chunks of rows with >= split arcs (largest work first),
-// then tiles of SMDP_WG consecutive rows.  In a tile, rows with >= heavy arcs
-// are reduced by their wave; the others are summed by their owner thread from
-// LDS windows that the whole workgroup fills with coalesced loads.  The last
-// workgroup combines the chunk partials of each split row in order, runs
-// their epilogues and finishes the pass.
-template <bool PR>
-__global__ __launch_bounds__(SMDP_WG) void k_rows_tuned(RArgs a, int k) {
-  if (PR && a.st->done) return;
-  const float base = PR ? iteration_base(a, k) : 0.f;
-  const int lane = lane_id();
-  __shared__ int s_item;
-  __shared__ int s_last;
-  __shared__ int s_start[SMDP_WG];
-  __shared__ int s_off[SMDP_WG];
-  __shared__ int s_scan[SMDP_WAVES_PER_WG];
-  __shared__ float s_p[kWin];
-  __shared__ float s_e[PR ? 1 : kWin];
-  __shared__ float2 s_red[SMDP_WAVES_PER_WG];
-  __shared__ double2 s_red2[SMDP_WAVES_PER_WG];
-  unsigned long long edges = 0, rows = 0, pushes = 0;
-  const int nitems = a.nchunks + a.ntiles;
-
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(&a.st->work_next, kGrab);
-    __syncthreads();
-    const int first = s_item;
-    __syncthreads();
-    if (first >= nitems) break;
-    for (int item = first; item < min(first + kGrab, nitems); ++item) {
-    if (item < a.nchunks) {
-      // ---- one chunk of a split row: binary search its row in mfirst
-      int lo = 0, hi = a.nm - 1;
-      while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (a.mfirst[mid] <= item) lo = mid;
-        else hi = mid - 1;
-      }
-      const int r = a.mrows[lo];
-      const int s = a.row[r] + (item - a.mfirst[lo]) * a.chunk;
-      const int e = min(a.row[r + 1], s + a.chunk);
-      CSum h = wg_row<PR>(a, s, e, s_red);
-      if (threadIdx.x == 0) {
-        a.mpart[item] = make_float2(h.s, h.c);
-        edges += e - s;
-      }
-      continue;
-    }
-    // ---- a tile of rows
-    const int tile = item - a.nchunks;
-    const int r = tile * SMDP_WG + (int)threadIdx.x;
-    const bool valid = r < a.n;
-    int s = 0, deg = 0;
-    if (valid) {
-      s = a.row[r];
-      deg = a.row[r + 1] - s;
-      ++rows;
-    }
-    const bool split = deg >= a.split;
-    const bool heavy = !split && deg >= a.heavy;
-    const int ldeg = (valid && !split && !heavy) ? deg : 0;
-    CSum acc;
-    // medium rows: wave-cooperative
-    uint64_t hm = ballot(heavy);
-    pushes += lane == 0 ? __popcll(hm) : 0;
-    while (hm) {
-      const int l = first_lane(hm);
-      hm &= hm - 1;
-      CSum h = wave_row<PR>(a, __shfl(s, l), __shfl(s, l) + __shfl(deg, l));
-      if (lane == l) acc = h;
-    }
-    if (heavy) edges += deg;
-    // light rows: LDS windows of products
-    s_start[threadIdx.x] = s;
-    int tot;
-    const int ex = wg_exclusive_scan(ldeg, s_scan, &tot);
-    s_off[threadIdx.x] = ex;
-    __syncthreads();
-    for (int wb = 0; wb < tot; wb += kWin) {
-      const int wn = min(kWin, tot - wb);
-      {
-        // kWin/SMDP_WG slots per thread: owners found together, then all
-        // column loads, then all gathers, so the gathers overlap.
-        constexpr int K = kWin / SMDP_WG;
-        int j[K], own[K], q[K], c[K];
-#pragma unroll
-        for (int i = 0; i < K; ++i) j[i] = min(wb + (int)threadIdx.x + i * SMDP_WG, wb + wn - 1);
-        tile_owners<K>(s_off, j, own);
-#pragma unroll
-        for (int i = 0; i < K; ++i) q[i] = s_start[own[i]] + (j[i] - s_off[own[i]]);
-#pragma unroll
-        for (int i = 0; i < K; ++i) c[i] = stream_load(a.col + q[i]);
-        if (PR) {
-          float g[K];
-#pragma unroll
-          for (int i = 0; i < K; ++i) g[i] = a.x[c[i]];
-#pragma unroll
-          for (int i = 0; i < K; ++i)
-            if (wb + (int)threadIdx.x + i * SMDP_WG < wb + wn) s_p[j[i] - wb] = g[i];
-        } else {
-#pragma clang fp contract(off)
-          float va[K], xb[K];
-#pragma unroll
-          for (int i = 0; i < K; ++i) {
-            va[i] = stream_load(a.val + q[i]);
-            xb[i] = a.x[c[i]];
-          }
-#pragma unroll
-          for (int i = 0; i < K; ++i) {
-            if (wb + (int)threadIdx.x + i * SMDP_WG < wb + wn) {
-              const float p = va[i] * xb[i];
-              s_p[j[i] - wb] = p;
-              s_e[j[i] - wb] = __builtin_fmaf(va[i], xb[i], -p);
-            }
-          }
-        }
-      }
-      __syncthreads();
-      const int lo_q = max(ex, wb), hi_q = min(ex + ldeg, wb + wn);
-      for (int q = lo_q; q < hi_q; ++q) {
-        acc.add(s_p[q - wb]);
-        if (!PR) acc.c += s_e[q - wb];
-      }
-      __syncthreads();
-    }
-    edges += ldeg;
-    double res = 0.0, dang = 0.0;
-    if (valid && !split) epilogue<PR>(a, r, acc.value(), base, res, dang);
-    if (PR) {
-      double2 t = wg_sum2(make_double2(res, dang), s_red2);
-      if (threadIdx.x == 0) a.tile_part[tile] = t;
-    }
-    }
-  }
-  count_work(a.cnt, edges, rows, pushes);
-  if (arrive_last(a.st, &s_last)) {
-    double res = 0.0, dang = 0.0;
-    for (int i = threadIdx.x; i < a.nm; i += SMDP_WG) {
-      CSum h;
-      for (int c = a.mfirst[i]; c < a.mfirst[i + 1]; ++c) {
-        CSum o;
-        o.s = a.mpart[c].x;
-        o.c = a.mpart[c].y;
-        h.merge(o);
-      }
-      epilogue<PR>(a, a.mrows[i], h.value(), base, res, dang);
-    }
-    finish_pass<PR>(a, k, make_double2(res, dang), s_red2);
   }
 }
 
@@ -569,13 +416,6 @@ __global__ void k_pr_init(float* rank, float* contrib, const int32_t* __restrict
 
 // ---------------------------------------------------------------- host side
 
-struct RowPlan {
-  int32_t split = -1, chunk = -1;
-  int32_t nm = 0, nchunks = 0;
-  int32_t* mrows = nullptr;
-  int32_t* mfirst = nullptr;
-};
-
 }  // namespace smdp
 
 // Extra per-graph buffers of the row-reduce family, kept outside smdp_graph's
@@ -600,19 +440,17 @@ struct BlockPlan {
   float2* bpart = nullptr;
 };
 struct RowBufs {
-  smdp::RowPlan plan;
   BlockPlan blk;
   smdp::RState* st = nullptr;
   double2* tile_part = nullptr;
   double2* heavy_part = nullptr;
   int32_t* hq = nullptr;
-  float2* mpart = nullptr;
-  int64_t mpart_cap = 0;
   float* contrib2 = nullptr;
   int64_t ndang = -1;         // out-degree-0 vertices, counted for out-degrees version ndang_version
   int32_t ndang_version = -1;
   void* binned = nullptr;  // binned layout of PageRank (binned.hip)
   void* merge = nullptr;   // merge-path SpMV plan (merge.hip)
+  void* prmerge = nullptr; // merge-path PageRank plan (merge.hip)
 };
 }  // namespace
 
@@ -627,8 +465,8 @@ static RowBufs* bufs_of(smdp_graph* g) {
 void rowbufs_free(smdp_graph* g) {
   RowBufs* b = static_cast<RowBufs*>(g->rowbufs);
   if (!b) return;
-  void* ptrs[] = {b->st,          b->tile_part,   b->heavy_part,   b->hq,        b->mpart,
-                  b->contrib2,    b->plan.mrows,  b->plan.mfirst,  b->blk.browp, b->blk.bcol,
+  void* ptrs[] = {b->st,          b->tile_part,   b->heavy_part,   b->hq,
+                  b->contrib2,    b->blk.browp,   b->blk.bcol,
                   b->blk.bval,    b->blk.bmega,   b->blk.bmega_off, b->blk.bpart,
                   b->blk.bmega_pos, b->blk.bmega_len, b->blk.bmask, b->blk.bmid, b->blk.bmid_off,
                   b->blk.bmid_pos, b->blk.bmid_len};
@@ -636,38 +474,9 @@ void rowbufs_free(smdp_graph* g) {
     if (p) (void)hipFree(p);
   binned_free(b->binned);
   merge_free(b->merge);
+  merge_free(b->prmerge);
   delete b;
   g->rowbufs = nullptr;
-}
-
-// Rows with >= split arcs and their chunk offsets: a one-time analysis per
-// (graph, split, chunk), kept with the resident graph.
-static int ensure_plan(smdp_graph* g, RowBufs* b, int32_t split, int32_t chunk) {
-  RowPlan& p = b->plan;
-  if (p.split == split && p.chunk == chunk) return SMDP_OK;
-  std::vector<int32_t> row((size_t)g->n + 1);
-  SMDP_HIP(hipMemcpy(row.data(), g->row, sizeof(int32_t) * row.size(), hipMemcpyDeviceToHost));
-  std::vector<int32_t> mrows, mfirst(1, 0);
-  for (int32_t r = 0; r < g->n; ++r) {
-    int32_t d = row[r + 1] - row[r];
-    if (d >= split) {
-      mrows.push_back(r);
-      mfirst.push_back(mfirst.back() + (d + chunk - 1) / chunk);
-    }
-  }
-  if (p.mrows) (void)hipFree(p.mrows);
-  if (p.mfirst) (void)hipFree(p.mfirst);
-  p.mrows = p.mfirst = nullptr;
-  p.nm = (int32_t)mrows.size();
-  p.nchunks = mfirst.back();
-  SMDP_CHECK(alloc_once(&p.mrows, std::max<int64_t>(1, p.nm)));
-  SMDP_CHECK(alloc_once(&p.mfirst, (int64_t)p.nm + 1));
-  if (p.nm) SMDP_HIP(hipMemcpy(p.mrows, mrows.data(), sizeof(int32_t) * p.nm, hipMemcpyHostToDevice));
-  SMDP_HIP(hipMemcpy(p.mfirst, mfirst.data(), sizeof(int32_t) * mfirst.size(), hipMemcpyHostToDevice));
-  SMDP_CHECK(ensure(&b->mpart, &b->mpart_cap, std::max<int32_t>(1, p.nchunks)));
-  p.split = split;
-  p.chunk = chunk;
-  return SMDP_OK;
 }
 
 // The column-blocked layout: one CSR per block of n/kXcd source ids, each
@@ -821,8 +630,7 @@ static void launch_pass(int sol, int grid, hipStream_t s, const RArgs& a, int k,
     case SMDP_SOL_NAIVE: hipLaunchKernelGGL((k_rows_lane<SMDP_SOL_NAIVE, PR>), g, b, 0, s, a, k); break;
     case SMDP_SOL_WAVE: hipLaunchKernelGGL((k_rows_lane<SMDP_SOL_WAVE, PR>), g, b, 0, s, a, k); break;
     case SMDP_SOL_BLOCK: hipLaunchKernelGGL((k_rows_lane<SMDP_SOL_BLOCK, PR>), g, b, 0, s, a, k); break;
-    case SMDP_SOL_GRID: hipLaunchKernelGGL((k_rows_lane<SMDP_SOL_GRID, PR>), g, b, 0, s, a, k); break;
-    default: hipLaunchKernelGGL((k_rows_tuned<PR>), g, b, 0, s, a, k); break;
+    default: hipLaunchKernelGGL((k_rows_lane<SMDP_SOL_GRID, PR>), g, b, 0, s, a, k); break;
   }
   prof_mark(ctx, 0);
   ++*launches;
@@ -842,9 +650,10 @@ static int prepare_args(smdp_graph* g, int app, int sol, RArgs* a, RowBufs** out
   const int ntiles = (g->n + SMDP_WG - 1) / SMDP_WG;
   SMDP_CHECK(alloc_once(&b->st, 1));
   SMDP_CHECK(alloc_once(&b->tile_part, std::max(1, ntiles)));
-  SMDP_CHECK(alloc_once(&b->heavy_part, std::max(1, g->n)));
-  SMDP_CHECK(alloc_once(&b->hq, std::max(1, g->n)));
-  if (sol == SMDP_SOL_TUNED) SMDP_CHECK(ensure_plan(g, b, std::max(p.split_threshold, p.heavy_threshold), p.chunk));
+  if (sol == SMDP_SOL_GRID) {
+    SMDP_CHECK(alloc_once(&b->heavy_part, std::max(1, g->n)));
+    SMDP_CHECK(alloc_once(&b->hq, std::max(1, g->n)));
+  }
   *a = RArgs{};
   a->row = g->row;
   a->col = g->col;
@@ -853,16 +662,9 @@ static int prepare_args(smdp_graph* g, int app, int sol, RArgs* a, RowBufs** out
   a->tile_part = b->tile_part;
   a->heavy_part = b->heavy_part;
   a->hq = b->hq;
-  a->mrows = b->plan.mrows;
-  a->mfirst = b->plan.mfirst;
-  a->mpart = b->mpart;
   a->n = g->n;
   a->ntiles = ntiles;
-  a->nm = sol == SMDP_SOL_TUNED ? b->plan.nm : 0;
-  a->nchunks = sol == SMDP_SOL_TUNED ? b->plan.nchunks : 0;
   a->heavy = p.heavy_threshold;
-  a->split = sol == SMDP_SOL_TUNED ? b->plan.split : INT32_MAX;
-  a->chunk = p.chunk;
   if (use_blocks(p, sol, g->n)) {
     // segments are about 1/kXcd of a row: the heavy degree is scaled down
     const int32_t heavy = std::max(2, p.heavy_threshold / kXcd);
@@ -881,7 +683,6 @@ static int prepare_args(smdp_graph* g, int app, int sol, RArgs* a, RowBufs** out
     a->bmid_off = b->blk.bmid_off;
     a->bmid_pos = b->blk.bmid_pos;
     a->bmid_len = b->blk.bmid_len;
-    a->split = split;
   }
   *out = b;
   return SMDP_OK;
@@ -904,12 +705,16 @@ int run_spmv(smdp_graph* g, int sol, smdp_stats* st) {
   const int grid = grid_size(ctx, params_of(ctx, SMDP_APP_SPMV));
   int launches = 0;
   SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
-  hipLaunchKernelGGL(k_pr_init, dim3(1), dim3(256), 0, s, (float*)nullptr, (float*)nullptr, (const int32_t*)nullptr, 0,
-                     0.f, b->st, 0.0, g->cnt);
-  ++launches;
-  // tuned solution on the plain CSR: merge-path SpMV (merge.hip)
-  if (g->n > 0 && sol == SMDP_SOL_TUNED && !a.browp) SMDP_CHECK(merge_spmv(g, &b->merge, s, &launches));
-  else if (g->n > 0) launch_pass<false>(sol, grid, s, a, 0, &launches, ctx);
+  if (g->n > 0 && sol == SMDP_SOL_TUNED && !a.browp) {
+    // tuned solution on the plain CSR: merge-path SpMV (merge.hip), which
+    // clears the counters itself
+    SMDP_CHECK(merge_spmv(g, &b->merge, s, &launches));
+  } else {
+    hipLaunchKernelGGL(k_pr_init, dim3(1), dim3(256), 0, s, (float*)nullptr, (float*)nullptr, (const int32_t*)nullptr,
+                       0, 0.f, b->st, 0.0, g->cnt);
+    ++launches;
+    if (g->n > 0) launch_pass<false>(sol, grid, s, a, 0, &launches, ctx);
+  }
   SMDP_HIP(hipGetLastError());
   SMDP_HIP(hipEventRecord(ctx->ev_end, s));
   SMDP_HIP(hipEventSynchronize(ctx->ev_end));
@@ -968,6 +773,9 @@ int run_pagerank(smdp_graph* g, const smdp_pr_opts* o, int sol, smdp_stats* st) 
     }
   }
   const bool use_bins = binned && ba.vals != nullptr;
+  // tuned solution on the plain in-CSR: merge-path tiles
+  const bool use_merge = sol == SMDP_SOL_TUNED && !use_bins && !a.browp;
+  if (use_merge) SMDP_CHECK(merge_pagerank_ensure(g, &b->prmerge, &a));
   prof_reset(ctx);
   const int grid = grid_size(ctx, p);
   int launches = 0;
@@ -993,6 +801,7 @@ int run_pagerank(smdp_graph* g, const smdp_pr_opts* o, int sol, smdp_stats* st) 
       a.rold = g->rank[k & 1];
       a.y = g->rank[(k + 1) & 1];
       if (use_bins) binned_pass(ctx, s, a, ba, k, &launches);
+      else if (use_merge) merge_pagerank_pass(g, b->prmerge, grid, a, k, &launches);
       else launch_pass<true>(sol, grid, s, a, k, &launches, ctx);
     }
   };
