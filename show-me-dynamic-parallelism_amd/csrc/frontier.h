@@ -16,9 +16,9 @@ struct Sink {
   WaveOut<kOutCap> wo;
   int32_t* q;
   int32_t* qlen;
-  unsigned long long pushes;
-  unsigned long long tries;  // atomicMin attempts (plain read said "improves")
-  unsigned long long wins;   // atomicMin that lowered the value
+  uint32_t pushes;  // of this launch, as the others
+  uint32_t tries;   // atomicMin attempts (plain read said "improves")
+  uint32_t wins;    // atomicMin that lowered the value
   __device__ __forceinline__ void init(int32_t* lds_region, int32_t* queue, int32_t* counter,
                                        int32_t queue_cap = INT32_MAX) {
     wo.init(lds_region, queue_cap);
@@ -33,34 +33,6 @@ struct Sink {
   }
   __device__ __forceinline__ void flush() { wo.flush(q, qlen); }
 };
-
-// Flushes the wave's queue staging and adds its work counters (one atomic per
-// counter per wave, on the workgroup's counter copy).  Wave-uniform.
-__device__ __forceinline__ void flush_counters(Counters* cnt, unsigned long long edges, unsigned long long verts,
-                                               unsigned long long p0, unsigned long long p1,
-                                               unsigned long long p2, unsigned long long p3,
-                                               Sink& out) {
-  out.flush();
-  unsigned long long tries = wave_sum(out.tries), wins = wave_sum(out.wins);
-  if (lane_id() == 0) {
-    if (tries) atomicAdd(&cnt_of(cnt)->atom_try, tries);
-    if (wins) atomicAdd(&cnt_of(cnt)->atom_win, wins);
-  }
-  edges = wave_sum(edges);
-  verts = wave_sum(verts);
-  p0 = wave_sum(p0);
-  p1 = wave_sum(p1);
-  p2 = wave_sum(p2);
-  p3 = wave_sum(p3);
-  if (lane_id() == 0) {
-    if (edges) atomicAdd(&cnt_of(cnt)->edges, edges);
-    if (verts) atomicAdd(&cnt_of(cnt)->verts, verts);
-    if (p0) atomicAdd(&cnt_of(cnt)->push[0], p0);
-    if (p1) atomicAdd(&cnt_of(cnt)->push[1], p1);
-    if (p2) atomicAdd(&cnt_of(cnt)->push[2], p2);
-    if (p3) atomicAdd(&cnt_of(cnt)->push[3], p3);
-  }
-}
 
 // End of a pass for the whole workgroup: the waves' staged queue entries go
 // out with one atomic for the workgroup (one per wave queued the workgroups'
@@ -125,7 +97,7 @@ __device__ __forceinline__ bool claim_items_wave(int32_t* ctr, int total, int gr
 
 // Word indices of the Counters fields, for wg_add_counters.
 enum : int {
-  kCntEdges = 0, kCntVerts = 1, kCntPush0 = 2, kCntPush3 = 5, kCntRounds = 6, kCntEdges2 = 9,
+  kCntEdges = 0, kCntVerts = 1, kCntPush0 = 2, kCntPush1 = 3, kCntPush2 = 4, kCntPush3 = 5, kCntRounds = 6, kCntEdges2 = 9,
   kCntTries = 10, kCntWins = 11, kCntSkipped = 12
 };
 
@@ -151,6 +123,29 @@ __device__ __forceinline__ void wg_add_counters(Counters* cnt, const unsigned lo
     }
   }
   __syncthreads();
+}
+
+// The same with 32-bit counts of one launch (a launch relaxes fewer than 2^31
+// arcs), summed with DPP steps instead of 64-bit shuffles through LDS; K <=
+// 64, s_red needs SMDP_WAVES_PER_WG * K words.
+template <int K>
+__device__ __forceinline__ void wg_add_counts(Counters* cnt, const uint32_t (&v)[K], const int (&field)[K],
+                                              uint32_t* s_red) {
+  const int wave = threadIdx.x / SMDP_WAVE;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t x = wave_total_dpp(v[k]);
+    if (lane_id() == SMDP_WAVE - 1) s_red[wave * K + k] = x;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if ((int)threadIdx.x == k) {
+      uint32_t sum = 0;
+      for (int w = 0; w < SMDP_WAVES_PER_WG; ++w) sum += s_red[w * K + k];
+      if (sum) atomicAdd(reinterpret_cast<unsigned long long*>(cnt_of(cnt)) + field[k], (unsigned long long)sum);
+    }
+  }
 }
 
 }  // namespace smdp

@@ -35,7 +35,6 @@ namespace smdp {
 constexpr int kWaveQ = 256;   // per-wave LDS queue capacity (SMDP_SOL_WAVE)
 constexpr int kBlockQ = 1024; // per-workgroup LDS queue capacity (SMDP_SOL_BLOCK)
 constexpr int kIlp = 4;       // arcs per thread per step in the tuned kernels
-constexpr int kTileGrab = 1;  // frontier tiles claimed per atomic
 constexpr int kSmallSplit = 32;  // split degree of the tuned solution when the queue is short
 constexpr int kDrainTile = 8;    // grid-queue entries per drain tile (a power of two, at most 64)
 
@@ -63,15 +62,32 @@ struct FArgs {
 };
 
 // Profiling log: round r's queue length and arcs (one atomic per wave).
-__device__ __forceinline__ void log_round(const FArgs& a, int r, int L, unsigned long long wave_arcs) {
+__device__ __forceinline__ void log_round(const FArgs& a, int r, int L, uint32_t arcs) {
   if (!a.rlog || r >= kRoundLogCap) return;
   if (blockIdx.x == 0 && threadIdx.x == 0 && L >= 0) a.rlog[2 * r] = (unsigned long long)L;
-  if (lane_id() == 0 && wave_arcs) atomicAdd(&a.rlog[2 * r + 1], wave_arcs);
+  const uint32_t wave_arcs = wave_total_dpp(arcs);
+  if (lane_id() == SMDP_WAVE - 1 && wave_arcs) atomicAdd(&a.rlog[2 * r + 1], (unsigned long long)wave_arcs);
 }
 
 template <bool BFS>
 __device__ __forceinline__ int arc_weight(const FArgs& a, int e) {
   return BFS ? 1 : stream_load(a.w + e);
+}
+
+// End of a round's kernel for the whole workgroup: its queue entries go out
+// with one atomic and its counters with one each.  Per wave, the same-address
+// atomics of a full grid (8192 waves, about 85M/s on one address) were what a
+// short round waited for.  With the static tiles below, RMAT-16 (18 rounds)
+// went from 34 to 21 us a drain and from 15 to 12 us a tile pass, 0.79 to
+// 0.56 ms a solve.
+__device__ __forceinline__ void end_round(const FArgs& a, Sink& out, uint32_t edges, uint32_t verts, uint32_t pw,
+                                          uint32_t pb, uint32_t pg, uint32_t edges2) {
+  __shared__ int s_n[SMDP_WAVES_PER_WG + 1];
+  __shared__ uint32_t s_red[SMDP_WAVES_PER_WG * 9];
+  wg_flush(out, s_n);
+  const uint32_t v[9] = {edges, verts, out.pushes, pw, pb, pg, edges2, out.tries, out.wins};
+  const int f[9] = {kCntEdges, kCntVerts, kCntPush0, kCntPush1, kCntPush2, kCntPush3, kCntEdges2, kCntTries, kCntWins};
+  wg_add_counts<9>(a.cnt, v, f, s_red);
 }
 
 // Relax one arc with candidate `alt`.  Returns true when this lane lowered
@@ -163,7 +179,7 @@ __device__ __forceinline__ void clear_slot(Ctl* ctl, int r) { ctl_clear(ctl, (r 
 // Wave-cooperative expansion of arcs [s, e) of one vertex with cost du.
 template <bool BFS>
 __device__ __forceinline__ void wave_expand(const FArgs& a, int s, int e, int du, int label,
-                                            unsigned long long& edges, Sink& out) {
+                                            uint32_t& edges, Sink& out) {
   const int lane = lane_id();
   for (int b = s; b < e; b += SMDP_WAVE) {
     int k = b + lane;
@@ -181,7 +197,7 @@ __device__ __forceinline__ void wave_expand(const FArgs& a, int s, int e, int du
 // Workgroup-cooperative expansion (all SMDP_WG threads call it).
 template <bool BFS>
 __device__ __forceinline__ void wg_expand(const FArgs& a, int s, int e, int du, int label,
-                                          unsigned long long& edges, Sink& out) {
+                                          uint32_t& edges, Sink& out) {
   for (int b = s; b < e; b += kIlp * SMDP_WG) {
     int k[kIlp], v[kIlp], alt[kIlp];
 #pragma unroll
@@ -249,7 +265,7 @@ __global__ __launch_bounds__(SMDP_WG) void k_expand_lane(FArgs a, int r) {
     __syncthreads();
   }
 
-  unsigned long long edges = 0, verts = 0, pw = 0, pb = 0, pg = 0;
+  uint32_t edges = 0, verts = 0, pw = 0, pb = 0, pg = 0;
   const int stride = gridDim.x * SMDP_WG;
   for (int base = blockIdx.x * SMDP_WG; base < L; base += stride) {
     const int i = base + (int)threadIdx.x;
@@ -350,9 +366,39 @@ __global__ __launch_bounds__(SMDP_WG) void k_expand_lane(FArgs a, int r) {
       }
     }
   }
-  log_round(a, r, L, wave_sum(edges));
-  flush_counters(a.cnt, edges, verts, out.pushes, pw, pb, pg, out);
+  log_round(a, r, L, edges);
+  end_round(a, out, edges, verts, pw, pb, pg, 0);
 }
+
+// The tiles a workgroup of a round takes.  Up to one tile per workgroup, tile
+// blockIdx.x and no other: a claim is two dependent round trips beyond L2 and
+// finding the eight counters exhausted up to eight more, which a short round
+// spent most of its time on.  Otherwise wave 0 claims one tile at a time.
+struct TileClaims {
+  int32_t* ctr;
+  int total;
+  bool one_each;
+  bool taken = false;
+  uint32_t dead = 0;  // wave 0: exhausted counters
+  __device__ __forceinline__ TileClaims(int32_t* ctr_, int total_)
+      : ctr(ctr_), total(total_), one_each(total_ <= (int)gridDim.x) {}
+  // The next tile, or -1.  All threads; two barriers unless one_each.
+  __device__ __forceinline__ int next(int* s_tile) {
+    if (one_each) {
+      const int t = taken || (int)blockIdx.x >= total ? -1 : (int)blockIdx.x;
+      taken = true;
+      return t;
+    }
+    __syncthreads();  // the last tile was read by every thread
+    if (threadIdx.x < SMDP_WAVE) {
+      int f = 0, e = 0;
+      const bool got = claim_items_wave(ctr, total, 1, dead, &f, &e);
+      if (threadIdx.x == 0) *s_tile = got ? f : -1;
+    }
+    __syncthreads();
+    return *s_tile;
+  }
+};
 
 // One round of the tuned solution: the workgroup takes tiles of SMDP_WG queue
 // entries from a shared counter, stages (first arc, degree, cost) in LDS,
@@ -370,13 +416,13 @@ __global__ __launch_bounds__(SMDP_WG) void k_expand_tile(FArgs a, int r) {
   if (L == 0) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)(r + 1));
   // workgroups past the tile count would only contend for the counter
-  if ((int)blockIdx.x * SMDP_WG * kTileGrab >= L) return;
+  if ((int)blockIdx.x * SMDP_WG >= L) return;
   const int32_t* qin = (r & 1) ? a.q1 : a.q0;
   int32_t* qout = (r & 1) ? a.q0 : a.q1;
   const int label = r + 1;
   const int lane = lane_id();
 
-  __shared__ int s_tile, s_tend;
+  __shared__ int s_tile;
   __shared__ int s_start[SMDP_WG];
   __shared__ int s_du[SMDP_WG];
   __shared__ int s_off[SMDP_WG];
@@ -386,20 +432,10 @@ __global__ __launch_bounds__(SMDP_WG) void k_expand_tile(FArgs a, int r) {
   Sink out;
   out.init(s_out + (threadIdx.x / SMDP_WAVE) * kOutCap, qout, &cout->qlen);
 
-  unsigned long long edges = 0, verts = 0, pg = 0;
+  uint32_t edges = 0, verts = 0, pg = 0;
   const int ntiles = (L + SMDP_WG - 1) / SMDP_WG;
-  int part = 0;  // thread 0: claim cursor
-  for (;;) {
-    if (threadIdx.x == 0) {
-      int f = 0, e = 0;
-      s_tile = claim_items(cin->tiles, ntiles, kTileGrab, part, &f, &e) ? f : -1;
-      s_tend = e;
-    }
-    __syncthreads();
-    const int first = s_tile, tend = s_tend;
-    __syncthreads();
-    if (first < 0) break;
-    for (int tile = first; tile < tend; ++tile) {
+  TileClaims claims(cin->tiles, ntiles);
+  for (int tile; (tile = claims.next(&s_tile)) >= 0;) {
     const int base = tile * SMDP_WG;
     const int i = base + (int)threadIdx.x;
     const bool valid = i < L;
@@ -460,10 +496,9 @@ __global__ __launch_bounds__(SMDP_WG) void k_expand_tile(FArgs a, int r) {
                               out);
     }
     __syncthreads();
-    }
   }
-  log_round(a, r, L, wave_sum(edges));
-  flush_counters(a.cnt, edges, verts, out.pushes, 0, 0, pg, out);
+  log_round(a, r, L, edges);
+  end_round(a, out, edges, verts, 0, 0, pg, 0);
 }
 
 // Phase 2 of the grid solutions: workgroups claim tiles of kDrainTile
@@ -492,16 +527,9 @@ __global__ __launch_bounds__(SMDP_WG) void k_drain(FArgs a, int r) {
   __shared__ int32_t s_pair[SMDP_WAVES_PER_WG * 2 * kIlp * SMDP_WAVE];  // relax_packed
   Sink out;
   out.init(s_out + (threadIdx.x / SMDP_WAVE) * kOutCap, qout, &cout->qlen);
-  unsigned long long edges = 0;
-  int part = 0;  // thread 0: claim cursor
-  for (;;) {
-    if (threadIdx.x == 0) {
-      int f = 0, e = 0;
-      s_tile = claim_items(cin->chunks, ntiles, 1, part, &f, &e) ? f : -1;
-    }
-    __syncthreads();
-    const int tile = s_tile;
-    if (tile < 0) break;
+  uint32_t edges = 0;
+  TileClaims claims(cin->chunks, ntiles);
+  for (int tile; (tile = claims.next(&s_tile)) >= 0;) {
     if (threadIdx.x < SMDP_WAVE) {
       const int idx = tile * ept + (int)threadIdx.x;
       int len = 0, st = 0, du = 0;
@@ -549,10 +577,8 @@ __global__ __launch_bounds__(SMDP_WG) void k_drain(FArgs a, int r) {
     }
     __syncthreads();
   }
-  log_round(a, r, -1, wave_sum(edges));
-  flush_counters(a.cnt, edges, 0, out.pushes, 0, 0, 0, out);
-  unsigned long long e2 = wave_sum(edges);
-  if (lane_id() == 0 && e2) atomicAdd(&cnt_of(a.cnt)->edges2, e2);
+  log_round(a, r, -1, edges);
+  end_round(a, out, edges, 0, 0, 0, 0, edges);
 }
 
 // Out-arcs of reached vertices (the GTEPS numerator).
@@ -739,25 +765,25 @@ static int ensure_relabel(smdp_graph* g, Relabel** out) {
   return SMDP_OK;
 }
 
-// Bit v of words[v / 32] set when row v has arcs.
+// Bit v of words[v / 32] set when row v has arcs.  A wave tests 64 vertices
+// with coalesced loads and stores the two words of its ballot (a thread per
+// word read its 33 offsets one after another: 8 us for 16K vertices).
 __global__ void k_hasout(const int32_t* __restrict__ row, int32_t n, uint32_t* words) {
-  const int32_t nw = (n + 31) / 32;
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nw; i += gridDim.x * blockDim.x) {
-    uint32_t b = 0;
-    for (int k = 0; k < 32; ++k) {
-      const int32_t v = i * 32 + k;
-      if (v < n && row[v + 1] > row[v]) b |= 1u << k;
-    }
-    words[i] = b;
+  const int64_t nw = ((int64_t)n + 31) / 32;
+  for (int64_t v0 = (int64_t)blockIdx.x * blockDim.x; v0 < n; v0 += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t v = v0 + threadIdx.x;
+    const uint64_t b = ballot(v < n && row[v + 1] > row[v]);
+    if ((threadIdx.x & 31) == 0 && v / 32 < nw) words[v / 32] = (uint32_t)(b >> (threadIdx.x & 32));
   }
 }
+
+static unsigned hasout_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 4096)); }
 
 int build_hasout(smdp_graph* g, const int32_t* row, uint32_t** out) {
   if (*out) return SMDP_OK;
   const int64_t nw = std::max<int64_t>(1, ((int64_t)g->n + 31) / 32);
   SMDP_CHECK(alloc_once(out, nw));
-  hipLaunchKernelGGL(k_hasout, dim3((unsigned)std::min<int64_t>((nw + 255) / 256, 4096)), dim3(256), 0,
-                     g->ctx->stream, row, g->n, *out);
+  hipLaunchKernelGGL(k_hasout, dim3(hasout_grid(g->n)), dim3(256), 0, g->ctx->stream, row, g->n, *out);
   SMDP_HIP(hipGetLastError());
   return SMDP_OK;
 }
@@ -1049,9 +1075,7 @@ int sssp_noalloc(smdp_ctx* ctx, int32_t n, int32_t m, const int32_t* d_row, cons
   if (sol == SMDP_SOL_TUNED) {
     // the has-arcs bits are rebuilt every call (the array keeps the last call's contents)
     g.hasout = reinterpret_cast<uint32_t*>(base + noalloc::kHasout);
-    const int64_t nw = ((int64_t)n + 31) / 32;
-    hipLaunchKernelGGL(k_hasout, dim3((unsigned)std::min<int64_t>((nw + 255) / 256, 4096)), dim3(256), 0, s,
-                       d_row, n, g.hasout);
+    hipLaunchKernelGGL(k_hasout, dim3(hasout_grid(n)), dim3(256), 0, s, d_row, n, g.hasout);
     SMDP_HIP(hipGetLastError());
   }
   // k_init_frontier clears the control blocks and counters and sets stamp; the
