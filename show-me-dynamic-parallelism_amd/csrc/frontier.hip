@@ -28,6 +28,7 @@
 
 #include "device_common.h"
 #include "frontier.h"
+#include "lds_sssp.h"
 #include "smdp_internal.h"
 
 namespace smdp {
@@ -605,6 +606,36 @@ __global__ void k_reached(const int32_t* __restrict__ row, const int32_t* __rest
   if (lane_id() == 0 && acc) atomicAdd(&cnt_of(cnt)->reached, acc);
 }
 
+// A whole solve in one workgroup with its distances in LDS (lds_sssp.h).
+// Writes the distances and every counter copy; done = 0, or minus the result
+// of a solve that did not end (kLds*).
+template <bool BFS>
+__global__ __launch_bounds__(kLdsThreads) void k_lds_solve(LdsGraph g, Counters* cnt) {
+  __shared__ LdsShared sh;
+
+  __shared__ unsigned long long s_tot[4];
+  if (threadIdx.x < 4) s_tot[threadIdx.x] = 0;
+  unsigned long long* c = reinterpret_cast<unsigned long long*>(cnt);
+  for (int i = threadIdx.x; i < (int)(kCntParts * sizeof(Counters) / 8); i += kLdsThreads) c[i] = 0;
+  LdsCount k;
+  LdsSolver<BFS, false> s(sh, g, k, 0, 1);
+  const int rounds = s.solve();
+  __syncthreads();
+  const unsigned long long v[4] = {k.edges, k.verts, k.wins, wave_sum(k.reached)};
+  if (lane_id() == 0)
+    for (int i = 0; i < 4; ++i) atomicAdd(&s_tot[i], v[i]);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    cnt->edges = s_tot[0];
+    cnt->verts = s_tot[1];
+    cnt->push[0] = s_tot[1] ? s_tot[1] - 1 : 0;  // every expanded vertex but the source was activated
+    cnt->atom_try = cnt->atom_win = s_tot[2];
+    cnt->reached = s_tot[3];
+    cnt->rounds = rounds > 0 ? rounds : 0;
+    cnt->done = rounds < 0 ? (unsigned long long)-rounds : 0;
+  }
+}
+
 template <bool BFS>
 static void launch_round(int sol, int grid, hipStream_t st, const FArgs& a, int r, int* launches) {
   dim3 g(grid), b(SMDP_WG);
@@ -852,6 +883,54 @@ static int finish_frontier(smdp_graph* g, const int32_t* row, int32_t inf, bool 
   return SMDP_OK;
 }
 
+// Graphs that one workgroup solves in LDS: all distances fit, and the arcs,
+// read by one CU, cost less than the launches of the rounds they replace.
+// Measured (device time, rounds against LDS): SSSP uniform 1024 x 8 180 / 39
+// us, 16384 x 8 338 / 112, 16384 x 32 498 / 208, 32768 x 16 526 / 257; RMAT-12
+// 230 / 75, RMAT-14 x 16 314 / 200, RMAT-15 x 16 (524K arcs) 393 / 418.  BFS
+// (one pass over the arcs, so fewer rounds to save) 16384 x 8 115 / 65, RMAT-15
+// x 16 123 / 180.  A round cap below what windowed rounds may need keeps the
+// unordered ones.
+constexpr int32_t kLdsMaxArcs = 3 << 17;
+constexpr int32_t kLdsMaxArcsBfs = 3 << 16;
+static bool use_lds(const smdp_params& p, const smdp_graph* g, bool bfs) {
+  return p.layout == SMDP_LAYOUT_AUTO && g->n <= kLdsVerts && g->m <= (bfs ? kLdsMaxArcsBfs : kLdsMaxArcs) &&
+         p.max_rounds >= 2 * g->n + 2;
+}
+
+// Returns kLdsWeight (and leaves the solve to the rounds) when a weight is out
+// of the LDS solve's range.
+static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
+  smdp_ctx* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  SMDP_CHECK(alloc_once(&g->dist, g->n));
+  LdsGraph a{};
+  a.row = g->row;
+  a.col = g->col;
+  a.w = g->w;
+  a.n = g->n;
+  a.src = src;
+  a.out = g->dist;
+  prof_reset(ctx);
+  SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
+  SMDP_CHECK(prof_mark(ctx, 0));
+  if (bfs) hipLaunchKernelGGL(k_lds_solve<true>, dim3(1), dim3(kLdsThreads), 0, s, a, g->cnt);
+  else hipLaunchKernelGGL(k_lds_solve<false>, dim3(1), dim3(kLdsThreads), 0, s, a, g->cnt);
+  SMDP_HIP(hipGetLastError());
+  SMDP_CHECK(prof_mark(ctx, 0));
+  SMDP_HIP(hipMemcpyAsync(ctx->pinned, g->cnt, kCntParts * sizeof(Counters), hipMemcpyDeviceToHost, s));
+  SMDP_HIP(hipEventRecord(ctx->ev_end, s));
+  SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  const int failed = (int)reinterpret_cast<const Counters*>(ctx->pinned)->done;
+  if (failed == -kLdsWeight) return kLdsWeight;
+  if (failed) return SMDP_ERR_OVERFLOW;
+  float ms = 0;
+  SMDP_HIP(hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end));
+  ctx->counters_staged = st != nullptr;
+  return finish_frontier(g, g->row, bfs ? SMDP_BFS_UNDEF : SMDP_SSSP_INF, bfs, false, ms, 1,
+                         ctx->profiling ? 0 : -1, false, st, true);
+}
+
 // Runs SSSP (bfs = false) or BFS from src with the given solution; results stay
 // in g->dist.
 int run_frontier(smdp_graph* g, int32_t src, int sol, bool bfs, smdp_stats* st) {
@@ -865,8 +944,12 @@ int run_frontier(smdp_graph* g, int32_t src, int sol, bool bfs, smdp_stats* st) 
   begin_run(g);
   const smdp_params& p = params_of(ctx, bfs ? SMDP_APP_BFS : SMDP_APP_SSSP);
   const bool tuned = sol == SMDP_SOL_TUNED;
-  SMDP_CHECK(ensure_frontier(g, tuned ? p.chunk : 0));
   const bool relabel = tuned && use_relabel(p, g);
+  if (tuned && !relabel && use_lds(p, g, bfs)) {
+    const int rc = run_lds(g, src, bfs, st);
+    if (rc != kLdsWeight) return rc;
+  }
+  SMDP_CHECK(ensure_frontier(g, tuned ? p.chunk : 0));
   const int32_t* row = g->row;
   const int32_t* col = g->col;
   const int32_t* w = g->w;
