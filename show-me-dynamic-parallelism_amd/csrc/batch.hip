@@ -15,7 +15,10 @@
 // the kernel with workgroup barriers between rounds (no grid-wide
 // synchronisation, no host round trip).  Workgroups take graphs from a
 // counter, largest first.  The launch is captured once in a hipGraph and
-// replayed.
+// replayed.  Distances stay in LDS (lds_sssp.h): a graph of more vertices than
+// one workgroup holds, or of many more arcs than its share of the batch, is
+// solved by a cluster of workgroups.  Graphs beyond a cluster, or with weights
+// outside [0, 2^30), keep their distances in memory (mg_solve).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +29,7 @@
 
 #include "device_common.h"
 #include "grid_barrier.h"
+#include "lds_sssp.h"
 #include "smdp_internal.h"
 
 namespace smdp {
@@ -327,6 +331,15 @@ struct GArgs {
   const int32_t* __restrict__ gbase;
   const int32_t* __restrict__ gsize;
   int32_t* gctl;                     // per group one 32-word line: queue lengths [0..2], arrivals [3], epoch [4]
+  // LDS clusters, described by clusters[]: workgroup b works on citem[cfirst[b]
+  // .. cfirst[b + 1]) (cluster << 8 | rank, clusters rising) before its group.
+  const int32_t* __restrict__ cfirst;
+  const int32_t* __restrict__ citem;
+  const struct MgCluster* __restrict__ clusters;
+  const uint8_t* __restrict__ lds;   // per graph: one workgroup can solve it in LDS
+  uint64_t* cflags;                  // every cluster's barrier flags
+  int32_t ncwg;                      // workgroups with cluster items
+  int32_t ncflags;                   // 64-bit words of cflags
   int32_t nplan;
   int32_t nsmall;
   int32_t ngroups;
@@ -340,12 +353,25 @@ struct GArgs {
   int32_t ng;
 };
 
+// One LDS cluster: its graph and size, and what LdsGraph needs.
+struct MgCluster {
+  int32_t graph, k, block, pad0;
+  uint32_t inv;
+  int32_t pad;
+  int64_t moff;    // first entry of its [k][k] message offsets
+  int64_t msg;     // first message of its buffers (both parities)
+  int64_t mtotal;  // messages of one parity
+  int64_t flags;   // first word of its [2][k][k] flags
+};
+
 constexpr int kMgOut = 256;
 constexpr int kMgGroupLine = 32;      // ints per group control line
 constexpr int kMgMaxGroup = 16;       // workgroups that solve one graph together, at most
 constexpr int kMgSpinLimit = 1 << 21; // polls before a group barrier gives up (about a second)
 
-__global__ __launch_bounds__(SMDP_WG) void k_mg_reset(int32_t* next, Counters* cnt, int32_t* gctl, int32_t ngroups) {
+__global__ __launch_bounds__(SMDP_WG) void k_mg_reset(int32_t* next, Counters* cnt, int32_t* gctl, int32_t ngroups,
+                                                      uint64_t* cflags, int32_t ncflags) {
+  for (int i = threadIdx.x; i < ncflags; i += blockDim.x) cflags[i] = 0;
   if (threadIdx.x == 0) *next = 0;
   unsigned long long* p = reinterpret_cast<unsigned long long*>(cnt);
   for (int i = threadIdx.x; i < (int)(kCntParts * sizeof(Counters) / 8); i += blockDim.x) p[i] = 0;
@@ -548,19 +574,87 @@ __device__ void mg_solve(const GArgs& a, int g, int rank, int k, int32_t* gq, Mg
   __syncthreads();
 }
 
-template <int NT>
-__global__ __launch_bounds__(NT) void k_mg(GArgs a) {
-  __shared__ MgShared<NT> sh;
+// Messages from each workgroup of a cluster to each other one: the arcs from
+// its vertices to theirs (one workgroup per (cluster, sender)), the most a
+// round can send.
+__global__ __launch_bounds__(kMgThreads) void k_mg_pairs(GArgs a, int64_t* count) {
+  __shared__ int32_t s_cnt[kLdsMaxCluster];
+  const int it = a.citem[blockIdx.x];
+  const MgCluster cl = a.clusters[it >> 8];
+  const int rank = it & 255;
+  if (threadIdx.x < kLdsMaxCluster) s_cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int n = a.nv[cl.graph];
+  const int32_t* row = a.row + a.rbase[cl.graph];
+  const int lo = min(n, rank * cl.block), hi = min(n, lo + cl.block);
+  const int s = row[lo], e = row[hi];
+  for (int q = s + (int)threadIdx.x; q < e; q += kMgThreads)
+    atomicAdd(&s_cnt[lds_owner((uint32_t)a.col[q], cl.block, cl.inv)], 1);
+  __syncthreads();
+  if ((int)threadIdx.x < cl.k) count[cl.moff + rank * cl.k + threadIdx.x] = (int)threadIdx.x == rank ? 0 : s_cnt[threadIdx.x];
+}
+
+template <bool CL>
+__device__ __forceinline__ void mg_lds(const GArgs& a, int g, const MgCluster* cl, int rank, const int64_t* moff,
+                                       uint64_t* msg, LdsShared& sh, unsigned long long& edges,
+                                       unsigned long long& verts) {
+  LdsGraph lg{};
+  lg.row = a.row + a.rbase[g];
+  lg.col = a.col;
+  lg.w = a.w;
+  lg.n = a.nv[g];
+  lg.src = a.src[g];
+  lg.out = a.dist + a.vbase[g];
+  if (CL) {
+    lg.block = cl->block;
+    lg.inv = cl->inv;
+    lg.msg = msg + cl->msg;
+    lg.moff = moff + cl->moff;
+    lg.mtotal = cl->mtotal;
+    lg.flags = a.cflags + cl->flags;
+  }
+  LdsCount c;
+  LdsSolver<false, CL> s(sh, lg, c, rank, CL ? cl->k : 1);
+  const int rounds = s.solve();
+  if (threadIdx.x == 0) {
+    // (a failure of any of a cluster's workgroups stays)
+    if (rounds < 0) atomicExch(&a.status[g], rounds);
+    else if (rank == 0) atomicCAS(&a.status[g], 0, rounds);
+  }
+  if (lane_id() == 0) {
+    edges += c.edges;
+    verts += c.verts;
+  }
+  __syncthreads();  // LDS is free for the next graph
+}
+
+// LDS: some of the batch's graphs are solved in LDS (the workgroup then holds
+// a CU's LDS; otherwise two workgroups share a CU).
+template <int NT, bool LDS>
+__global__ __launch_bounds__(NT) void k_mg(GArgs a, const int64_t* moff, uint64_t* msg) {
+  constexpr size_t kRaw = LDS ? sizeof(LdsShared) : sizeof(MgShared<NT>);
+  static_assert(sizeof(MgShared<NT>) <= sizeof(LdsShared), "one block of LDS for both");
+  __shared__ __align__(16) char raw[kRaw];
   __shared__ int s_g;
+  MgShared<NT>& sh = *reinterpret_cast<MgShared<NT>*>(raw);
   unsigned long long edges = 0, verts = 0;
-  // the group this workgroup belongs to, if any (groups come first: their
-  // workgroups are dispatched, and resident, before the others)
+  // The clusters this workgroup belongs to, in the order every workgroup takes
+  // them (the first unfinished one then always has all its workgroups), and
+  // its group.  These workgroups come first: they are dispatched, and
+  // resident, before the others.
+  if (LDS && (int)blockIdx.x < a.ncwg) {
+    for (int i = a.cfirst[blockIdx.x]; i < a.cfirst[blockIdx.x + 1]; ++i) {
+      const int it = a.citem[i];
+      const MgCluster* cl = a.clusters + (it >> 8);
+      mg_lds<true>(a, cl->graph, cl, it & 255, moff, msg, *reinterpret_cast<LdsShared*>(raw), edges, verts);
+    }
+  }
   if ((int)blockIdx.x < a.nplan) {
     const int j = a.plan[blockIdx.x];
-    mg_solve<NT, true>(a, a.ggraph[j], (int)blockIdx.x - a.gbase[j], a.gsize[j], a.gctl + j * kMgGroupLine, sh,
-                       edges, verts);
+    mg_solve<NT, true>(a, a.ggraph[j], (int)blockIdx.x - a.gbase[j], a.gsize[j], a.gctl + j * kMgGroupLine, sh, edges,
+                       verts);
   }
-  // then graphs without a group, one workgroup each, largest first
+  // then graphs without either, one workgroup each, largest first
   for (;;) {
     if (threadIdx.x == 0) {
       const int t = atomicAdd(a.next, 1);
@@ -570,7 +664,10 @@ __global__ __launch_bounds__(NT) void k_mg(GArgs a) {
     const int g = s_g;
     __syncthreads();
     if (g < 0) break;
-    mg_solve<NT, false>(a, g, 0, 1, nullptr, sh, edges, verts);
+    if (LDS && a.lds[g])
+      mg_lds<false>(a, g, nullptr, 0, nullptr, nullptr, *reinterpret_cast<LdsShared*>(raw), edges, verts);
+    else
+      mg_solve<NT, false>(a, g, 0, 1, nullptr, sh, edges, verts);
   }
   edges = wave_sum(edges);
   verts = wave_sum(verts);
@@ -846,6 +943,14 @@ struct smdp_batch {
   int32_t* d_gsize = nullptr;
   int32_t* d_gctl = nullptr;
   int32_t ngroups = 0;
+  int32_t* d_cfirst = nullptr;
+  int32_t* d_citem = nullptr;
+  smdp::MgCluster* d_clusters = nullptr;
+  uint8_t* d_lds = nullptr;
+  uint64_t* d_cflags = nullptr;
+  int64_t* d_moff = nullptr;
+  uint64_t* d_msg = nullptr;
+  std::vector<uint8_t> fit;  // per graph: its weights suit an LDS solve
   smdp::Counters* d_cnt = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -856,39 +961,111 @@ struct smdp_batch {
 
 using namespace smdp;
 
-// Work plan of a batch for parameters p, and its hipGraph (reset + solve),
-// replacing the previous plan.  A workgroup's fair share is the batch's arcs
-// over the grid (p.wg_per_cu workgroups per CU, at most 2); a graph of more
-// than p.group_share percent of one share is solved by a group of ceil(m /
-// share) workgroups (at most kMgMaxGroup), as long as all grouped workgroups
-// can be resident at once; the rest are claimed one per workgroup, largest
-// first.  On the 256-graph batch (69M arcs): 20.9 ms with no groups, 6.7 ms
-// with groups above two shares, 5.4 ms above one; groups of up to 32 changed
-// nothing.
-static int batch_plan(smdp_batch* b, const smdp_params& p) {
-  smdp_ctx* ctx = b->ctx;
+static void batch_plan_free(smdp_batch* b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;
-  for (int32_t** q : {&b->d_order, &b->d_plan, &b->d_ggraph, &b->d_gbase, &b->d_gsize, &b->d_gctl}) {
+  for (int32_t** q : {&b->d_order, &b->d_plan, &b->d_ggraph, &b->d_gbase, &b->d_gsize, &b->d_gctl, &b->d_cfirst, &b->d_citem}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }
+  if (b->d_clusters) (void)hipFree(b->d_clusters);
+  if (b->d_lds) (void)hipFree(b->d_lds);
+  if (b->d_cflags) (void)hipFree(b->d_cflags);
+  if (b->d_moff) (void)hipFree(b->d_moff);
+  if (b->d_msg) (void)hipFree(b->d_msg);
+  b->d_clusters = nullptr;
+  b->d_lds = nullptr;
+  b->d_cflags = nullptr;
+  b->d_moff = nullptr;
+  b->d_msg = nullptr;
+}
+
+// Clusters are worth their exchanges from 4 workgroups on (or where the
+// vertices need more than one), up to one per kClusterArcs arcs; a graph that
+// one workgroup holds is left to it below kClusterMin arcs.  Single graphs, k
+// workgroups, us: 32768 x 16 (1: 286, 2: 373, 4: 286, 8: 311), 32768 x 32
+// (390, 564, 349, 327), 65536 x 8 (2: 431, 4: 335, 8: 347, 16: 447), 65536 x 32
+// (2: 1000, 4: 561, 8: 462, 16: 515).
+constexpr int64_t kClusterArcs = int64_t(1) << 18;
+constexpr int64_t kClusterMin = int64_t(1) << 20;
+
+// Work plan of a batch for parameters p, and its hipGraph (reset + solve),
+// replacing the previous plan.  A workgroup's fair share is the batch's arcs
+// over the grid (p.wg_per_cu workgroups per CU, at most 2).
+// A graph that an LDS solve takes goes to one workgroup, or to a cluster of
+// them, ceil(m / share) within the limits above, when it has more than
+// kLdsVerts vertices or at least kClusterMin arcs.  Of the others, a graph of more than p.group_share percent
+// of one share is solved by a group of ceil(m / share) workgroups (at most
+// kMgMaxGroup).  The workgroups of clusters and groups are resident at once
+// and can belong to several clusters in turn; the rest of the graphs are
+// claimed one per workgroup, largest first.
+// 256 graphs, 85M arcs: 6.8 ms with distances in memory and groups, 0.64 ms in
+// LDS with clusters (0.95 ms when a cluster's messages were placed by one LDS
+// atomic per receiver instead of one per lane).  Groups, 69M arcs: 20.9 ms with
+// none, 6.7 ms above two shares, 5.4 ms above one; up to 32 changed nothing.
+static int batch_plan(smdp_batch* b, const smdp_params& p) {
+  smdp_ctx* ctx = b->ctx;
+  batch_plan_free(b);
   const int32_t ng = b->ng;
   std::vector<int32_t> order(ng);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->m[x] > b->m[y]; });
-  const int grid = std::max(1, std::min<int>(ng, ctx->cus * std::max(1, std::min(2, p.wg_per_cu))));
+  const bool lds = std::any_of(order.begin(), order.end(), [&](int32_t i) {
+    return b->fit[i] && b->nv[i] <= kLdsVerts * kLdsMaxCluster;
+  });
+  const int wgs = ctx->cus * (lds ? 1 : std::max(1, std::min(2, p.wg_per_cu)));
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_mg<kMgThreads>),
-                                                   kMgThreads, 0) != hipSuccess)
-    per_cu = 0;
-  const int resident = std::min(grid, per_cu * ctx->cus);
-  const double share = (double)b->etot / grid * (p.group_share > 0 ? p.group_share : 100) / 100.0;
+  const void* kernel = lds ? reinterpret_cast<const void*>(k_mg<kMgThreads, true>)
+                           : reinterpret_cast<const void*>(k_mg<kMgThreads, false>);
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMgThreads, 0) != hipSuccess) per_cu = 0;
+  const int resident = std::min(wgs, per_cu * ctx->cus);
+  const double share = (double)b->etot / wgs * (p.group_share > 0 ? p.group_share : 100) / 100.0;
   std::vector<int32_t> plan, ggraph, gbase, gsize, small;
+  std::vector<std::vector<int32_t>> items((size_t)std::max(1, resident));  // cluster items of each workgroup
+  std::vector<double> load(items.size(), 0.0);                             // and their arcs
+  std::vector<MgCluster> clusters;
+  std::vector<uint8_t> in_lds((size_t)ng, 0);
+  int64_t nmoff = 0, nflags = 0;
   for (int32_t gi : order) {
-    const int k = (int)std::min<int64_t>(kMgMaxGroup, (int64_t)std::ceil(b->m[gi] / std::max(1.0, share)));
+    const int64_t n = b->nv[gi], m = b->m[gi];
+    if (b->fit[gi] && n <= (int64_t)kLdsVerts * kLdsMaxCluster) {
+      int64_t k = (n + kLdsVerts - 1) / kLdsVerts;
+      if (k > 1 || m >= kClusterMin)
+        k = std::max(k, std::min<int64_t>({(int64_t)kLdsMaxCluster, (int64_t)std::ceil(m / std::max(1.0, share)),
+                                           std::max<int64_t>(4, m / kClusterArcs)}));
+      const int64_t block = ((n + k - 1) / k + 63) / 64 * 64;
+      k = (n + block - 1) / block;
+      if (k >= 2 && k <= resident) {
+        // the least loaded workgroups take it
+        std::vector<int32_t> by(load.size());
+        std::iota(by.begin(), by.end(), 0);
+        std::partial_sort(by.begin(), by.begin() + k, by.end(),
+                          [&](int x, int y) { return load[x] != load[y] ? load[x] < load[y] : x < y; });
+        for (int j = 0; j < k; ++j) {
+          items[(size_t)by[(size_t)j]].push_back((int32_t)clusters.size() << 8 | j);
+          load[(size_t)by[(size_t)j]] += (double)m / k + kClusterArcs;
+        }
+        MgCluster c{};
+        c.graph = gi;
+        c.k = (int32_t)k;
+        c.block = (int32_t)block;
+        c.inv = (uint32_t)(((uint64_t(1) << 32) + block - 1) / block);
+        c.moff = nmoff;
+        c.flags = nflags;
+        nmoff += k * k;
+        nflags += 2 * k * k;
+        clusters.push_back(c);
+        continue;
+      }
+      if (n <= kLdsVerts) {
+        in_lds[gi] = 1;
+        small.push_back(gi);
+        continue;
+      }
+    }
+    const int k = (int)std::min<int64_t>(kMgMaxGroup, (int64_t)std::ceil(m / std::max(1.0, share)));
     if (k >= 2 && (int)plan.size() + k <= resident) {
       ggraph.push_back(gi);
       gbase.push_back((int32_t)plan.size());
@@ -898,6 +1075,14 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
       small.push_back(gi);
     }
   }
+  std::vector<int32_t> cfirst(1, 0), citem;
+  int ncwg = 0;
+  for (size_t i = 0; i < items.size(); ++i) {
+    if (!items[i].empty()) ncwg = (int)i + 1;
+    citem.insert(citem.end(), items[i].begin(), items[i].end());
+    cfirst.push_back((int32_t)citem.size());
+  }
+  const int grid = std::max<int>(1, std::min<int>(wgs, std::max<int>(ncwg, (int)plan.size()) + (int)small.size()));
   int rc = SMDP_OK;
   auto up32 = [&](int32_t** d, const int32_t* h, int64_t cnt) {
     if (rc != SMDP_OK) return;
@@ -912,7 +1097,14 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
   up32(&b->d_gbase, gbase.data(), (int64_t)gbase.size());
   up32(&b->d_gsize, gsize.data(), (int64_t)gsize.size());
   up32(&b->d_gctl, nullptr, (int64_t)ggraph.size() * kMgGroupLine);
+  up32(&b->d_cfirst, cfirst.data(), (int64_t)cfirst.size());
+  up32(&b->d_citem, citem.data(), (int64_t)citem.size());
   if (rc != SMDP_OK) return rc;
+  SMDP_CHECK(alloc_once(&b->d_lds, ng));
+  SMDP_HIP(hipMemcpy(b->d_lds, in_lds.data(), (size_t)ng, hipMemcpyHostToDevice));
+  SMDP_CHECK(alloc_once(&b->d_clusters, std::max<int64_t>(1, (int64_t)clusters.size())));
+  SMDP_CHECK(alloc_once(&b->d_cflags, std::max<int64_t>(1, nflags)));
+  SMDP_CHECK(alloc_once(&b->d_moff, std::max<int64_t>(1, nmoff)));
   GArgs& a = b->args;
   a.row = b->d_row;
   a.col = b->d_col;
@@ -927,6 +1119,13 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
   a.gbase = b->d_gbase;
   a.gsize = b->d_gsize;
   a.gctl = b->d_gctl;
+  a.cfirst = b->d_cfirst;
+  a.citem = b->d_citem;
+  a.clusters = b->d_clusters;
+  a.lds = b->d_lds;
+  a.cflags = b->d_cflags;
+  a.ncwg = ncwg;
+  a.ncflags = (int32_t)nflags;
   a.nplan = (int32_t)plan.size();
   a.nsmall = (int32_t)small.size();
   a.ngroups = b->ngroups;
@@ -939,13 +1138,41 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
   a.cnt = b->d_cnt;
   a.ng = ng;
   b->grid = grid;
+  hipStream_t s = ctx->stream;
+  if (!clusters.empty()) {
+    // message buffers: the arcs between each pair of a cluster's workgroups
+    SMDP_HIP(hipMemcpyAsync(b->d_clusters, clusters.data(), sizeof(MgCluster) * clusters.size(), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_mg_pairs, dim3((unsigned)citem.size()), dim3(kMgThreads), 0, s, b->args, b->d_moff);
+    SMDP_HIP(hipGetLastError());
+    std::vector<int64_t> moff((size_t)nmoff);
+    SMDP_HIP(hipMemcpyAsync(moff.data(), b->d_moff, sizeof(int64_t) * moff.size(), hipMemcpyDeviceToHost, s));
+    SMDP_HIP(hipStreamSynchronize(s));
+    int64_t total = 0;
+    for (MgCluster& c : clusters) {
+      int64_t at = 0;
+      for (int64_t i = c.moff; i < c.moff + (int64_t)c.k * c.k; ++i) {
+        const int64_t cnt = moff[(size_t)i];
+        moff[(size_t)i] = at;
+        at += cnt;
+      }
+      c.mtotal = at;
+      c.msg = total;
+      total += 2 * at;
+    }
+    SMDP_CHECK(alloc_once(&b->d_msg, std::max<int64_t>(1, total)));
+    SMDP_HIP(hipMemcpy(b->d_moff, moff.data(), sizeof(int64_t) * moff.size(), hipMemcpyHostToDevice));
+    SMDP_HIP(hipMemcpy(b->d_clusters, clusters.data(), sizeof(MgCluster) * clusters.size(), hipMemcpyHostToDevice));
+  }
   // Capture reset + solve once; every run replays the graph.  No memset nodes:
   // counters are cleared by a kernel.
-  hipStream_t s = ctx->stream;
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return SMDP_ERR_DEVICE;
-  hipLaunchKernelGGL(k_mg_reset, dim3(1), dim3(256), 0, s, b->d_next, b->d_cnt, b->d_gctl, b->ngroups);
+  hipLaunchKernelGGL(k_mg_reset, dim3(1), dim3(256), 0, s, b->d_next, b->d_cnt, b->d_gctl, b->ngroups, b->d_cflags,
+                     (int32_t)nflags);
   hipLaunchKernelGGL(k_mg_status_clear, dim3(std::max(1, (ng + 255) / 256)), dim3(256), 0, s, b->d_status, ng);
-  hipLaunchKernelGGL(k_mg<kMgThreads>, dim3(b->grid), dim3(kMgThreads), 0, s, b->args);
+  if (lds)
+    hipLaunchKernelGGL((k_mg<kMgThreads, true>), dim3(b->grid), dim3(kMgThreads), 0, s, b->args, b->d_moff, b->d_msg);
+  else
+    hipLaunchKernelGGL((k_mg<kMgThreads, false>), dim3(b->grid), dim3(kMgThreads), 0, s, b->args, b->d_moff, b->d_msg);
   if (hipStreamEndCapture(s, &b->graph) != hipSuccess) return SMDP_ERR_DEVICE;
   if (hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0) != hipSuccess) return SMDP_ERR_DEVICE;
   return SMDP_OK;
@@ -972,11 +1199,9 @@ int smdp_sssp_multi_source(smdp_ctx* ctx, const smdp_csr* h, const int32_t* srcs
 void smdp_batch_destroy(smdp_batch* b) {
   if (!b) return;
   (void)hipSetDevice(b->ctx->device);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  void* ptrs[] = {b->d_row,   b->d_col,   b->d_w,  b->d_rbase, b->d_vbase, b->d_nv,   b->d_src,    b->d_order,
-                  b->d_dist,  b->d_stamp, b->d_qa, b->d_qb,    b->d_next,  b->d_status, b->d_cnt,
-                  b->d_plan,  b->d_ggraph, b->d_gbase, b->d_gsize, b->d_gctl};
+  batch_plan_free(b);
+  void* ptrs[] = {b->d_row, b->d_col,   b->d_w,  b->d_rbase, b->d_vbase,  b->d_nv,  b->d_src,
+                  b->d_dist, b->d_stamp, b->d_qa, b->d_qb,    b->d_next, b->d_status, b->d_cnt};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete b;
@@ -1007,12 +1232,19 @@ int smdp_batch_create(smdp_ctx* ctx, const smdp_csr* graphs, int32_t ng, const i
     etot += c.m;
   }
   if (etot > INT32_MAX) return SMDP_ERR_ARG;
-  std::vector<int32_t> row(rtot), col(std::max<int64_t>(1, etot)), w(std::max<int64_t>(1, etot)), nv(ng), order(ng);
+  std::vector<int32_t> row(rtot), col(std::max<int64_t>(1, etot)), w(std::max<int64_t>(1, etot)), nv(ng);
+  std::vector<uint32_t> wbits(ng);  // per graph: every weight's bits together
   for (int32_t i = 0; i < ng; ++i) {
     const smdp_csr& c = graphs[i];
     for (int32_t v = 0; v <= c.n; ++v) row[rbase[i] + v] = (int32_t)(ebase[i] + c.row[v]);
     std::copy(c.col, c.col + c.m, col.begin() + ebase[i]);
-    std::copy(c.w, c.w + c.m, w.begin() + ebase[i]);
+    int32_t* dw = w.data() + ebase[i];
+    uint32_t all = 0;
+    for (int32_t e = 0; e < c.m; ++e) {
+      dw[e] = c.w[e];
+      all |= (uint32_t)c.w[e];
+    }
+    wbits[i] = all;
     nv[i] = c.n;
   }
   smdp_batch* b = new smdp_batch();
@@ -1022,7 +1254,13 @@ int smdp_batch_create(smdp_ctx* ctx, const smdp_csr* graphs, int32_t ng, const i
   b->vbase = vbase;
   b->etot = etot;
   b->m.resize(ng);
-  for (int32_t i = 0; i < ng; ++i) b->m[i] = graphs[i].m;
+  b->fit.assign((size_t)ng, 0);
+  for (int32_t i = 0; i < ng; ++i) {
+    b->m[i] = graphs[i].m;
+    // an LDS solve takes weights in [0, 2^30); a cluster counts a round's
+    // messages in 24 bits
+    b->fit[i] = wbits[i] < (uint32_t)kLdsWeightLimit && graphs[i].m < (1 << 24);
+  }
   int rc = SMDP_OK;
   auto up32 = [&](int32_t** d, const int32_t* h, int64_t cnt) {
     if (rc != SMDP_OK) return;

@@ -69,7 +69,7 @@ struct LdsGraph {
   int32_t* out;                     // n distances
   // cluster of k workgroups: workgroup i owns vertices [i * block, (i + 1) * block)
   int32_t block;
-  uint32_t inv;                     // ceil(2^32 / block): v / block = v * inv >> 32 for v < 2^20
+  uint32_t inv;                     // ceil(2^32 / block): v * inv >> 32 is v / block or one more
   uint64_t* msg;                    // messages (target << 32 | candidate word), both parities
   const int64_t* moff;              // [k][k]: first message of the pair (sender, receiver), parity 0
   int64_t mtotal;                   // messages of one parity
@@ -91,6 +91,7 @@ struct LdsShared {
   int32_t mn;                            // cluster: smallest distance anywhere
   int32_t mcnt[kLdsMaxCluster];          // cluster: messages queued for each workgroup this round
   int32_t got[kLdsMaxCluster];           // cluster: messages received from each
+  uint64_t* mbase[2][kLdsMaxCluster];    // cluster: message buffers to each, by parity
 };
 static_assert(sizeof(LdsShared) <= 160 * 1024, "the LDS of a CU");
 
@@ -139,6 +140,12 @@ __device__ __forceinline__ uint64_t low_lanes(int cnt) {
 // p[off / 4] with a 32-bit byte offset (scalar base, one vector register).
 __device__ __forceinline__ int load_at(const int32_t* p, uint32_t off) {
   return *reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(p) + off);
+}
+
+// The workgroup of a cluster that owns vertex v < 2^20.
+__device__ __forceinline__ int lds_owner(uint32_t v, int32_t block, uint32_t inv) {
+  const uint32_t d = (uint32_t)(((uint64_t)v * inv) >> 32);
+  return (int)d - (d * (uint32_t)block > v ? 1 : 0);
 }
 
 template <bool BFS, bool CL>
@@ -205,34 +212,33 @@ struct LdsSolver {
     }
 #pragma unroll
     for (int t = 0; t < kLdsIlp; ++t) lower(__builtin_amdgcn_ballot_w64(a[t] < cur[t]) & ok[t], v[t], a[t]);
-    if (CL) {
-#pragma unroll
-      for (int t = 0; t < kLdsIlp; ++t) send(v[t], a[t], ok[t]);
-    }
+    if (CL) send(v, a, ok);
   }
 
-  // Messages of a cluster: candidates for other workgroups' vertices.
-  __device__ __forceinline__ void send(int lv, uint32_t a, uint64_t ok) {
-    // (a candidate at or beyond the unreached word lowers nothing)
-    const bool rem = (uint32_t)lv >= (uint32_t)nl && a < (uint32_t)SMDP_SSSP_INF * 2;
-    uint64_t left = __builtin_amdgcn_ballot_w64(rem) & ok;
-    if (!left) return;
-    const bool mine = __builtin_amdgcn_inverse_ballot_w64(left);
-    if (mine) low = min(low, a);
-    const uint32_t v = (uint32_t)(lv + lo);
-    const int dest = (int)(((uint64_t)v * g.inv) >> 32);
-    while (left) {
-      const int d = __builtin_amdgcn_readlane(dest, first_lane(left));
-      const uint64_t m = __builtin_amdgcn_ballot_w64(dest == d) & left;
-      left &= ~m;
-      int b = 0;
-      if (lane == 0)
-        b = __hip_atomic_fetch_add(&sh.mcnt[d], __popcll(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      b = __builtin_amdgcn_readfirstlane(b);
-      if (__builtin_amdgcn_inverse_ballot_w64(m))
-        __hip_atomic_store(g.msg + parity * g.mtotal + g.moff[rank * k + d] + b + mbcnt(m), (uint64_t)v << 32 | a,
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // Messages of a cluster: candidates for other workgroups' vertices.  Every
+  // lane takes its own place in its receiver's buffer (a loop over the
+  // receivers present, one LDS atomic each, cost 16 of them per 64 arcs in a
+  // cluster of 16).
+  __device__ __forceinline__ void send(const int (&lv)[kLdsIlp], const uint32_t (&a)[kLdsIlp],
+                                       const uint64_t (&ok)[kLdsIlp]) {
+    uint64_t m[kLdsIlp];
+    int at[kLdsIlp], dest[kLdsIlp];
+#pragma unroll
+    for (int t = 0; t < kLdsIlp; ++t) {
+      // (a candidate at or beyond the unreached word lowers nothing)
+      m[t] = __builtin_amdgcn_ballot_w64((uint32_t)lv[t] >= (uint32_t)nl && a[t] < (uint32_t)SMDP_SSSP_INF * 2) & ok[t];
+      dest[t] = at[t] = 0;
+      if (__builtin_amdgcn_inverse_ballot_w64(m[t])) {
+        low = min(low, a[t]);
+        dest[t] = lds_owner((uint32_t)(lv[t] + lo), g.block, g.inv);
+        at[t] = __hip_atomic_fetch_add(&sh.mcnt[dest[t]], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
     }
+#pragma unroll
+    for (int t = 0; t < kLdsIlp; ++t)
+      if (__builtin_amdgcn_inverse_ballot_w64(m[t]))
+        __hip_atomic_store(sh.mbase[parity][dest[t]] + at[t], (uint64_t)(uint32_t)(lv[t] + lo) << 32 | a[t],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
   // Expands the last `cnt` (<= 64) entries of the wave's list of length `n`.
@@ -444,13 +450,17 @@ struct LdsSolver {
     const uint32_t inf = (uint32_t)SMDP_SSSP_INF * 2;
     // whole blocks: the words past nl stay unreached
     for (int i = tid; i < (nl + kLdsBlock - 1) / kLdsBlock * kLdsBlock; i += kLdsThreads) sh.x[i] = inf;
+    if (tid < kLdsMaxCluster) sh.mcnt[tid] = 0;
+    if (CL && tid < k) {
+      sh.mbase[0][tid] = g.msg + g.moff[rank * k + tid];
+      sh.mbase[1][tid] = sh.mbase[0][tid] + g.mtotal;
+    }
     if (tid < 3) {
       sh.smin[tid] = INT32_MAX;
       sh.nchunk[tid] = 0;
       sh.bad[tid] = 0;
     }
     const int win = window(sh.got);
-    if (tid < kLdsMaxCluster) sh.mcnt[tid] = 0;
     __syncthreads();
     if (tid == 0 && (uint32_t)(g.src - lo) < (uint32_t)nl) sh.x[g.src - lo] = 1;  // distance 0, active
     __syncthreads();
