@@ -390,7 +390,9 @@ struct LArgs {
   // the last drain ran, rd[2] set once a layer is empty (done), rd[3] set
   // when a barrier between short layers gave up waiting.
   int32_t* rd;
-  uint32_t* bar;  // flags of k_layer_short's barrier (two parities of 64-bit flags), zeroed before each launch
+  uint32_t* bar;  // flags of k_layer_short's barrier (a line for each parity), zeroed before each launch
+  struct LayerEntry* seg;  // k_layer_short's queue segments: two parities of kLayerWgs, seg_cap entries each
+  int32_t seg_cap;         // min(n, kFlagCount): a segment that overflows ends the short run
 };
 
 constexpr int kLayerIlp = 4;
@@ -499,23 +501,41 @@ __global__ __launch_bounds__(SMDP_WG) void k_layer_count_chunks(LArgs a) {
 // Colour 1 for the vertices without preceding neighbours: the queue of round 0.
 // A vertex that no row lists (no transposed arcs) has nobody to notify and is
 // coloured without being queued; RMAT-23's first layer is mostly such.
+// The queue's counter takes one atomic per kSeedQueue vertices of a workgroup
+// (RMAT-20: 17 us; with one per wave, 8192 of them, 96: the card performs about 85
+// million same-address atomics a second).
+constexpr int kSeedQueue = 2048;
 __global__ __launch_bounds__(SMDP_WG) void k_layer_seed(LArgs a) {
-  __shared__ int32_t s_out[SMDP_WAVES_PER_WG * kCOut];
-  WaveOut<kCOut> out;
-  out.init(s_out + (threadIdx.x / SMDP_WAVE) * kCOut);
+  __shared__ int32_t s_q[kSeedQueue];
+  __shared__ int s_n, s_base;
+  if (threadIdx.x == 0) s_n = 0;
   // colour 1 exists whenever n > 0, even if none of its vertices is queued
   if (blockIdx.x == 0 && threadIdx.x == 0 && a.n > 0) atomicMax(&cnt_of(a.cnt)->rounds, 1ull);
-  for (int base = blockIdx.x * SMDP_WG; base < a.n; base += gridDim.x * SMDP_WG) {
-    const int v = base + (int)threadIdx.x;
-    bool ready = false, queue = false;
-    if (v < a.n) {
-      ready = a.pend[v] == 0;
+  __syncthreads();
+  for (int64_t base = (int64_t)blockIdx.x * SMDP_WG; base < a.n; base += gridDim.x * SMDP_WG) {
+    const int64_t i = base + threadIdx.x;
+    const int v = (int)i;
+    bool queue = false;
+    if (i < a.n) {
+      const bool ready = a.pend[v] == 0;
       a.color[v] = ready ? 1 : 0;
       queue = ready && a.trow[v + 1] > a.trow[v];
     }
-    out.push(queue, v, a.q0, &a.ctl[0].qlen);
+    const uint64_t m = ballot(queue);
+    int at = 0;
+    if (lane_id() == 0 && m) at = atomicAdd(&s_n, __popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at) + mbcnt(m);
+    if (queue) s_q[at] = v;
+    __syncthreads();
+    const int n = s_n;
+    if (n > kSeedQueue - SMDP_WG || base + (int64_t)gridDim.x * SMDP_WG >= a.n) {
+      if (threadIdx.x == 0) s_base = n ? atomicAdd(&a.ctl[0].qlen, n) : 0;
+      __syncthreads();
+      for (int k = threadIdx.x; k < n; k += SMDP_WG) a.q0[s_base + k] = s_q[k];
+      if (threadIdx.x == 0) s_n = 0;
+    }
+    __syncthreads();
   }
-  out.flush(a.q0, &a.ctl[0].qlen);
 }
 
 // Arcs u[t] -> v[t] of the transposed CSR, K per lane (ok[t]: the arc exists;
@@ -604,7 +624,6 @@ constexpr int kShortMinWG = 128;
 // Expands short layer r (L <= kShortL queued vertices) on workgroups
 // 0 .. G-1 of the launch, G = min(workgroups, max(L / kShortPerWG,
 // kShortMinWG)); the others return at once.  s_raw: 3 * kShortL ints.
-template <bool COH>
 __device__ __forceinline__ void short_layer(const LArgs& a, int r, int L, int32_t* s_raw, int* s_scan,
                                             int32_t* s_pack, WaveOut<kCOut>& out, unsigned long long& edges,
                                             unsigned long long& verts, unsigned long long& pushes) {
@@ -622,7 +641,7 @@ __device__ __forceinline__ void short_layer(const LArgs& a, int r, int L, int32_
 #pragma unroll
   for (int k = 0; k < E; ++k) {
     const int i = min((int)threadIdx.x * E + k, L - 1);
-    vv[k] = COH ? __hip_atomic_load(qin + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : qin[i];
+    vv[k] = qin[i];
   }
 #pragma unroll
   for (int k = 0; k < E; ++k) {
@@ -708,7 +727,7 @@ __global__ __launch_bounds__(SMDP_WG) void k_layer_expand(LArgs a) {
   unsigned long long edges = 0, verts = 0, pushes = 0, pg = 0;
 
   if (L <= kShortL) {
-    short_layer<false>(a, r, L, s_raw, s_scan, s_pack, out, edges, verts, pushes);
+    short_layer(a, r, L, s_raw, s_scan, s_pack, out, edges, verts, pushes);
   } else {
   const LayerShape sh = layer_shape(a, L, a.grid);  // launched with a.grid workgroups
   const int ntiles = (L + sh.tile - 1) / sh.tile;
@@ -809,62 +828,135 @@ __global__ __launch_bounds__(SMDP_WG) void k_layer_expand(LArgs a) {
 }
 
 // Runs short layers one after another in one launch: layers rd[1] + 1,
-// rd[1] + 2, ... while they hold at most kShortL vertices, with a flag
-// barrier (below) after each (a layer's queue is complete only when every workgroup
-// has pushed).  Then rd[0] = the first layer not run, for k_layer_expand.
-// RMAT-23 has ~2300 such layers; one expand and one drain launch per layer
-// cost about 18 us, mostly launch and ramp.
-constexpr int kFlagGrid = 64;  // workgroups the flag barrier serves (one flag per lane of a wave)
-static_assert(2 * kFlagGrid * 2 <= kBarLines * 32, "two parities of 64-bit flags fit the barrier lines");
+// rd[1] + 2, ... while they hold at most kShortL vertices.  Then rd[0] = the
+// first layer not run, for k_layer_expand.
+//
+// A short layer is a chain of latencies, not work: the layers of a
+// symmetrised RMAT-20 graph with random priorities hold 500 vertices and
+// 16000 arcs in the mean, one arc per thread of the launch.  So each step of the chain is made
+// to wait for as little as possible:
+// - Workgroup b queues what it releases in a segment of its own (an LDS
+//   counter gives the place), since a shared queue's counter takes one
+//   atomic per wave and the card performs about 85 million same-address
+//   atomics a second: 3 us a layer.
+// - An entry carries the vertex, its first arc, its arc count and its
+//   priority.  The lane that takes an arc off pend[] loads them beside the
+//   atomic, whether or not it turns out to be the last one.
+// - The barrier's flag carries the segment's entry and arc counts, so every
+//   workgroup knows its share of the layer's arcs from the flags alone and
+//   reads only the entries of that share.
+// - The flags of one parity are one 128-byte line, polled by one wave of each
+//   workgroup: a barrier alone takes 0.9 us with 32 workgroups, and 1.9 us
+//   with 64 workgroups and their 64-bit flags in four lines.
+// What is left of a layer (RMAT-20: 4.9 us) is four dependent trips to memory
+// (flag, entries, arcs, pend) and the slowest of the 32 workgroups in them.
+// Fewer arcs per thread beat more loads in flight: 16 workgroups of 1024 took
+// 6.3 ms per colouring of that graph, 32 of 512 6.0, 32 of 1024 5.5.  Only
+// every kLayerStride-th workgroup of the launch takes part: workgroups go to
+// the XCDs in turn, so the run stays on two of them, whose L2s hold the
+// entries, the flags and pend's neighbourhoods (on eight XCDs 5.75 ms, on four
+// 5.5, on one 5.3 to 6.0).  Nothing depends on where they run.
+// Per colouring, before (64 workgroups of 256, one queue) and now, random
+// priorities: RMAT-13 0.98 / 0.60 ms, RMAT-18 4.9 / 2.9, RMAT-20 9.7 / 5.4,
+// RMAT-23 32.4 / 24.8.
+constexpr int kLayerWgs = 32;
+constexpr int kLayerStride = 4;
+constexpr int kLayerThreads = 1024;
+constexpr int kLayerWaves = kLayerThreads / SMDP_WAVE;
+constexpr int kLayerStage = 4;  // entries a lane stages at a time
+static_assert(kLayerWgs <= 32 && 2 * 32 <= kBarLines * 32, "one line of 32-bit flags per parity");
 
-// Flag barrier between the short layers (at most kFlagGrid workgroups).
-// Workgroup b stores (epoch << 32 | entries it queued in this layer) in its
-// flag of the epoch's parity; wave 0 reads every flag, one per lane, until
-// all carry the epoch, and the sum of their entries is the next layer's
-// length, returned to the whole workgroup (-1 after about a second of
-// polling: not every workgroup is resident).  A workgroup writes the flags
-// of one parity again only at epoch e + 2, after every workgroup stored its
-// epoch e + 1 flag, which each does after it read all of epoch e: no read of
-// epoch e sees a later count.  queued: this wave's entries (read on lane 0).
+// A flag: the epoch's tag (1, 2, 3 in turn for the epochs of one parity),
+// entries queued, their arcs.  A count that does not fit is stored as its
+// largest value and ends the short run: such a layer is not short.
+constexpr int kFlagArcBits = 20, kFlagCountBits = 10;
+constexpr uint32_t kFlagArcs = (1u << kFlagArcBits) - 1, kFlagCount = (1u << kFlagCountBits) - 1;
+__device__ __forceinline__ uint32_t flag_tag(uint32_t epoch) { return 1u + (epoch >> 1) % 3u; }
+
+// One queued vertex: its first arc in the high half of x and the vertex in the
+// low half, its priority in the high half of y and its arc count in the low
+struct LayerEntry {
+  uint64_t x, y;
+};
+
+// Segment of workgroup b in the layers of one parity; cap entries each.
+__device__ __forceinline__ LayerEntry* layer_segment(const LArgs& a, int parity, int b) {
+  return a.seg + (int64_t)(parity * kLayerWgs + b) * a.seg_cap;
+}
+
+__device__ __forceinline__ void store_entry(LayerEntry* e, int v, int start, int deg, uint32_t prio) {
+  __hip_atomic_store(&e->x, (uint64_t)(uint32_t)start << 32 | (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&e->y, (uint64_t)prio << 32 | (uint32_t)deg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+constexpr int kLayerLong = INT32_MAX;  // counts that do not fit a flag
+constexpr int kLayerLost = -1;         // the barrier gave up
+
+// What the workgroups know of a layer after the barrier before it.
+struct LayerShares {
+  int entry0[kLayerWgs + 1];      // entries of the segments before b
+  int arc0[kLayerWgs + 1];        // arcs of the segments before b
+  int len;                        // entries of the layer, kLayerLong or kLayerLost
+  int n;                          // entries this workgroup has queued in the layer at work
+  uint32_t arcs;                  // their arcs
+  int mine;                       // n at the barrier
+};
+
+// Flag barrier between the short layers (at most kLayerWgs workgroups).
+// Workgroup b stores (epoch, entries, arcs) of what it queued in its flag of
+// the epoch's parity; wave 0 reads every flag, one per lane, until all carry
+// the epoch, and scans the counts.  Gives up after about a second of polling:
+// not every workgroup is resident.  A workgroup writes the flags (and its
+// segment) of one parity again only at epoch e + 2, after every workgroup
+// stored its epoch e + 1 flag, which each does after it read all of epoch e:
+// no read of epoch e sees a later value, and a flag holds epoch e - 2, e or
+// nothing while e is waited for, so two bits tell them apart.
 //
 // What crosses workgroups between layers is stored and read device-coherent
-// (queue entries, the cleared control slot, the flags: global_store /
-// global_load with sc1), and each wave waits for its stores to complete
-// before the flag is written, so no agent-scope release (an L2 write-back)
-// or acquire (an L2 invalidate) is needed.  Colours are read only after the
-// kernel; pend[] changes only by atomics, which are performed beyond L2.
-// Against the two-level atomic barrier with agent-scope fences, RMAT-23's
-// colouring went from 35.4 to 33.9 ms (flags with the fences kept: 34.6).
-__device__ __forceinline__ int flag_barrier(uint64_t* flags, uint32_t epoch, int queued, int* s_cnt, int* s_len) {
-  if (lane_id() == 0 && queued) atomicAdd(s_cnt, queued);
+// (entries, the cleared control slot, the flags: global_store / global_load
+// with sc1), and each wave waits for its stores to complete before the flag
+// is written, so no agent-scope release (an L2 write-back) or acquire (an L2
+// invalidate) is needed.  Colours are read only after the kernel; pend[]
+// changes only by atomics.
+__device__ __forceinline__ int layer_barrier(uint32_t* flags, uint32_t epoch, LayerShares& sh) {
   __builtin_amdgcn_s_waitcnt(0);  // this wave's coherent stores are complete
   __syncthreads();
-  uint64_t* f = flags + (epoch & 1) * kFlagGrid;
+  uint32_t* f = flags + (epoch & 1) * 32;
   if (threadIdx.x < SMDP_WAVE) {
     const int lane = threadIdx.x;
-    const int G = gridDim.x;
+    const int G = gridDim.x / kLayerStride;
+    const uint32_t tag = flag_tag(epoch);
     if (lane == 0) {
-      const uint64_t mine = ((uint64_t)epoch << 32) | (uint32_t)*s_cnt;
-      *s_cnt = 0;  // the next adds come after the __syncthreads below
-      __hip_atomic_store(f + blockIdx.x, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int n = sh.n;
+      const uint32_t mine = tag << 30 | min((uint32_t)n, kFlagCount) << kFlagArcBits | min(sh.arcs, kFlagArcs);
+      sh.mine = n;
+      sh.n = 0;  // the next adds come after the __syncthreads below
+      sh.arcs = 0;
+      // an exchange is seen 0.2 us sooner than a store
+      (void)__hip_atomic_exchange(f + blockIdx.x / kLayerStride, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    uint64_t v = 0;
+    uint32_t v = 0;
     bool ok = true;
     for (int spins = 0;;) {
-      v = lane < G ? __hip_atomic_load(f + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                   : (uint64_t)epoch << 32;
-      if (ballot((uint32_t)(v >> 32) < epoch) == 0) break;
-      __builtin_amdgcn_s_sleep(2);
+      v = lane < G ? __hip_atomic_load(f + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag << 30;
+      if (ballot(v >> 30 != tag) == 0) break;
+      __builtin_amdgcn_s_sleep(1);
       if (++spins > kBarSpinLimit) {
         ok = false;
         break;
       }
     }
-    const unsigned long long tot = wave_sum((unsigned long long)(lane < G ? (uint32_t)v : 0u));
-    if (lane == 0) *s_len = ok ? (int)tot : -1;
+    const uint32_t n = (v >> kFlagArcBits) & kFlagCount, arcs = v & kFlagArcs;
+    const int cn = wave_scan_dpp((int)n), ca = wave_scan_dpp((int)arcs);
+    if (lane < G) {
+      sh.entry0[lane + 1] = cn;
+      sh.arc0[lane + 1] = ca;
+    }
+    const bool big = ballot(n == kFlagCount || arcs == kFlagArcs) != 0;
+    if (lane == G - 1) sh.len = !ok ? kLayerLost : big ? kLayerLong : cn;
   }
   __syncthreads();
-  return *s_len;
+  return sh.len;
 }
 
 // ctl_clear with device-coherent stores (no L2 write-back publishes them).
@@ -875,43 +967,161 @@ __device__ __forceinline__ void ctl_clear_coherent(Ctl* ctl, int slot) {
     __hip_atomic_store(c + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(SMDP_WG) void k_layer_short(LArgs a) {
-  __shared__ int32_t s_raw[3 * kShortL];
-  __shared__ int s_scan[SMDP_WAVES_PER_WG];
-  __shared__ int32_t s_out[SMDP_WAVES_PER_WG * kCOut];
-  __shared__ int32_t s_pack[SMDP_WAVES_PER_WG * kLayerIlp * SMDP_WAVE];  // notify_packed
-  __shared__ int s_cnt, s_len;
+__global__ __launch_bounds__(kLayerThreads) void k_layer_short(LArgs a) {
+  __shared__ int s_of[kShortL];   // first arc of the layer of each staged entry
+  __shared__ int4 s_ent[kShortL];  // vertex, its first arc less s_of, priority
+  __shared__ LayerShares sh;
+  __shared__ int s_base;
   const int r0 = a.rd[1];
   if (a.ctl[r0 & 3].qlen == 0) return;  // the colouring is complete (every workgroup sees it)
-  if (threadIdx.x == 0) s_cnt = 0;
-  WaveOut<kCOut> out;
-  out.init(s_out + (threadIdx.x / SMDP_WAVE) * kCOut, INT32_MAX, true);
-  unsigned long long edges = 0, verts = 0, pushes = 0;
-  uint64_t* flags = reinterpret_cast<uint64_t*>(a.bar);
+  const int L = a.ctl[(r0 + 1) & 3].qlen;  // written by the kernels before this one
+  if (blockIdx.x % kLayerStride) return;
+  const int b = blockIdx.x / kLayerStride, G = gridDim.x / kLayerStride;
   int r = r0 + 1;
-  int L = a.ctl[r & 3].qlen;  // written by the kernels before this one
+  if (L == 0 || L > kShortL) {
+    if (b == 0 && threadIdx.x == 0) a.rd[0] = r;
+    return;
+  }
+  const int lane = lane_id(), wave = threadIdx.x / SMDP_WAVE;
+  unsigned long long edges = 0, verts = 0, pushes = 0;
+  if (threadIdx.x == 0) {
+    sh.entry0[0] = 0;
+    sh.arc0[0] = 0;
+    sh.n = 0;
+    sh.arcs = 0;
+  }
+  __syncthreads();
+  {  // an equal part of the queued layer into each segment
+    const int32_t* qin = (r & 1) ? a.q1 : a.q0;
+    const int i0 = L * b / G, i1 = L * (b + 1) / G;
+    LayerEntry* seg = layer_segment(a, 1, b);
+    uint32_t arcs = 0;
+    for (int i = i0 + (int)threadIdx.x; i < i1; i += kLayerThreads) {
+      const int v = qin[i], st = a.trow[v], deg = a.trow[v + 1] - st;
+      store_entry(seg + (i - i0), v, st, deg, a.prio ? a.prio[v] : 0u);
+      arcs += (uint32_t)deg;
+    }
+    arcs = wave_total_dpp(arcs);
+    if (lane == SMDP_WAVE - 1 && arcs) atomicAdd(&sh.arcs, arcs);
+    if (threadIdx.x == 0) sh.n = i1 - i0;
+  }
   for (uint32_t epoch = 1;; ++epoch) {
-    if (L == 0 || L > kShortL) break;
-    ctl_clear_coherent(a.ctl, (r + 2) & 3);  // workgroup 0; no one uses that slot until layer r + 1
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)(r + 1));
-    const unsigned long long before = pushes;
-    short_layer<true>(a, r, L, s_raw, s_scan, s_pack, out, edges, verts, pushes);
-    out.flush((r & 1) ? a.q0 : a.q1, &a.ctl[(r + 1) & 3].qlen);
-    L = flag_barrier(flags, epoch, (int)(pushes - before), &s_cnt, &s_len);
-    if (L < 0) {
+    const int len = layer_barrier(a.bar, epoch, sh);
+    if (len == kLayerLost) {
       if (threadIdx.x == 0) a.rd[3] = 1;
       break;
     }
+    if (len == 0) break;
+    if (len > kShortL) {
+      // for k_layer_expand: the segments into the queue (what did not fit a
+      // segment is there, and so is the layer this launch began with)
+      if (epoch == 1) break;
+      const int mine = min(sh.mine, a.seg_cap);
+      if (threadIdx.x == 0) s_base = atomicAdd(&a.ctl[r & 3].qlen, mine);
+      __syncthreads();
+      const LayerEntry* seg = layer_segment(a, epoch & 1, b);
+      int32_t* q = ((r & 1) ? a.q1 : a.q0) + s_base;
+      for (int i = threadIdx.x; i < mine; i += kLayerThreads)
+        q[i] = (int)(uint32_t)__hip_atomic_load(&seg[i].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      break;
+    }
+    ctl_clear_coherent(a.ctl, (r + 2) & 3);  // workgroup 0; no one uses that slot until layer r + 1
+    const int A = sh.arc0[G];
+    if (b == 0 && threadIdx.x == 0) {
+      verts += len;
+      edges += A;
+    }
+    // This workgroup's arcs [j0, j1) of the layer lie in the segments f .. l.
+    const int j0 = (int)((int64_t)A * b / G), j1 = (int)((int64_t)A * (b + 1) / G);
+    const uint64_t in = ballot(lane < G && sh.arc0[min(lane, G)] < j1 && sh.arc0[min(lane + 1, G)] > j0);
+    int nent = 0;
+    if (in) {
+      const int f = first_lane(in), l = 63 - __builtin_clzll(in);
+      nent = sh.entry0[l + 1] - sh.entry0[f];
+      for (int w = f + wave; w <= l; w += kLayerWaves) {
+        const LayerEntry* seg = layer_segment(a, epoch & 1, w);
+        const int cnt = sh.entry0[w + 1] - sh.entry0[w], at = sh.entry0[w] - sh.entry0[f];
+        int of = sh.arc0[w];
+        for (int i0 = 0; i0 < cnt; i0 += kLayerStage * SMDP_WAVE) {
+          LayerEntry e[kLayerStage];
+#pragma unroll
+          for (int k = 0; k < kLayerStage; ++k) {
+            const int i = i0 + k * SMDP_WAVE + lane;
+            e[k].x = e[k].y = 0;
+            if (i < cnt) {
+              e[k].x = __hip_atomic_load(&seg[i].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              e[k].y = __hip_atomic_load(&seg[i].y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < kLayerStage; ++k) {
+            const int i = i0 + k * SMDP_WAVE + lane;
+            if (i0 + k * SMDP_WAVE >= cnt) break;
+            const int deg = (int)(uint32_t)e[k].y;
+            const int incl = wave_scan_dpp(deg);
+            if (i < cnt) {
+              s_of[at + i] = of + incl - deg;
+              s_ent[at + i] = make_int4((int)(uint32_t)e[k].x, (int)(uint32_t)(e[k].x >> 32) - (of + incl - deg),
+                                        (int)(uint32_t)(e[k].y >> 32), 0);
+            }
+            of += __builtin_amdgcn_readlane(incl, SMDP_WAVE - 1);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    Ctl* cout = a.ctl + ((r + 1) & 3);
+    int32_t* qover = (r & 1) ? a.q0 : a.q1;
+    LayerEntry* out = layer_segment(a, (epoch + 1) & 1, b);
+    const int top = nent ? 1 << (31 - __builtin_clz(nent)) : 0;
+    for (int jb = j0; jb < j1; jb += kLayerThreads) {
+      const int j = jb + (int)threadIdx.x;
+      const bool ok = j < j1;
+      int own = 0;
+      for (int step = top; step; step >>= 1) {
+        const int mid = own + step;
+        if (mid < nent && s_of[min(mid, nent - 1)] <= j) own = mid;
+      }
+      int v = 0, old = 0, st = 0, en = 0;
+      uint32_t pv = 0;
+      if (ok) {
+        const int4 e = s_ent[own];
+        v = stream_load(a.tcol + e.y + j);
+        if (a.prio) pv = stream_load(a.tprio + e.y + j);
+        const uint32_t pu = (uint32_t)e.z;
+        if (pu < pv || (pu == pv && e.x < v)) {
+          old = atomicSub(&a.pend[v], 1);
+          st = a.trow[v];
+          en = a.trow[v + 1];
+        }
+      }
+      const bool won = old == 1;  // 0 where nothing was taken off
+      const uint64_t m = ballot(won);
+      if (!m) continue;
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&sh.n, __popcll(m));
+      const uint32_t arcs = wave_total_dpp(won ? (uint32_t)(en - st) : 0u);
+      if (lane == SMDP_WAVE - 1) atomicAdd(&sh.arcs, arcs);
+      at = __builtin_amdgcn_readfirstlane(at) + mbcnt(m);
+      if (lane == 0) pushes += __popcll(m);
+      if (won) {
+        a.color[v] = r + 2;
+        if (at < a.seg_cap) store_entry(out + at, v, st, en - st, pv);
+        else qover[atomicAdd(&cout->qlen, 1)] = v;
+      }
+    }
     ++r;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.rd[0] = r;
+  if (b == 0 && threadIdx.x == 0) a.rd[0] = r;
   edges = wave_sum(edges);
   verts = wave_sum(verts);
   pushes = wave_sum(pushes);
-  if (lane_id() == 0) {
+  if (lane == 0) {
     if (edges) atomicAdd(&cnt_of(a.cnt)->edges, edges);
     if (verts) atomicAdd(&cnt_of(a.cnt)->verts, verts);
     if (pushes) atomicAdd(&cnt_of(a.cnt)->push[0], pushes);
+    // the last layer run has colour r
+    if (b == 0 && wave == 0) atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)r);
   }
 }
 
@@ -1020,6 +1230,7 @@ struct ColorBufs {
   int32_t* tcol = nullptr;
   int32_t* rd = nullptr;     // tuned: device layer indices (LArgs::rd)
   uint32_t* bar = nullptr;   // tuned: barrier flags of k_layer_short
+  smdp::LayerEntry* seg = nullptr;  // tuned: queue segments of k_layer_short
   uint32_t* cprio = nullptr;  // tuned, with priorities: prio[col[e]] per arc
   uint32_t* tprio = nullptr;  // tuned, with priorities: prio[tcol[e]] per arc
   uint32_t prio_version = 0;  // the graph's priority upload cprio/tprio hold (0: none)
@@ -1038,6 +1249,7 @@ void colorbufs_free(smdp_graph* g) {
   if (b->tcol) (void)hipFree(b->tcol);
   if (b->rd) (void)hipFree(b->rd);
   if (b->bar) (void)hipFree(b->bar);
+  if (b->seg) (void)hipFree(b->seg);
   if (b->cprio) (void)hipFree(b->cprio);
   if (b->tprio) (void)hipFree(b->tprio);
   delete b;
@@ -1102,6 +1314,8 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
   SMDP_CHECK(ensure_transpose(g, b));
   SMDP_CHECK(alloc_once(&b->rd, 4));
   SMDP_CHECK(alloc_once(&b->bar, kBarLines * 32));
+  const int32_t seg_cap = (int32_t)std::min<int64_t>(n1, (int64_t)kFlagCount);
+  SMDP_CHECK(alloc_once(&b->seg, (int64_t)2 * kLayerWgs * seg_cap));
   if (use_prio && b->prio_version != g->prio_version) {
     // the arcs' priorities, aligned with col and tcol: once per priority upload
     const int64_t m1 = std::max<int64_t>(1, g->m);
@@ -1139,21 +1353,20 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
   a.grid = grid;
   a.rd = b->rd;
   a.bar = reinterpret_cast<uint32_t*>(b->bar);
+  a.seg = b->seg;
+  a.seg_cap = seg_cap;
   // k_layer_short: its workgroups meet at barriers between layers, so all
-  // must be resident at once.  The grid is a quarter of the CUs (its barrier costs
-  // more per workgroup than a short layer gains from more of them: on
-  // RMAT-23, 256/128/64/32/16/8 workgroups took 48.6/43.0/39.1/42.6/56.0/
-  // 83.8 ms per colouring), capped at what the device holds, and launched
-  // after the stream's previous kernels finished, so it fits on the idle
+  // must be resident at once: few of them, capped at what the device holds, and launched
+  // after the stream's previous kernels finished, so they fit on the idle
   // device; a barrier that waits too long (another process holding CUs)
   // makes the run return SMDP_ERR_DEVICE instead of hanging.  A plain launch
   // rather than a cooperative one: rocprofv3 ended with a segmentation fault
   // in its exit handlers after cooperative launches.
   int per_cu = 0;
   SMDP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_layer_short),
-                                                          SMDP_WG, 0));
+                                                          kLayerThreads, 0));
   if (per_cu < 1) return SMDP_ERR_DEVICE;
-  const int short_grid = std::min({std::max(8, ctx->cus / 4), per_cu * ctx->cus, kFlagGrid});
+  const int short_grid = std::min(per_cu * ctx->cus, kLayerWgs);
   hipStream_t s = ctx->stream;
   prof_reset(ctx);
   int launches = 0;
@@ -1161,7 +1374,8 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
   hipLaunchKernelGGL(k_layer_init, dim3(1), dim3(256), 0, s, g->ctl, g->cnt, a.rd);
   hipLaunchKernelGGL(k_layer_count, dim3(grid), dim3(SMDP_WG), 0, s, a);
   hipLaunchKernelGGL(k_layer_count_chunks, dim3(grid), dim3(SMDP_WG), 0, s, a);
-  hipLaunchKernelGGL(k_layer_seed, dim3(std::min<int64_t>((n1 + SMDP_WG - 1) / SMDP_WG, grid)), dim3(SMDP_WG), 0, s, a);
+  hipLaunchKernelGGL(k_layer_seed, dim3(std::min<int64_t>({(n1 + SMDP_WG - 1) / SMDP_WG, grid, 4 * ctx->cus})),
+                     dim3(SMDP_WG), 0, s, a);
   launches += 4;
   // A step is one layer on the whole grid (expand, then the drain of its
   // chunks) followed by the run of short layers after it in one launch.  The
@@ -1184,7 +1398,7 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
       hipLaunchKernelGGL(k_layer_drain, dim3(drain_grid), dim3(SMDP_WG), 0, s, a);
       SMDP_CHECK(prof_mark(ctx, 1));
       SMDP_CHECK(prof_mark(ctx, 0));
-      hipLaunchKernelGGL(k_layer_short, dim3(short_grid), dim3(SMDP_WG), 0, s, a);
+      hipLaunchKernelGGL(k_layer_short, dim3(short_grid * kLayerStride), dim3(kLayerThreads), 0, s, a);
       SMDP_CHECK(prof_mark(ctx, 0));
       launches += 3;
     }

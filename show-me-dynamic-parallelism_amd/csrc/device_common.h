@@ -281,17 +281,20 @@ __device__ __forceinline__ CSum wave_csum_dpp(CSum x) {
   return t;
 }
 
-// Sum over the wave in lane 63 (other lanes hold partial sums): DPP shifts
-// within each row of 16, then the row totals passed on by row broadcasts.
-__device__ __forceinline__ uint32_t wave_total_dpp(uint32_t x) {
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);  // row_shr:1
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);  // row_shr:2
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);  // row_shr:4
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);  // row_shr:8
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+// Inclusive scan over the wave: DPP shifts within each row of 16, then the
+// row totals passed on by row broadcasts.
+__device__ __forceinline__ int wave_scan_dpp(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
   return x;
 }
+
+// Sum over the wave in lane 63 (other lanes hold partial sums).
+__device__ __forceinline__ uint32_t wave_total_dpp(uint32_t x) { return (uint32_t)wave_scan_dpp((int)x); }
 
 // FP64 sum over the wave with DPP steps; every lane returns the same value,
 // formed from the row sums in lanes 15, 31, 47, 63 in that order.

@@ -104,17 +104,6 @@ struct LdsCount {
 // Results of a solve below 0.
 constexpr int kLdsRoundCap = -1, kLdsTimeout = -2, kLdsWeight = -3;
 
-// Inclusive wave scan with DPP steps.
-__device__ __forceinline__ int wave_scan_dpp(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);   // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);   // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);   // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);   // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31
-  return x;
-}
-
 // Smallest x of the wave, in lane 63.
 __device__ __forceinline__ int wave_min_dpp(int x) {
   x = min(x, __builtin_amdgcn_update_dpp(INT32_MAX, x, 0x111, 0xF, 0xF, false));
