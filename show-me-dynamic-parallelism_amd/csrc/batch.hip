@@ -2,14 +2,13 @@
 // source per process run: SSSP_GPU, apps/sssp/src/sssp_wrapper.cu:304-341).
 //
 // Many sources on one graph: distances are laid out [vertex][64] so the 64
-// lanes of a wave hold the 64 sources of one vertex.  A frontier vertex is
-// expanded by one wave: for each arc (u,v,w) the wave reads the 256 bytes of
-// dist[v][*] in one coalesced access and relaxes all sources at once, so one
-// read of the CSR serves every source.  The frontier is the union over
-// sources; a vertex is queued once per round whatever source improved it.
-// Vertices with at least `split` arcs are cut into chunks of `chunk` arcs that
-// any wave can take in a second kernel.  More than 64 sources run as groups of
-// 64.
+// lanes of a wave hold the 64 sources of one vertex.  For each arc (u,v,w) of
+// a frontier vertex a wave reads the 256 bytes of dist[v][*] in one coalesced
+// access and relaxes all sources at once, so one read of the CSR serves every
+// source.  The frontier is the union over sources; a vertex is queued once
+// per round whatever source improved it.  Every round runs in one launch
+// (k_ms_run): a pass counts the frontier's arcs, a second gives every wave an
+// equal share of them.  More than 64 sources run as groups of 64.
 //
 // Many small graphs: one workgroup solves one whole graph, every round inside
 // the kernel with workgroup barriers between rounds (no grid-wide
@@ -28,6 +27,7 @@
 #include <vector>
 
 #include "device_common.h"
+#include "frontier.h"
 #include "grid_barrier.h"
 #include "lds_sssp.h"
 #include "smdp_internal.h"
@@ -39,8 +39,18 @@ constexpr int kMsOut = 512;
 #define SMDP_MS_ILP 8
 #endif
 constexpr int kMsIlp = SMDP_MS_ILP;  // target rows of 64 distances a wave loads at once
-static_assert(kMsIlp <= SMDP_WAVE, "lane t queues arc t's target");
 constexpr int kLanes = SMDP_WAVE;  // sources per group
+
+// Reference distances of a group of sources (see ms_bound).
+struct MsRef {
+  unsigned long long hub;  // arcs << 32 | ~vertex of the vertex of most arcs (the lowest such)
+  int32_t gen;             // distances taken so far, 0: none or no longer in use
+  int32_t pad[29];
+  int32_t off[kLanes];     // distances of the hub when last taken, SMDP_SSSP_INF: source left out
+};
+constexpr int kMsGrid = 2048;  // most workgroups of k_ms_run
+constexpr int kMsRefRound = 2;  // reference distances are taken after this round at the earliest
+constexpr int kMsGens = 3;      // and at most so often
 
 struct MArgs {
   const int32_t* __restrict__ row;
@@ -48,6 +58,11 @@ struct MArgs {
   const int32_t* __restrict__ w;
   int32_t* mdist;  // [n][64]
   int32_t* stamp;
+  int32_t* bound;  // [kMsGens][n] upper bound of a vertex's distances over the reference ones, INT32_MAX: none
+  MsRef* ref;
+  int32_t* qoff;   // [n] arcs of the queue entries before this one in its workgroup's part
+  int32_t* qm;     // [n] ms_bound of the queue entries
+  int32_t* tot;    // [kMsGrid] arcs of each workgroup's part of the queue
   int32_t* q0;
   int32_t* q1;
   Chunk* hq;
@@ -57,7 +72,30 @@ struct MArgs {
   int32_t chunk;
 };
 
-// Relax arcs [s, e) of u for all 64 sources held by the lanes.  Wave-uniform.
+// The distance rows of an arc's target are 256 bytes, and on RMAT-20 only a
+// fifth of the arcs a round expands lower any of the 64 distances.  Distances
+// from different sources differ mostly by how far each source is from the
+// core of the graph, so a single number per vertex tells most of the useless
+// arcs: with off[s] = the hub's distance from source s at some moment,
+//   bound[v] >= max over s of d(v, s) - off[s]    (kept when v was expanded;
+//                                                  distances only fall)
+//   m(u)      = min over the s that reach u of d(u, s) - off[s]
+// and m(u) + w >= bound[v] means d(u, s) + w >= d(v, s) for every s, so the
+// row of v need not be read.  off may hold any numbers as long as every use
+// has the same; a source that had not reached the hub when off was taken is
+// in no bound, and a vertex that it reaches skips no arc.  Returns m(u), or
+// INT32_MIN where nothing may be skipped; *bound: INT32_MAX for none.
+__device__ __forceinline__ int ms_bound(int du, int off, int* bound) {
+  constexpr int kLow = -SMDP_SSSP_INF;  // below this the differences could leave 32 bits
+  const bool reached = du < SMDP_SSSP_INF, in = off < SMDP_SSSP_INF, low = du <= kLow;
+  const int most = ~__builtin_amdgcn_readlane(wave_min_dpp(in ? ~(du - off) : INT32_MAX), SMDP_WAVE - 1);
+  *bound = ballot(in && (!reached || low)) ? INT32_MAX : most;
+  const int least = __builtin_amdgcn_readlane(wave_min_dpp(reached ? du - off : INT32_MAX), SMDP_WAVE - 1);
+  return ballot(reached && (!in || low)) ? INT32_MIN : least;
+}
+
+// Relax arcs [s, e) of u for all 64 sources held by the lanes (host-driven
+// rounds; k_ms_run's are ms_relax_pass).  Wave-uniform.
 __device__ __forceinline__ void ms_arcs(const MArgs& a, int s, int e, int du, int label, WaveOut<kMsOut>& out,
                                         int32_t* qout, int32_t* qlen, unsigned long long& edges,
                                         unsigned long long& wins) {
@@ -106,13 +144,29 @@ __device__ __forceinline__ void ms_arcs(const MArgs& a, int s, int e, int du, in
   }
 }
 
-__global__ void k_ms_init(int32_t* mdist, int32_t* stamp, int32_t n, const int32_t* __restrict__ srcs, int32_t k,
-                          int32_t* q0, Ctl* ctl, Counters* cnt) {
+// The hub first: its one atomic per workgroup completes under the fill.
+__global__ __launch_bounds__(SMDP_WG) void k_ms_init(MArgs a, int32_t n) {
+  __shared__ unsigned long long s_hub[SMDP_WAVES_PER_WG];
+  int32_t* mdist = a.mdist;
+  Ctl* ctl = a.ctl;
+  unsigned long long hub = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    a.stamp[i] = -1;
+    for (int g = 0; g < kMsGens; ++g) a.bound[(int64_t)g * n + i] = INT32_MAX;
+    const unsigned long long deg = (unsigned long long)(uint32_t)(a.row[i + 1] - a.row[i]);
+    hub = max(hub, deg << 32 | (uint32_t)~(uint32_t)i);
+  }
+#pragma unroll
+  for (int off = SMDP_WAVE / 2; off > 0; off >>= 1) hub = max(hub, __shfl_xor(hub, off));
+  if (lane_id() == 0) s_hub[threadIdx.x / SMDP_WAVE] = hub;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < SMDP_WAVES_PER_WG; ++k) hub = max(hub, s_hub[k]);
+    if (hub) atomicMax(&a.ref->hub, hub);
+  }
   const int64_t total = (int64_t)n * kLanes;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x)
     mdist[i] = SMDP_SSSP_INF;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    stamp[i] = -1;
   if (blockIdx.x == 0) {
     int32_t* c = reinterpret_cast<int32_t*>(ctl);
     for (int i = threadIdx.x; i < 4 * kCtlInts; i += blockDim.x) c[i] = 0;
@@ -230,29 +284,207 @@ __global__ __launch_bounds__(SMDP_WG) void k_ms_drain(MArgs a, int r) {
   ms_counters(a, edges, 0, wins, 0, edges);
 }
 
+// First pass of a round: workgroup b takes the b-th equal part of the L queue
+// entries, and stores the arcs before each (qoff), its bound (qm, INT32_MIN
+// while there are no reference distances) and the part's arcs (tot).
+constexpr int kMsRows = 8;  // distance rows a wave loads at once
+__device__ __forceinline__ void ms_count_pass(const MArgs& a, const int32_t* qin, int L, int32_t* bound, int off,
+                                              int* s_scan) {
+  const int lane = lane_id(), wave = threadIdx.x / SMDP_WAVE;
+  const int b = blockIdx.x, G = gridDim.x;
+  const int i0 = (int)((int64_t)L * b / G), i1 = (int)((int64_t)L * (b + 1) / G);
+  int before = 0;
+  for (int ib = i0; ib < i1; ib += SMDP_WG) {
+    const int i = ib + (int)threadIdx.x;
+    int deg = 0;
+    if (i < i1) {
+      const int u = qin[i];
+      deg = a.row[u + 1] - a.row[u];
+      if (!bound) a.qm[i] = INT32_MIN;
+    }
+    int sum;
+    const int ex = wg_exclusive_scan(deg, s_scan, &sum);
+    if (i < i1) a.qoff[i] = before + ex;
+    before += sum;
+  }
+  if (threadIdx.x == 0) __hip_atomic_store(a.tot + b, before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!bound) return;
+  for (int i = i0 + wave * kMsRows; i < i1; i += SMDP_WAVES_PER_WG * kMsRows) {
+    const int mine = qin[min(i + (lane & (kMsRows - 1)), i1 - 1)];
+    int d[kMsRows], m = 0, bd = 0;
+#pragma unroll
+    for (int t = 0; t < kMsRows; ++t)
+      d[t] = a.mdist[(int64_t)__builtin_amdgcn_readlane(mine, t) * kLanes + lane];
+#pragma unroll
+    for (int t = 0; t < kMsRows; ++t) {
+      int bt;
+      const int mt = ms_bound(d[t], off, &bt);
+      m = lane == t ? mt : m;
+      bd = lane == t ? bt : bd;
+    }
+    if (lane < kMsRows && i + lane < i1) {
+      a.qm[i + lane] = m;
+      if (bd != INT32_MAX) __hip_atomic_store(bound + mine, bd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// Second pass: each wave relaxes an equal part of the round's arcs, found by
+// the workgroups' totals (s_pre: their prefix sums) and the entries' offsets.
+// A batch of up to 64 arcs, one per lane, loads its targets, weights and the
+// targets' bounds at once; the arcs left then go kMsIlp at a time, all lanes
+// on one arc's 64 sources, with the rows of all of them loaded before any is
+// used.  The targets of a batch are queued together.  Returns the arcs.
+__device__ __forceinline__ int ms_relax_pass(const MArgs& a, const int32_t* qin, int L, int label, const int* s_pre,
+                                             const int32_t* bound, Sink& out, unsigned long long& wins, int& skips) {
+  const int lane = lane_id(), wave = threadIdx.x / SMDP_WAVE;
+  const int G = gridDim.x, A = s_pre[G];
+  const int gw = blockIdx.x * SMDP_WAVES_PER_WG + wave, nw = G * SMDP_WAVES_PER_WG;
+  const int j0 = (int)((int64_t)A * gw / nw), j1 = (int)((int64_t)A * (gw + 1) / nw);
+  if (j0 >= j1) return 0;
+  int sg = 0;  // the part that holds arc j0
+  for (int step = kMsGrid / 2; step; step >>= 1)
+    if (sg + step < G && s_pre[sg + step] <= j0) sg += step;
+  sg = __builtin_amdgcn_readfirstlane(sg);
+  int i = (int)((int64_t)L * sg / G), end = (int)((int64_t)L * (sg + 1) / G);
+  int base = s_pre[sg];
+  // its entries: the last of them with qoff <= j0 - base is among i .. i + 63
+  for (int cnt = end - i; cnt > SMDP_WAVE;) {
+    const int step = (cnt + SMDP_WAVE - 1) / SMDP_WAVE;
+    const bool le = lane * step < cnt && a.qoff[i + min(lane * step, cnt - 1)] <= j0 - base;
+    const int at = (__popcll(ballot(le)) - 1) * step;
+    i += at;
+    cnt = min(step, cnt - at);
+  }
+  for (int jb = j0; jb < j1;) {
+    // entries i .. i + 63 of the part, one per lane
+    const bool ok = i + lane < end;
+    const int e = min(i + lane, end - 1);
+    const int wu = qin[e], wm = a.qm[e];
+    const int wof = ok ? base + a.qoff[e] : INT32_MAX;
+    const int wst = a.row[wu] - wof;
+    const int wend = i + SMDP_WAVE < end ? base + a.qoff[i + SMDP_WAVE] : s_pre[sg + 1];
+    const int jend = min(j1, wend);
+    for (; jb < jend; jb += SMDP_WAVE) {
+      const int j = min(jb + lane, jend - 1);
+      int own = 0;
+#pragma unroll
+      for (int step = SMDP_WAVE / 2; step; step >>= 1) own += __shfl(wof, own + step) <= j ? step : 0;
+      const int k = __shfl(wst, own) + j, cu = __shfl(wu, own), m = __shfl(wm, own);
+      const int cv = a.col[k], cw = a.w[k];
+      bool relax = jb + lane < jend;
+      if (bound) {
+        const int bv = bound[cv];
+        relax = relax && (m == INT32_MIN || bv == INT32_MAX || (int64_t)m + cw < (int64_t)bv);
+      }
+      uint64_t left = ballot(relax), hits = 0;
+      skips += min(jend - jb, SMDP_WAVE) - __popcll(left);
+      while (left) {
+        int v[kMsIlp], du[kMsIlp], dv[kMsIlp], alt[kMsIlp], jj[kMsIlp];
+        const int here = __popcll(left);
+#pragma unroll
+        for (int t = 0; t < kMsIlp; ++t) {
+          jj[t] = left ? first_lane(left) : jj[t ? t - 1 : 0];
+          left &= left - 1;
+          v[t] = __builtin_amdgcn_readlane(cv, jj[t]);
+          du[t] = a.mdist[(int64_t)__builtin_amdgcn_readlane(cu, jj[t]) * kLanes + lane];
+          dv[t] = a.mdist[(int64_t)v[t] * kLanes + lane];
+        }
+        // A candidate below the distance just read lowers that distance in this
+        // round, through itself or a lower candidate, so its atomicMin returns
+        // nothing and the wave does not wait for it.
+#pragma unroll
+        for (int t = 0; t < kMsIlp; ++t) {
+          alt[t] = du[t] + __builtin_amdgcn_readlane(cw, jj[t]);
+          const bool imp = t < here && du[t] < SMDP_SSSP_INF && alt[t] < dv[t];
+          if (imp) __hip_atomic_fetch_min(&a.mdist[(int64_t)v[t] * kLanes + lane], alt[t], __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+          const uint64_t won = ballot(imp);
+          wins += __popcll(won);
+          hits |= (uint64_t)(won != 0) << jj[t];
+        }
+      }
+      bool push = false;
+      if ((hits >> lane) & 1)
+        push = a.stamp[cv] != label && atomicExch(&a.stamp[cv], label) != label;
+      out.push(push, cv);
+    }
+    if (jb >= jend) jb = jend;
+    if (i + SMDP_WAVE < end) {
+      i += SMDP_WAVE;
+    } else if (jb < j1) {
+      do ++sg;
+      while (s_pre[sg + 1] <= jb);
+      i = (int)((int64_t)L * sg / G);
+      end = (int)((int64_t)L * (sg + 1) / G);
+      base = s_pre[sg];
+    }
+  }
+  return j1 - j0;
+}
+
+// Keeps the reference distances (wave 0 of workgroup 0, between the two
+// barriers of round r, when every workgroup has read the ones in use; for the
+// rounds after r).  They are taken once the hub is reached by three quarters
+// of the k sources and again, with bounds of their own, when more reach it: a
+// source left out keeps the vertices it reaches from skipping arcs, so only
+// one that never gets to the hub should be.  Where they tell little (a uniform
+// graph), by this workgroup's arcs of the round, they are given up: 262144
+// vertices of 8 arcs took 3.6 ms with bounds to the end, 3.3 without.
+struct MsRefKeeper {
+  int gen = 0, alive = 0, rounds = 0;
+  bool done = false;
+  __device__ __forceinline__ void step(const MArgs& a, int r, int k, int seen, int skipped) {
+    if (done || r < kMsRefRound) return;
+    const int lane = lane_id();
+    const int hub = (int)~(uint32_t)a.ref->hub;
+    int d = __hip_atomic_load(a.mdist + (int64_t)hub * kLanes + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (d <= -SMDP_SSSP_INF) d = SMDP_SSSP_INF;
+    const int c = __popcll(ballot(lane < k && d < SMDP_SSSP_INF));
+    ++rounds;
+    if (gen == 0 ? 4 * c >= 3 * k : c > alive && gen < kMsGens) {
+      __hip_atomic_store(&a.ref->off[lane], d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ++gen;
+      alive = c;
+      rounds = 0;
+      if (lane == 0) __hip_atomic_store(&a.ref->gen, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (gen && rounds >= 2 && skipped < seen / 8) {
+      done = true;
+      if (lane == 0) __hip_atomic_store(&a.ref->gen, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+};
+
 // Every round of one group of sources in one launch whose workgroups are all
 // resident (the grid is sized to what the device holds), with a grid barrier
-// after the expansion pass and, when the round pushed chunks, after the chunk
-// pass.  Every workgroup reads the queue lengths after a barrier, so all take
-// the same barriers and stop together.  flags[0] = 1 when a barrier gave up
-// waiting; flags[1 + group] = the rounds run, or -1 when rmax was reached.
-// The launch needs no host check between rounds, so it can be captured in a
-// hipGraph with the initialisation and replayed.
-#ifndef SMDP_MS_WAVES
-#define SMDP_MS_WAVES 0
-#endif
-#if SMDP_MS_WAVES > 0
-#define SMDP_MS_RUN_ATTR __attribute__((amdgpu_waves_per_eu(SMDP_MS_WAVES, SMDP_MS_WAVES)))
-#else
-#define SMDP_MS_RUN_ATTR
-#endif
-__global__ __launch_bounds__(SMDP_WG) SMDP_MS_RUN_ATTR void k_ms_run(MArgs a, uint32_t* bar, int32_t* flags, int group,
-                                                                     int rmax) {
-  __shared__ int32_t s_out[SMDP_WAVES_PER_WG * kMsOut];
+// after each of the two passes.
+// Bound: the atomics and rows of the arcs that do lower a distance (RMAT-20 x
+// 64: 1.9e8 distances lowered), then the barriers (a round of RMAT-20 spends
+// 110 us of 250 on the count, the barriers and the wait for the last wave).
+// Two things made it faster than one wave per frontier vertex with chunks for
+// vertices of 512 arcs and more (8.8 ms for RMAT-20 x 64; RMAT-17 3.3, RMAT-13
+// 1.8, RMAT-18 x 5 3.5, uniform 2^18 x 8 3.8): equal shares of the arcs, which
+// no wave's 511-arc vertex and no chunk counter hold up (5.7 ms, 1.5, 0.44,
+// 1.8, 3.3), and the bounds of ms_bound (3.5 ms, 1.1, 0.41, 1.3, 3.3).  Five
+// waves per SIMD: four took 4.0 ms, six 4.0, eight 4.6 (spills).
+// Every workgroup reads the queue length after a barrier, so all take the
+// same barriers and stop together.  flags[0] = 1
+// when a barrier gave up waiting; flags[1 + group] = the rounds run, or -1
+// when rmax was reached.  The launch needs no host check between rounds, so
+// it can be captured in a hipGraph with the initialisation and replayed.
+__global__ __launch_bounds__(SMDP_WG) __attribute__((amdgpu_waves_per_eu(5, 5))) void k_ms_run(
+    MArgs a, uint32_t* bar, int32_t* flags, int group, int k, int n, int rmax) {
+  __shared__ int s_pre[kMsGrid + 1];
+  __shared__ int32_t s_out[SMDP_WAVES_PER_WG * kOutCap];
+  __shared__ int s_scan[SMDP_WAVES_PER_WG + 1];
+  __shared__ int s_seen[SMDP_WAVES_PER_WG], s_skip[SMDP_WAVES_PER_WG];
+  static_assert(SMDP_WAVES_PER_WG == 4, "summed below");
   __shared__ int s_ok;
-  WaveOut<kMsOut> out;
-  out.init(s_out + (threadIdx.x / SMDP_WAVE) * kMsOut);
-  unsigned long long edges = 0, verts = 0, wins = 0, pg = 0, edges2 = 0;
+  const int G = gridDim.x;
+  MsRefKeeper keeper;
+  Sink out;
+  out.init(s_out + (threadIdx.x / SMDP_WAVE) * kOutCap, nullptr, nullptr);  // the queue is set each round
+  unsigned long long edges = 0, verts = 0, wins = 0;
   uint32_t epoch = 0;
   int r = 0;
   bool capped = false;
@@ -265,32 +497,69 @@ __global__ __launch_bounds__(SMDP_WG) SMDP_MS_RUN_ATTR void k_ms_run(MArgs a, ui
     }
     if (blockIdx.x == 0) {
       ctl_clear(a.ctl, (r + 2) & 3);  // round r + 1's output slot; no workgroup of round r uses it
-      if (threadIdx.x == 0) atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)(r + 1));
+      if (threadIdx.x == 0) {
+        atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)(r + 1));
+        verts += L;
+      }
     }
-    ms_expand_pass(a, r, L, out, edges, verts, wins, pg);
+    const int32_t* qin = (r & 1) ? a.q1 : a.q0;
+    const int gen = __hip_atomic_load(&a.ref->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int off = gen ? __hip_atomic_load(&a.ref->off[lane_id()], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    int32_t* bound = gen ? a.bound + (int64_t)(gen - 1) * n : nullptr;
+    ms_count_pass(a, qin, L, bound, off, s_scan);
     if (!grid_barrier(bar, ++epoch, &s_ok)) {
       if (threadIdx.x == 0) atomicExch(&flags[0], 1);
       break;
     }
-    const int H = __hip_atomic_load(&a.ctl[r & 3].hlen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (H > 0) {
-      const unsigned long long e0 = edges;
-      ms_drain_pass(a, r, H, out, edges, wins);
-      edges2 += edges - e0;
-      if (!grid_barrier(bar, ++epoch, &s_ok)) {
-        if (threadIdx.x == 0) atomicExch(&flags[0], 1);
-        break;
+    {  // prefix sums of the parts' arcs
+      constexpr int E = kMsGrid / SMDP_WG;
+      int x[E], sum = 0;
+#pragma unroll
+      for (int t = 0; t < E; ++t) {
+        const int i = (int)threadIdx.x * E + t;
+        x[t] = i < G ? __hip_atomic_load(a.tot + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        sum += x[t];
       }
+      int all, run = wg_exclusive_scan(sum, s_scan, &all);
+#pragma unroll
+      for (int t = 0; t < E; ++t) {
+        const int i = (int)threadIdx.x * E + t;
+        if (i < G) s_pre[i] = run;
+        run += x[t];
+      }
+      if (threadIdx.x == 0) s_pre[G] = all;
+      __syncthreads();
+    }
+    out.q = (r & 1) ? a.q0 : a.q1;
+    out.qlen = &a.ctl[(r + 1) & 3].qlen;
+    int skips = 0;
+    const int arcs = ms_relax_pass(a, qin, L, r + 1, s_pre, bound, out, wins, skips);
+    if (lane_id() == 0) {
+      edges += arcs;
+      s_seen[threadIdx.x / SMDP_WAVE] = arcs;
+      s_skip[threadIdx.x / SMDP_WAVE] = skips;
+    }
+    wg_flush(out, s_scan);
+    if (blockIdx.x == 0 && threadIdx.x < SMDP_WAVE)
+      keeper.step(a, r, k, s_seen[0] + s_seen[1] + s_seen[2] + s_seen[3], s_skip[0] + s_skip[1] + s_skip[2] + s_skip[3]);
+    if (!grid_barrier(bar, ++epoch, &s_ok)) {
+      if (threadIdx.x == 0) atomicExch(&flags[0], 1);
+      break;
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) flags[1 + group] = capped ? -1 : r;
-  ms_counters(a, edges, verts, wins, pg, edges2);
+  if (lane_id() != 0) wins = 0;
+  ms_counters(a, edges, verts, wins, 0, 0);
 }
 
 // Resets a group's barrier lines (every group's persistent launch counts its
-// epochs from 1) and, for the first group, the batch's flags and counters.
-__global__ void k_ms_reset(uint32_t* bar, int32_t* flags, int32_t nflags, Counters* cnt, int first) {
+// epochs from 1) and reference distances, and, for the first group, the batch's flags and counters.
+__global__ void k_ms_reset(uint32_t* bar, MsRef* ref, int32_t* flags, int32_t nflags, Counters* cnt, int first) {
   for (int i = threadIdx.x; i < kBarLines * 32; i += blockDim.x) bar[i] = 0;
+  if (threadIdx.x == 0) {
+    ref->hub = 0;
+    ref->gen = 0;
+  }
   if (!first) return;
   for (int i = threadIdx.x; i < nflags; i += blockDim.x) flags[i] = 0;
   unsigned long long* p = reinterpret_cast<unsigned long long*>(cnt);
@@ -695,6 +964,11 @@ struct MsPlan {
   int32_t* mres = nullptr;    // [k][n], source-major
   int64_t mres_cap = 0;
   uint32_t* bar = nullptr;    // kBarLines * 32 barrier words
+  int32_t* bound = nullptr;   // [kMsGens][n] MArgs::bound
+  smdp::MsRef* ref = nullptr;
+  int32_t* qoff = nullptr;    // [n], [n], [kMsGrid]: of k_ms_run's passes
+  int32_t* qm = nullptr;
+  int32_t* tot = nullptr;
   int32_t* flags = nullptr;   // [0] a barrier gave up; [1 + j] rounds of group j (-1: round cap)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -714,7 +988,7 @@ void msplan_free(smdp_graph* g) {
   MsPlan* pl = static_cast<MsPlan*>(g->msplan);
   if (!pl) return;
   pl->drop_graph();
-  void* ptrs[] = {pl->d_srcs, pl->mres, pl->bar, pl->flags};
+  void* ptrs[] = {pl->d_srcs, pl->mres, pl->bar, pl->bound, pl->ref, pl->qoff, pl->qm, pl->tot, pl->flags};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   delete pl;
@@ -729,13 +1003,18 @@ int msplan_result(smdp_graph* g, const int32_t** out, int64_t* count) {
   return SMDP_OK;
 }
 
-static MArgs ms_args(smdp_graph* g, const smdp_params& p) {
+static MArgs ms_args(smdp_graph* g, const MsPlan* pl, const smdp_params& p) {
   MArgs a;
   a.row = g->row;
   a.col = g->col;
   a.w = g->w;
   a.mdist = g->mdist;
   a.stamp = g->stamp;
+  a.bound = pl->bound;
+  a.ref = pl->ref;
+  a.qoff = pl->qoff;
+  a.qm = pl->qm;
+  a.tot = pl->tot;
   a.q0 = g->q[0];
   a.q1 = g->q[1];
   a.hq = g->hq;
@@ -752,14 +1031,13 @@ static MArgs ms_args(smdp_graph* g, const smdp_params& p) {
 static int ms_rounds_host(smdp_graph* g, MsPlan* pl, const smdp_params& p, uint64_t* rounds, uint64_t* launches) {
   smdp_ctx* ctx = g->ctx;
   hipStream_t s = ctx->stream;
-  const MArgs a = ms_args(g, p);
+  const MArgs a = ms_args(g, pl, p);
   const int grid = grid_size(ctx, p);
-  hipLaunchKernelGGL(k_ms_reset, dim3(1), dim3(256), 0, s, pl->bar, pl->flags, 1 + pl->groups, g->cnt, 1);
+  hipLaunchKernelGGL(k_ms_reset, dim3(1), dim3(256), 0, s, pl->bar, pl->ref, pl->flags, 1 + pl->groups, g->cnt, 1);
   ++*launches;
   for (int j = 0; j < pl->groups; ++j) {
     const int s0 = j * kLanes, kk = std::min<int32_t>(kLanes, pl->k - s0);
-    hipLaunchKernelGGL(k_ms_init, dim3(2048), dim3(256), 0, s, g->mdist, g->stamp, g->n, pl->d_srcs + s0, kk, g->q[0],
-                       g->ctl, g->cnt);
+    hipLaunchKernelGGL(k_ms_init, dim3(2048), dim3(SMDP_WG), 0, s, a, g->n);
     hipLaunchKernelGGL(k_ms_seed, dim3(1), dim3(64), 0, s, g->mdist, g->stamp, pl->d_srcs + s0, kk, g->q[0], g->ctl);
     *launches += 2;
     int r = 0;
@@ -816,7 +1094,13 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_ms_run), SMDP_WG, 0) !=
       hipSuccess)
     per_cu = 0;
-  const int pgrid = std::min(grid_size(ctx, p), per_cu * ctx->cus);
+  // A round's barriers cost by the workgroup, its arcs by their share of them,
+  // so the best grid grows with the square root of the arcs.  Measured best
+  // (workgroups): 8192 arcs 32 to 128, 65536 128, 262144 256, 2^20 512, 2^22
+  // 768 to 1024, 2^24 all that fit (1280); from half to twice as many it is
+  // within 15 %.
+  const int want = std::max(32, (int)std::sqrt((double)g->m / 4));
+  const int pgrid = std::min({grid_size(ctx, p), per_cu * ctx->cus, kMsGrid, want});
   const int rmax = (int)std::min<int64_t>(p.max_rounds, n + 1);  // more rounds than vertices: a negative cycle
   const int groups = (k + kLanes - 1) / kLanes;
   const void* bufs[7] = {g->mdist, g->stamp, g->q[0], g->q[1], g->hq, g->ctl, g->cnt};
@@ -834,6 +1118,11 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
       SMDP_CHECK(alloc_once(&pl->flags, 1 + groups));
     }
     SMDP_CHECK(alloc_once(&pl->bar, (int64_t)kBarLines * 32));
+    SMDP_CHECK(alloc_once(&pl->bound, (int64_t)kMsGens * n));
+    SMDP_CHECK(alloc_once(&pl->ref, 1));
+    SMDP_CHECK(alloc_once(&pl->qoff, n));
+    SMDP_CHECK(alloc_once(&pl->qm, n));
+    SMDP_CHECK(alloc_once(&pl->tot, kMsGrid));
     SMDP_CHECK(ensure(&pl->mres, &pl->mres_cap, (int64_t)k * n));
     pl->k = k;
     pl->groups = groups;
@@ -843,17 +1132,18 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
     pl->rmax = rmax;
     std::copy(bufs, bufs + 7, pl->bufs);
     if (pgrid >= 1) {
-      const MArgs a = ms_args(g, p);
+      const MArgs a = ms_args(g, pl, p);
       SMDP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       for (int j = 0; j < groups; ++j) {
         const int s0 = j * kLanes, kk = std::min<int32_t>(kLanes, k - s0);
         // kernels clear the barrier lines, flags and counters (no memset nodes)
-        hipLaunchKernelGGL(k_ms_reset, dim3(1), dim3(256), 0, s, pl->bar, pl->flags, 1 + groups, g->cnt, j == 0);
-        hipLaunchKernelGGL(k_ms_init, dim3(2048), dim3(256), 0, s, g->mdist, g->stamp, g->n, pl->d_srcs + s0, kk,
-                           g->q[0], g->ctl, g->cnt);
+        hipLaunchKernelGGL(k_ms_reset, dim3(1), dim3(256), 0, s, pl->bar, pl->ref, pl->flags, 1 + groups, g->cnt,
+                           j == 0);
+        hipLaunchKernelGGL(k_ms_init, dim3(2048), dim3(SMDP_WG), 0, s, a, g->n);
         hipLaunchKernelGGL(k_ms_seed, dim3(1), dim3(64), 0, s, g->mdist, g->stamp, pl->d_srcs + s0, kk, g->q[0],
                            g->ctl);
-        hipLaunchKernelGGL(k_ms_run, dim3(pgrid), dim3(SMDP_WG), 0, s, a, pl->bar, pl->flags, j, rmax);
+        hipLaunchKernelGGL(k_ms_run, dim3(pgrid), dim3(SMDP_WG), 0, s, a, pl->bar, pl->flags, j, kk, g->n,
+                           rmax);
         hipLaunchKernelGGL(k_ms_transpose, dim3((unsigned)((n + 63) / 64)), dim3(64, 16), 0, s, g->mdist, g->n, kk,
                            pl->mres + (int64_t)s0 * n);
       }
