@@ -119,13 +119,15 @@ typedef struct {
                                   iteration is two streaming passes through LDS instead of random gathers */
 #define SMDP_LAYOUT_HOT     3  /* SSSP/BFS tuned: the solve runs on a copy of the graph with vertices renumbered by
                                   falling in-degree (built once per resident graph; results are reported in the
-                                  caller's numbering).  Automatic picks it for resident graphs of >= 2^20 arcs. */
+                                  caller's numbering).  Automatic picks it for BFS on resident graphs of more than
+                                  2^25 arcs (or 2^23 vertices); smaller ones are solved on the graph as given, in one
+                                  launch. */
 #define SMDP_LAYOUT_BUCKETS 4  /* SSSP tuned: bucketed rounds (delta-stepping) on the renumbered copy.  Vertices are
                                   taken in order of distance buckets of width delta; within a bucket, arcs that stay in
                                   the bucket are relaxed until no distance in it changes, then every other arc of the
                                   bucket's vertices is relaxed once.  Automatic picks it for resident graphs of
-                                  >= 2^20 arcs without negative weights; a negative weight falls back to
-                                  SMDP_LAYOUT_HOT. */
+                                  >= 2^23 arcs (or more than 2^23 vertices and 2^20 arcs) without negative weights; a
+                                  negative weight falls back to SMDP_LAYOUT_HOT. */
 #define SMDP_LAYOUT_XCD8    8  /* sources split into 8 blocks, one per XCD, so each XCD gathers from a slice
                                   that fits its L2 */
 
@@ -301,8 +303,9 @@ int smdp_autotune(smdp_graph* gr, int app, int32_t src, const char* cache_path,
  * first (SMDP_ERR_ARG when row is not monotone from 0 to m or a column is out of
  * range).  All calls on one GPU share that array, so calls that overlap on one
  * GPU (from other threads or contexts) race.  Profiling is ignored, and
- * SMDP_SOL_TUNED runs unordered rounds on the graph as given (no renumbered
- * copy, no buckets). */
+ * SMDP_SOL_TUNED runs on the graph as given (no renumbered copy, no buckets):
+ * in one workgroup, in rounds of one launch, or in rounds the host drives, by
+ * size. */
 #define SMDP_NOALLOC_MAX_N (1 << 19)
 #define SMDP_NOALLOC_MAX_M (1 << 23)
 int smdp_sssp_device_noalloc(smdp_ctx* ctx, int32_t n, int32_t m, const int32_t* d_row, const int32_t* d_col,

@@ -368,7 +368,7 @@ int smdp_device_info(smdp_ctx* ctx, char* name, int name_len, char* arch, int ar
 int smdp_set_profiling(smdp_ctx* ctx, int on) {
   if (!ctx) return SMDP_ERR_ARG;
   SMDP_HIP(hipSetDevice(ctx->device));
-  if (on && !ctx->rlog) SMDP_CHECK(alloc_once(&ctx->rlog, 2 * (int64_t)kRoundLogCap));
+  if (on && !ctx->rlog) SMDP_CHECK(alloc_once(&ctx->rlog, 3 * (int64_t)kRoundLogCap));
   ctx->profiling = on ? 1 : 0;
   prof_reset(ctx);
   return SMDP_OK;
@@ -467,11 +467,12 @@ void smdp_graph_destroy(smdp_graph* g) {
     g->ctl = nullptr;
     g->cnt = nullptr;
     g->hq = nullptr;
+    g->rqueue = nullptr;
   }
   void* bufs[] = {g->row,    g->col,      g->w,       g->dist,     g->stamp,  g->hasout, g->q[0],  g->q[1],
                   g->hq,     g->ctl,      g->cnt,     g->val,      g->x,      g->y,     g->outdeg,
                   g->rank[0], g->rank[1], g->contrib, g->partials, g->chunk_part, g->prio, g->resume,
-                  g->rmax,   g->mdist,    g->tree_lo, g->tree_inner};
+                  g->rmax,   g->mdist,    g->tree_lo, g->tree_inner, g->rqueue};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   rowbufs_free(g);
@@ -576,16 +577,27 @@ int graph_create_transient(smdp_ctx* ctx, const smdp_csr* h, smdp_graph** out) {
                           al(4 * sizeof(Ctl)),                al(kCntParts * sizeof(Counters)),
                           al(4 * (size_t)n),                  al(4 * (size_t)n),  al(4 * (size_t)n),
                           al(4 * (size_t)n),                  al(sizeof(Chunk) * (size_t)hq_cap)};
-  size_t total = 0;
-  for (size_t b : sizes) total += b;
+  // k_rounds uses its own queues in place of the others
+  bool rounds = n <= kRoundMaxN && m <= kRoundMaxArcs;
+  const size_t rqueue = rounds ? al(2 * sizeof(RoundEntry) * (size_t)round_queue_cap(n, m)) : 0;
+  size_t plain = 0;
+  for (size_t b : sizes) plain += b;
+  const size_t total = std::max(plain, plain - sizes[7] - sizes[8] - sizes[9] + rqueue);
   if (total > ctx->arena_bytes) {
     if (ctx->arena) (void)hipFree(ctx->arena);
     ctx->arena = nullptr;
     ctx->arena_bytes = 0;
-    const size_t want = total + total / 4;
+    size_t want = total + total / 4;
     if (hipMalloc(&ctx->arena, want) != hipSuccess) {
+      // without k_rounds' queues
+      (void)hipGetLastError();
       ctx->arena = nullptr;
-      return SMDP_ERR_NOMEM;
+      rounds = false;
+      want = plain + plain / 4;
+      if (hipMalloc(&ctx->arena, want) != hipSuccess) {
+        ctx->arena = nullptr;
+        return SMDP_ERR_NOMEM;
+      }
     }
     ctx->arena_bytes = want;
   }
@@ -611,6 +623,7 @@ int graph_create_transient(smdp_ctx* ctx, const smdp_csr* h, smdp_graph** out) {
   g->q[1] = static_cast<int32_t*>(take(sizes[8]));
   g->hq = static_cast<Chunk*>(take(sizes[9]));
   g->hq_cap = hq_cap;
+  if (rounds) g->rqueue = reinterpret_cast<RoundEntry*>(g->q[0]);
   return graph_fill(ctx, h, g, out);
 }
 }  // namespace smdp

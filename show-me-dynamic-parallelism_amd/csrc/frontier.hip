@@ -29,6 +29,7 @@
 #include "device_common.h"
 #include "frontier.h"
 #include "lds_sssp.h"
+#include "rounds.h"
 #include "smdp_internal.h"
 
 namespace smdp {
@@ -813,7 +814,8 @@ static unsigned hasout_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, s
 int build_hasout(smdp_graph* g, const int32_t* row, uint32_t** out) {
   if (*out) return SMDP_OK;
   const int64_t nw = std::max<int64_t>(1, ((int64_t)g->n + 31) / 32);
-  SMDP_CHECK(alloc_once(out, nw));
+  if (g->hasout_mem) *out = g->hasout_mem;
+  else SMDP_CHECK(alloc_once(out, nw));
   hipLaunchKernelGGL(k_hasout, dim3(hasout_grid(g->n)), dim3(256), 0, g->ctx->stream, row, g->n, *out);
   SMDP_HIP(hipGetLastError());
   return SMDP_OK;
@@ -931,6 +933,99 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
                          ctx->profiling ? 0 : -1, false, st, true);
 }
 
+// Graphs whose rounds run in one launch (rounds.h), beyond those of use_lds.
+// Measured (device time, host-driven rounds or, for resident SSSP of 2^20 arcs
+// and more, buckets on the renumbered copy / one launch): SSSP RMAT-15 x 16
+// 550 / 208 us, RMAT-16 x 17 844 / 320, RMAT-17 x 16 1006 / 405 (buckets 673),
+// RMAT-18 x 16 buckets 798 / 700, RMAT-19 x 16 856 / 778, RMAT-20 x 8 845 /
+// 891, RMAT-20 x 16 1036 / 1916, uniform 2^18 x 8 buckets 1494 / 640, 2^20 x 4
+// 2663 / 984, 2^20 x 16 1605 / 2665: buckets from 2^23 arcs.  BFS: Zipf tree of
+// 50000 87 / 32, 2^18 119 / 49, 2^22 200 / 113, RMAT-17 x 16 233 / 169, RMAT-20
+// x 16 629 / 381, uniform 2^22 x 8 1102 / 964, RMAT-22 x 16 1059 / 1293.  The
+// renumbered copy, built on the host by the first run (143 ms for RMAT-20), is
+// not needed either.  Drop-in SSSP of 2^22 arcs and more keeps the rounds that
+// the host drives, whose launches its statistics report.
+static bool use_rounds(const smdp_params& p, const smdp_graph* g, bool bfs) {
+  if (p.layout != SMDP_LAYOUT_AUTO) return false;
+  if (g->hasout_mem) return g->n <= kRoundFixedN;  // the fixed array holds no larger queues
+  return g->n <= kRoundMaxN && g->m <= (bfs ? kRoundMaxArcs : g->transient ? kRoundMaxArcsDropin : kRoundMaxArcsSssp);
+}
+
+// Reads the per-round log of k_rounds: queue lengths, arcs and clocks.
+static int collect_rounds_log(smdp_ctx* ctx, int rounds) {
+  const int k = std::min(rounds, kRoundLogCap - 1);
+  std::vector<unsigned long long> h(3 * (size_t)kRoundLogCap);
+  SMDP_HIP(hipMemcpy(h.data(), ctx->rlog, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost));
+  int khz = 0;
+  SMDP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+  ctx->log_qlen.assign(k, 0);
+  ctx->log_arcs.assign(k, 0);
+  ctx->log_ms.assign(k, 0.0);
+  for (int i = 0; i < k; ++i) {
+    ctx->log_qlen[i] = (int64_t)h[2 * i];
+    ctx->log_arcs[i] = (int64_t)h[2 * i + 1];
+    const unsigned long long* clock = h.data() + 2 * kRoundLogCap + i;
+    if (khz > 0) ctx->log_ms[i] = (double)(clock[1] - clock[0]) / khz;
+  }
+  return SMDP_OK;
+}
+
+// Returns kRoundsRetry (and leaves the solve to the host-driven rounds) when
+// the workgroups were not all resident or there is no memory for the queues.
+static int run_rounds(smdp_graph* g, int32_t src, bool bfs, const smdp_params& p, smdp_stats* st) {
+  smdp_ctx* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  const int32_t inf = bfs ? SMDP_BFS_UNDEF : SMDP_SSSP_INF;
+  SMDP_CHECK(alloc_once(&g->dist, g->n));
+  if (!bfs) SMDP_CHECK(alloc_once(&g->stamp, g->n));
+  const int64_t qcap = round_queue_cap(g->n, g->m);
+  if (alloc_once(&g->rqueue, 2 * qcap) != SMDP_OK) {
+    (void)hipGetLastError();  // the host-driven rounds need less memory
+    return kRoundsRetry;
+  }
+  RoundArgs a;
+  a.row = g->row;
+  a.col = g->col;
+  a.w = g->w;
+  a.dist = g->dist;
+  a.stamp = bfs ? nullptr : g->stamp;
+  a.queue = g->rqueue;
+  a.ctl = reinterpret_cast<RoundCtl*>(g->ctl);
+  a.cnt = g->cnt;
+  a.n = g->n;
+  a.qcap = (int32_t)qcap;
+  a.rlog = ctx->profiling ? ctx->rlog : nullptr;
+  prof_reset(ctx);
+  a.rmax = (int32_t)std::min<int64_t>(p.max_rounds, (int64_t)g->n + 1);  // more rounds than vertices: a negative cycle
+  // Workgroups: RMAT-16 x 17 took 334 us on 128, 320 on 192, 326 on 256; uniform
+  // 33000 x 4 220 on 96 to 128, 235 on 192, 266 on 256.
+  const int grid = std::max(1, std::min({kRoundWgs, ctx->cus * 3 / 4, std::max(32, g->m / 1024)}));
+  SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
+  hipLaunchKernelGGL(k_rounds_init, dim3((unsigned)std::min<int64_t>(((int64_t)g->n + 255) / 256, 1024)), dim3(256), 0, s,
+                     a, inf, src);
+  SMDP_CHECK(prof_mark(ctx, 0));
+  if (bfs) hipLaunchKernelGGL(k_rounds<true>, dim3(grid), dim3(kRoundThreads), 0, s, a, inf);
+  else hipLaunchKernelGGL(k_rounds<false>, dim3(grid), dim3(kRoundThreads), 0, s, a, inf);
+  SMDP_HIP(hipGetLastError());
+  SMDP_CHECK(prof_mark(ctx, 0));
+  SMDP_HIP(hipMemcpyAsync(ctx->pinned, g->cnt, kCntParts * sizeof(Counters), hipMemcpyDeviceToHost, s));
+  SMDP_HIP(hipEventRecord(ctx->ev_end, s));
+  SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  const Counters* c = reinterpret_cast<const Counters*>(ctx->pinned);
+  unsigned long long end = 0, rounds = 0;
+  for (int i = 0; i < kCntParts; ++i) {
+    end = std::max(end, c[i].done);
+    rounds = std::max(rounds, c[i].rounds);
+  }
+  if (end == kRoundsRetry) return kRoundsRetry;
+  if (end) return SMDP_ERR_OVERFLOW;
+  float ms = 0;
+  SMDP_HIP(hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end));
+  if (a.rlog) SMDP_CHECK(collect_rounds_log(ctx, (int)rounds));
+  ctx->counters_staged = st != nullptr;
+  return finish_frontier(g, g->row, inf, bfs, false, ms, 2, -1, false, st, true);
+}
+
 // Runs SSSP (bfs = false) or BFS from src with the given solution; results stay
 // in g->dist.
 int run_frontier(smdp_graph* g, int32_t src, int sol, bool bfs, smdp_stats* st) {
@@ -944,11 +1039,15 @@ int run_frontier(smdp_graph* g, int32_t src, int sol, bool bfs, smdp_stats* st) 
   begin_run(g);
   const smdp_params& p = params_of(ctx, bfs ? SMDP_APP_BFS : SMDP_APP_SSSP);
   const bool tuned = sol == SMDP_SOL_TUNED;
-  const bool relabel = tuned && use_relabel(p, g);
-  if (tuned && !relabel && use_lds(p, g, bfs)) {
+  if (tuned && use_lds(p, g, bfs)) {
     const int rc = run_lds(g, src, bfs, st);
     if (rc != kLdsWeight) return rc;
   }
+  if (tuned && use_rounds(p, g, bfs)) {
+    const int rc = run_rounds(g, src, bfs, p, st);
+    if (rc != kRoundsRetry) return rc;
+  }
+  const bool relabel = tuned && use_relabel(p, g);
   SMDP_CHECK(ensure_frontier(g, tuned ? p.chunk : 0));
   const int32_t* row = g->row;
   const int32_t* col = g->col;
@@ -1099,7 +1198,9 @@ constexpr int64_t kQ0 = kStamp + align(4 * kMaxN);
 constexpr int64_t kQ1 = kQ0 + align(4 * kMaxN);
 constexpr int64_t kHasout = kQ1 + align(4 * kMaxN);
 constexpr int64_t kHq = kHasout + align(4 * ((kMaxN + 31) / 32));
+constexpr int64_t kRoundQueue = kQ0;  // k_rounds uses neither the queues nor the grid queue
 constexpr int64_t kEnd = kHq + align((int64_t)sizeof(Chunk) * kHqCap);
+static_assert(kRoundQueue + 2 * (int64_t)sizeof(RoundEntry) * kRoundFixedN <= kEnd, "its queues fit in their place");
 static_assert(kEnd <= kNoAllocScratchBytes, "the working buffers fit the fixed array");
 }  // namespace noalloc
 
@@ -1151,16 +1252,12 @@ int sssp_noalloc(smdp_ctx* ctx, int32_t n, int32_t m, const int32_t* d_row, cons
   g.q[1] = reinterpret_cast<int32_t*>(base + noalloc::kQ1);
   g.hq = reinterpret_cast<Chunk*>(base + noalloc::kHq);
   g.hq_cap = noalloc::kHqCap;
+  g.rqueue = reinterpret_cast<RoundEntry*>(base + noalloc::kRoundQueue);
   g.ctl = reinterpret_cast<Ctl*>(base + noalloc::kCtl);
   g.cnt = reinterpret_cast<Counters*>(base + noalloc::kCnt);
   g.transient = true;  // no renumbered copy
   g.forest = 0;
-  if (sol == SMDP_SOL_TUNED) {
-    // the has-arcs bits are rebuilt every call (the array keeps the last call's contents)
-    g.hasout = reinterpret_cast<uint32_t*>(base + noalloc::kHasout);
-    hipLaunchKernelGGL(k_hasout, dim3(hasout_grid(n)), dim3(256), 0, s, d_row, n, g.hasout);
-    SMDP_HIP(hipGetLastError());
-  }
+  g.hasout_mem = reinterpret_cast<uint32_t*>(base + noalloc::kHasout);
   // k_init_frontier clears the control blocks and counters and sets stamp; the
   // queues and the grid queue are written before they are read
   const int prof = ctx->profiling;

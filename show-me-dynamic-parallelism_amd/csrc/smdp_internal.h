@@ -21,6 +21,20 @@ namespace smdp {
 constexpr int kClaimParts = 8;
 constexpr int kClaimStride = 32;  // ints between two counters
 
+// Queue entry of k_rounds (rounds.h): the vertex's first arc in the high half
+// of x and the vertex in the low; the queued arcs before it in y.
+struct RoundEntry {
+  uint64_t x, y;
+};
+// What k_rounds solves: see use_rounds.
+constexpr int32_t kRoundMaxN = 1 << 23;
+constexpr int32_t kRoundFixedN = 1 << 18;  // with its queues in the fixed array
+constexpr int32_t kRoundMaxArcs = 1 << 25;
+constexpr int32_t kRoundMaxArcsSssp = (1 << 23) - 1;
+constexpr int32_t kRoundMaxArcsDropin = (1 << 22) - 1;
+// Entries of one queue: the vertices with arcs, and a source without.
+inline int64_t round_queue_cap(int64_t n, int64_t m) { return std::min(n, m + 1); }
+
 struct Ctl {
   int32_t qlen;        // frontier entries of this round
   int32_t hlen;        // grid-queue entries pushed during this round
@@ -203,6 +217,8 @@ struct smdp_graph {
   bool arena = false;        // row, col, w, ctl, cnt, dist, stamp, q and hq live in the context's arena
   int8_t forest = -1;        // every vertex has at most one in-arc: 1 yes, 0 no, -1 not checked yet
   uint32_t* hasout = nullptr; // tuned frontier: bit v set when row v has arcs
+  uint32_t* hasout_mem = nullptr;  // where hasout is built instead of memory of its own
+  smdp::RoundEntry* rqueue = nullptr;  // tuned frontier: the two queues of k_rounds (rounds.h)
   int32_t* tree_lo = nullptr; // tree: level bookkeeping and slots (tree.hip)
   int32_t* tree_inner = nullptr; // tree: per vertex, its arcs to vertices that have arcs (tree.hip)
 };
