@@ -936,12 +936,12 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
 // Graphs whose rounds run in one launch (rounds.h), beyond those of use_lds.
 // Measured (device time, host-driven rounds or, for resident SSSP of 2^20 arcs
 // and more, buckets on the renumbered copy / one launch): SSSP RMAT-15 x 16
-// 550 / 208 us, RMAT-16 x 17 844 / 320, RMAT-17 x 16 1006 / 405 (buckets 673),
-// RMAT-18 x 16 buckets 798 / 700, RMAT-19 x 16 856 / 778, RMAT-20 x 8 845 /
+// 550 / 201 us, RMAT-16 x 17 844 / 305, RMAT-17 x 16 1006 / 382 (buckets 673),
+// RMAT-18 x 16 buckets 798 / 626, RMAT-19 x 16 856 / 778, RMAT-20 x 8 845 /
 // 891, RMAT-20 x 16 1036 / 1916, uniform 2^18 x 8 buckets 1494 / 640, 2^20 x 4
 // 2663 / 984, 2^20 x 16 1605 / 2665: buckets from 2^23 arcs.  BFS: Zipf tree of
-// 50000 87 / 32, 2^18 119 / 49, 2^22 200 / 113, RMAT-17 x 16 233 / 169, RMAT-20
-// x 16 629 / 381, uniform 2^22 x 8 1102 / 964, RMAT-22 x 16 1059 / 1293.  The
+// 50000 87 / 32, 2^18 119 / 49, 2^22 200 / 114, RMAT-17 x 16 233 / 169, RMAT-20
+// x 16 629 / 322, uniform 2^22 x 8 1102 / 964, RMAT-22 x 16 1059 / 1293.  The
 // renumbered copy, built on the host by the first run (143 ms for RMAT-20), is
 // not needed either.  Drop-in SSSP of 2^22 arcs and more keeps the rounds that
 // the host drives, whose launches its statistics report.

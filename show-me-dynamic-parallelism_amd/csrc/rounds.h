@@ -4,7 +4,7 @@
 // drain kernel it took 33 us on RMAT-16 (65536 vertices, 2^20 arcs), most of
 // it with a few thousand arcs to do.  Here all rounds run in one launch of at
 // most kRoundWgs workgroups that meet at a barrier (5 us for a round of a few
-// arcs, 10 for some tens of thousands, 84 for RMAT-17's largest with 1.9
+// arcs, 10 for some tens of thousands, 80 for RMAT-17's largest with 1.9
 // million, where the loads and atomics of dist bind), and the chain is cut
 // down:
 // - A workgroup keeps what it queues in LDS, each entry with its vertex, first
@@ -31,7 +31,7 @@ namespace smdp {
 constexpr int kRoundWgs = 256;       // most workgroups (one per CU)
 constexpr int kRoundThreads = 1024;
 constexpr int kRoundOut = 8192;      // entries a workgroup keeps before they go to the queue
-constexpr int kRoundIlp = 4;         // arcs per thread and step
+constexpr int kRoundIlp = 2;         // arcs per thread and step
 
 // A workgroup's part of a queue: arcs before it and first entry in the high
 // and low half of at, entries in count.  Found with the queue's counters, it
@@ -137,62 +137,80 @@ struct RoundCount {
   uint32_t tries = 0, wins = 0, pushes = 0;
 };
 
-// Relaxes the window's arcs jb + thread + k * kRoundThreads below jend, K per
-// thread.  Wave-uniform.
+// Relaxes the window's arcs jb + K * thread + k below jend, K per thread.
+// Wave-uniform.  A thread's arcs follow one another, so one search finds them
+// all.  Two of them measured best: RMAT-17 x 16 382 us, three 388, four 392,
+// six 396; BFS on a tree of 4M 114, 121, 132, 153, on RMAT-20 322, 325, 341,
+// 334 (four arcs kRoundThreads apart, each with its search: 406, 113, 382).
 template <bool BFS, int K>
 __device__ __forceinline__ void round_arcs(const RoundArgs& a, RoundShared& sh, int jb, int jend, int top, int r,
                                            RoundCount& n) {
   const int lane = lane_id();
   int j[K], own[K], v[K], alt[K], seen[K];
+  const int j0 = jb + (int)threadIdx.x * K;
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    j[k] = min(jb + (int)threadIdx.x + k * kRoundThreads, jend - 1);
-    own[k] = 0;
+  for (int k = 0; k < K; ++k) j[k] = min(j0 + k, jend - 1);
+  own[0] = 0;
+  for (int step = top; step; step >>= 1) {
+    const int i = own[0] + step;
+    if (i < kRoundThreads && sh.of[min(i, kRoundThreads - 1)] <= j[0]) own[0] = i;
   }
-  for (int step = top; step; step >>= 1)
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i = own[k] + step;
-      if (i < kRoundThreads && sh.of[min(i, kRoundThreads - 1)] <= j[k]) own[k] = i;
-    }
+  for (int k = 1; k < K; ++k) {
+    own[k] = own[k - 1];
+    // every queued vertex has an arc, so the next arc is this entry's or the next's
+    if (own[k] + 1 < kRoundThreads && sh.of[min(own[k] + 1, kRoundThreads - 1)] <= j[k]) ++own[k];
+  }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int e = sh.st[own[k]] + j[k];
-    v[k] = stream_load(a.col + e);
-    alt[k] = BFS ? r + 1 : sh.du[own[k]] + stream_load(a.w + e);
+    v[k] = a.col[e];
+    alt[k] = BFS ? r + 1 : sh.du[own[k]] + a.w[e];
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) seen[k] = agent_load(a.dist + v[k]);
+  // Only the atomic is under a condition: loads in a branch were waited for
+  // there, slot after slot.  A lane without a candidate loads vertex 0's words.
   int old[K], stamp[K], st[K], deg[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
+    const bool want = j0 + k < jend && alt[k] < seen[k];
     old[k] = INT32_MIN;
-    stamp[k] = st[k] = deg[k] = 0;
-    if (jb + (int)threadIdx.x + k * kRoundThreads < jend && alt[k] < seen[k]) {
-      old[k] = atomicMin(&a.dist[v[k]], alt[k]);
-      if (!BFS) stamp[k] = agent_load(a.stamp + v[k]);
-      st[k] = a.row[v[k]];
-      deg[k] = a.row[v[k] + 1] - st[k];
-      ++n.tries;
-    }
+    if (want) old[k] = atomicMin(&a.dist[v[k]], alt[k]);
+    v[k] = want ? v[k] : 0;
+    n.tries += want;
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const bool won = old[k] != INT32_MIN && alt[k] < old[k];
+    stamp[k] = BFS ? 0 : agent_load(a.stamp + v[k]);
+    st[k] = a.row[v[k]];
+    deg[k] = a.row[v[k] + 1];
+  }
+  // the first of the round's improvements of v queues it; the flags stay in
+  // vector registers (K masks more spilled the scalar ones: 40 % slower)
+  int push[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    deg[k] -= st[k];
+    const int won = old[k] != INT32_MIN && alt[k] < old[k] ? 1 : 0;
     n.wins += won;
-    bool push = won && deg[k] > 0;
-    // the first of the round's improvements of v queues it
-    if (!BFS && push) push = stamp[k] != r + 1 && atomicExch(&a.stamp[v[k]], r + 1) != r + 1;
-    const uint64_t m = ballot(push);
+    push[k] = deg[k] > 0 && (BFS || stamp[k] != r + 1) ? won : 0;
+    asm("" : "+v"(push[k]));
+    if (!BFS && push[k]) stamp[k] = atomicExch(&a.stamp[v[k]], r + 1);
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const bool push_k = push[k] && (BFS || stamp[k] != r + 1);
+    const uint64_t m = ballot(push_k);
     if (!m) continue;
-    const int incl = wave_scan_dpp(push ? deg[k] : 0);
+    const int incl = wave_scan_dpp(push_k ? deg[k] : 0);
     const int arcs = __builtin_amdgcn_readlane(incl, SMDP_WAVE - 1);
     unsigned long long at = 0;
     if (lane == 0) at = atomicAdd(&sh.out, (unsigned long long)__popcll(m) << 32 | (uint32_t)arcs);
     const int before = __builtin_amdgcn_readfirstlane((int)(uint32_t)at);
     const int pos = __builtin_amdgcn_readfirstlane((int)(at >> 32)) + mbcnt(m);
-    n.pushes += push;
-    if (push) {
+    n.pushes += push_k;
+    if (push_k) {
       sh.v[pos] = v[k];
       sh.start[pos] = st[k];
       sh.before[pos] = before + incl - deg[k];
