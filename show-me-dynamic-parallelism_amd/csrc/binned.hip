@@ -17,10 +17,9 @@
 //    bin-major value array, each segment a run of its own.
 //  * reduce (k_bin_reduce): a work item is one bin.  Its values are one
 //    contiguous run; the workgroup copies them into LDS at each arc's in-CSR
-//    position, sums every row from LDS in arc order with the compensated sum
-//    of device_common.h and runs the PageRank epilogue.  Rows of at least
-//    kBinWide arcs have a bin of their own, cut into pieces; the last
-//    workgroup merges each wide row's piece sums in order.
+//    position, sums every row from LDS in FP64 and runs the PageRank epilogue.
+//    Rows of at least kBinWide arcs have a bin of their own, cut into pieces;
+//    the last workgroup merges each wide row's piece sums in order.
 // Per arc and iteration the passes move 2 + 4 bytes (scatter) and 4 + 2 bytes
 // (reduce).  Results do not depend on the schedule: every light row is summed
 // in in-CSR arc order by one thread, every heavy row by one wave in a fixed
@@ -62,7 +61,7 @@ constexpr int kFront = 4;                     // entries before vals and dst: a 
 constexpr int kSrcPad = kScatterBlock + 8;    // entries past m in src: a scatter block may read that far
 constexpr int64_t kMaxSegments = int64_t(1) << 27;  // bound on nchunks x nbins (host plan memory)
 
-static_assert(kBinCap <= 65535 && kSrcChunk <= 65536, "positions and offsets are stored in 16 bits");
+static_assert(4 * kBinCap <= 65535 && kSrcChunk <= 65536, "positions (in bytes) and offsets are stored in 16 bits");
 static_assert(kBinWide <= kBinCap, "a row below kBinWide always fits in a bin");
 static_assert(kSrcChunk % (4 * kScatNT) == 0, "contributions are loaded as float4, kSrcChunk/4/kScatNT each");
 
@@ -172,16 +171,74 @@ __device__ __forceinline__ double2 bin_sum2(double2 v, double2* lds) {
   return t;
 }
 
+// What a thread holds of one bin of rows: its loads are issued while the bin
+// before it is summed.
+struct BinRegs {
+  static constexpr int kRowLoads = (kBinRows + 1 + kBinNT - 1) / kBinNT;
+  int roff[kRowLoads];
+  uint16_t perm[kRowsPerThread];
+  f32x4 v[kQuads];
+  u16x4 dd[kQuads];
+};
+
+// p[i] of a uniform p, at a 32-bit offset (one register instead of two).
+template <typename T>
+__device__ __forceinline__ const T& at(const T* p, int i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (uint32_t)i * (uint32_t)sizeof(T));
+}
+
+// s[off / 4] = x.
+__device__ __forceinline__ void store_at(float* s, uint16_t off, float x) {
+  *reinterpret_cast<float*>(reinterpret_cast<char*>(s) + off) = x;
+}
+
+// Issues every load that the sums of the bin d0 need: row offsets, the degree
+// order and the whole run of values and positions (kQuads groups of 4 arcs
+// per thread cover a full bin).
+// Loads go to clamped positions (a bin has at least one row; a bin without
+// arcs loads the group of 4 below its start, kFront entries of padding at arc
+// 0): a load under a per-lane condition made the compiler wait for it before
+// the next one, which held back the bin's value loads by three round trips.
+// Values loaded past nr or outside [beg, end) are never used.
+__device__ __forceinline__ void bin_load(const RArgs& a, const BArgs& b, const int4& d0, BinRegs& g) {
+  const int beg = d0.x, end = d0.y, r0 = d0.z, nr = d0.w;
+  const int a0 = beg & ~3;
+  const int nq = (end - a0 + 3) >> 2;
+#pragma unroll
+  for (int q = 0; q < BinRegs::kRowLoads; ++q) g.roff[q] = at(a.row + r0, min((int)threadIdx.x + q * kBinNT, nr));
+#pragma unroll
+  for (int q = 0; q < kRowsPerThread; ++q) {
+    const int r = min((int)threadIdx.x + q * kBinNT, nr - 1);
+    g.perm[q] = at(b.rperm + r0, r);
+  }
+  static_assert(kQuads * kBinNT * 4 >= kBinCap + 3, "one round of quads covers a bin");
+#pragma unroll
+  for (int t = 0; t < kQuads; ++t) {
+    const int qi = min(t * kBinNT + (int)threadIdx.x, nq - 1);
+    // (from the group below: a bin without arcs has qi = -1)
+    g.v[t] = __builtin_nontemporal_load(&at(reinterpret_cast<const f32x4*>(b.vals + a0) - 1, qi + 1));
+    g.dd[t] = __builtin_nontemporal_load(&at(reinterpret_cast<const u16x4*>(b.dst + a0) - 1, qi + 1));
+  }
+}
+
 // Reduce items are claimed from a counter, one at a time (about 4300 claims per
 // RMAT-22 iteration, well within one counter's rate; eight partitioned
-// counters were measured 10% slower here).  A workgroup claims
-// its next item when it starts one and reads that item's descriptor while it
-// sums the rows of the current one, so neither latency is on its path.
-__global__ __launch_bounds__(kBinNT, 2) void k_bin_reduce(RArgs a, BArgs b, int k) {
+// counters were measured 10% slower here).  A workgroup claims two items
+// ahead: the claim and the descriptor of an item return while the one before
+// the last is summed, and a bin's loads are issued before the rows of the bin
+// before it are summed, so the memory has work during the sums.  Rows are
+// summed in FP64 (two instructions per arc, where a compensated FP32 sum
+// takes seven), and only a wave that holds an end of the bin tests its arcs
+// one by one.  On RMAT-22 (67M arcs) a pass went from 136 to 126 us: 4 TB/s
+// over the 500 MB of arcs and rows it moves; without the sums it takes 113,
+// without LDS stores as well 112.  Two workgroups per CU need at most 128
+// registers (one took 157 us): hence the scalar descriptors and the 32-bit
+// offsets.
+__global__ __launch_bounds__(kBinNT, 4) void k_bin_reduce(RArgs a, BArgs b, int k) {
   if (a.st->done) return;
   const float base = iteration_base(a, k);
   const int lane = lane_id();
-  const int wave = threadIdx.x / SMDP_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SMDP_WAVE);
   __shared__ float s_v[kBinCap];
   __shared__ uint16_t s_row[kBinRows + 2];  // row offsets in the bin
   __shared__ uint16_t s_perm[kBinRows];     // the bin's rows by falling degree
@@ -190,115 +247,114 @@ __global__ __launch_bounds__(kBinNT, 2) void k_bin_reduce(RArgs a, BArgs b, int 
   __shared__ int s_next;
   __shared__ float2 s_red[kW];
   __shared__ double2 s_red2[kW];
-  unsigned long long edges = 0, rows = 0, pushes = 0;
+  uint32_t edges = 0, rows = 0, pushes = 0;  // of the launch's part of a pass: below 2^31 arcs
   const int nitems = b.nitems;
-  if (threadIdx.x == 0) s_next = atomicAdd(&a.st->work_next, 1);
+  // ---- pieces of wide rows: one compensated sum over a contiguous run each
+  for (int p = blockIdx.x; p < b.npieces; p += gridDim.x) {
+    const int4 d = b.r_item[2 * p];
+    const int a0 = d.x & ~3;
+    const int nq = (d.y - a0 + 3) >> 2;
+    CSum acc;
+    for (int qb = 0; qb < nq; qb += kQuads * kBinNT) {
+      f32x4 v[kQuads];
+#pragma unroll
+      for (int t = 0; t < kQuads; ++t) {
+        const int qi = min(qb + t * kBinNT + (int)threadIdx.x, nq - 1);
+        v[t] = __builtin_nontemporal_load(&at(reinterpret_cast<const f32x4*>(b.vals + a0), qi));
+      }
+#pragma unroll
+      for (int t = 0; t < kQuads; ++t) {
+        const int qi = qb + t * kBinNT + (int)threadIdx.x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = a0 + 4 * qi + e;
+          if (qi < nq && j >= d.x && j < d.y) acc.add(v[t][e]);
+        }
+      }
+    }
+    if (threadIdx.x == 0) edges += d.y - d.x;
+    const CSum h = wg_csum<kBinNT>(acc, s_red);
+    if (threadIdx.x == 0) b.wpart[b.r_item[2 * p + 1].z] = make_float2(h.s, h.c);
+  }
+  // the first bin is the workgroup's own, the others are claimed from the counter
+  const int claims = b.npieces + (int)gridDim.x;
+  if (threadIdx.x == 0) s_next = claims + atomicAdd(&a.st->work_next, 1);
   __syncthreads();
-  int it = s_next;
+  // (item numbers are uniform: descriptors and what they point to take scalar registers)
+  int it = b.npieces + (int)blockIdx.x, it1 = __builtin_amdgcn_readfirstlane(s_next);
   __syncthreads();  // s_next is written again below
-  int4 d0 = make_int4(0, 0, 0, 0), d1 = make_int4(0, 0, 0, 0);
+  int4 d0 = make_int4(0, 0, 0, 0), d1 = d0, e0 = d0, e1 = d0;  // of this bin and the next
   if (it < nitems) {
     d0 = b.r_item[2 * it];
     d1 = b.r_item[2 * it + 1];
   }
+  if (it1 < nitems) {
+    e0 = b.r_item[2 * it1];
+    e1 = b.r_item[2 * it1 + 1];
+  }
+  BinRegs g;
+  if (it < nitems) bin_load(a, b, d0, g);
   while (it < nitems) {
     int nxt = 0;
-    if (threadIdx.x == 0) nxt = atomicAdd(&a.st->work_next, 1);  // the next item, claimed now
+    if (threadIdx.x == 0) nxt = claims + atomicAdd(&a.st->work_next, 1);  // the bin after the next, claimed now
     const int beg = d0.x, end = d0.y, r0 = d0.z, nr = d0.w;
     const int nwave_rows = d1.x, ngroup_rows = d1.y, part = d1.z;
     // the run [beg, end) is read as aligned groups of 4 arcs
     const int a0 = beg & ~3;
     const int nq = (end - a0 + 3) >> 2;
-    if (nr < 0) {
-      // ---- a piece of a wide row: one compensated sum over a contiguous run
-      if (threadIdx.x == 0) s_next = nxt;
-      __syncthreads();
-      it = s_next;
-      if (it < nitems) {
-        d0 = b.r_item[2 * it];
-        d1 = b.r_item[2 * it + 1];
-      }
-      CSum acc;
-      for (int qb = 0; qb < nq; qb += kQuads * kBinNT) {
-        f32x4 v[kQuads];
+    // ---- a bin of rows, loaded into g
 #pragma unroll
-        for (int t = 0; t < kQuads; ++t) {
-          const int qi = min(qb + t * kBinNT + (int)threadIdx.x, nq - 1);
-          v[t] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(b.vals + a0) + qi);
-        }
-#pragma unroll
-        for (int t = 0; t < kQuads; ++t) {
-          const int qi = qb + t * kBinNT + (int)threadIdx.x;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int j = a0 + 4 * qi + e;
-            if (qi < nq && j >= beg && j < end) acc.add(v[t][e]);
-          }
-        }
-      }
-      if (threadIdx.x == 0) edges += end - beg;
-      const CSum h = wg_csum<kBinNT>(acc, s_red);
-      if (threadIdx.x == 0) b.wpart[part] = make_float2(h.s, h.c);
-      continue;
-    }
-    // ---- a bin of rows.  Every load the bin needs is issued before any of
-    // them is used: row offsets, the degree order, old ranks and
-    // out-degrees of this thread's rows, and the whole run of values and
-    // positions (kQuads groups of 4 arcs per thread cover a full bin).
-    constexpr int kRowLoads = (kBinRows + 1 + kBinNT - 1) / kBinNT;
-    int roff[kRowLoads];
-    uint16_t perm[kRowsPerThread];
-    float rold[kRowsPerThread];
-    int od[kRowsPerThread];
-    // Loads go to clamped positions (a bin has at least one row; a bin without
-    // arcs loads the group of 4 below its start, kFront entries of padding at
-    // arc 0): a load under a per-lane condition made the compiler wait for it
-    // before the next one, which held back the bin's value loads by three
-    // round trips.  Values loaded past nr or outside [beg, end) are never used.
-#pragma unroll
-    for (int q = 0; q < kRowLoads; ++q) roff[q] = a.row[r0 + min((int)threadIdx.x + q * kBinNT, nr)];
-#pragma unroll
-    for (int q = 0; q < kRowsPerThread; ++q) {
-      const int r = r0 + min((int)threadIdx.x + q * kBinNT, nr - 1);
-      perm[q] = b.rperm[r];
-      rold[q] = a.rold[r];
-      od[q] = a.outdeg[r];
-    }
-    static_assert(kQuads * kBinNT * 4 >= kBinCap + 3, "one round of quads covers a bin");
-    f32x4 v[kQuads];
-    u16x4 dd[kQuads];
-#pragma unroll
-    for (int t = 0; t < kQuads; ++t) {
-      const int qi = min(t * kBinNT + (int)threadIdx.x, nq - 1);
-      v[t] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(b.vals + a0) + qi);
-      dd[t] = __builtin_nontemporal_load(reinterpret_cast<const u16x4*>(b.dst + a0) + qi);
-    }
-#pragma unroll
-    for (int q = 0; q < kRowLoads; ++q) {
+    for (int q = 0; q < BinRegs::kRowLoads; ++q) {
       const int i = (int)threadIdx.x + q * kBinNT;
-      if (i <= nr) s_row[i] = (uint16_t)(roff[q] - beg);
+      if (i <= nr) s_row[i] = (uint16_t)(g.roff[q] - beg);
     }
 #pragma unroll
     for (int q = 0; q < kRowsPerThread; ++q) {
       const int r = (int)threadIdx.x + q * kBinNT;
-      if (r < nr) s_perm[r] = perm[q];
+      if (r < nr) s_perm[r] = g.perm[q];
     }
 #pragma unroll
     for (int t = 0; t < kQuads; ++t) {
-      const int qi = t * kBinNT + (int)threadIdx.x;
+      const int q0 = t * kBinNT + wave * SMDP_WAVE;  // the wave's first group
+      if (q0 > 0 && q0 + SMDP_WAVE < nq) {
+        // whole groups of the bin's: no arc of them needs a test
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int j = a0 + 4 * qi + e;
-        if (qi < nq && j >= beg && j < end) s_v[dd[t][e]] = v[t][e];
+        for (int e = 0; e < 4; ++e) store_at(s_v, g.dd[t][e], g.v[t][e]);
+      } else if (q0 < nq) {
+        const int qi = q0 + lane;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = a0 + 4 * qi + e;
+          if (qi < nq && j >= beg && j < end) store_at(s_v, g.dd[t][e], g.v[t][e]);
+        }
       }
     }
     if (threadIdx.x == 0) s_next = nxt;
     __syncthreads();
-    it = s_next;
+    it = it1;
+    it1 = __builtin_amdgcn_readfirstlane(s_next);
+    // after the last bin its own loads are made again (a load under a condition
+    // kept the registers of both sides)
     if (it < nitems) {
-      d0 = b.r_item[2 * it];
-      d1 = b.r_item[2 * it + 1];
+      d0 = e0;
+      d1 = e1;
     }
+    // for the epilogue of this bin, and the next one's loads
+    float rold[kRowsPerThread];
+    int od[kRowsPerThread];
+#pragma unroll
+    for (int q = 0; q < kRowsPerThread; ++q) {
+      const int r = min((int)threadIdx.x + q * kBinNT, nr - 1);
+      rold[q] = at(a.rold + r0, r);
+      od[q] = at(a.outdeg + r0, r);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    bin_load(a, b, d0, g);
+    if (it1 < nitems) {
+      e0 = b.r_item[2 * it1];
+      e1 = b.r_item[2 * it1 + 1];
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // Row sums.  Rows in falling degree order: the first nwave_rows take a
     // wave each, the next ngroup_rows 8 lanes each, the rest one lane each,
     // so the lanes of one task have rows of about the same length.
@@ -310,35 +366,35 @@ __global__ __launch_bounds__(kBinNT, 2) void k_bin_reduce(RArgs a, BArgs b, int 
       if (task < nwave_rows) {
         const int r = s_perm[task];
         const int s = s_row[r], e = s_row[r + 1];
-        CSum acc;
+        double acc = 0.0;
         int q = s + lane;
         for (; q + 3 * SMDP_WAVE < e; q += 4 * SMDP_WAVE) {
           const float x0 = s_v[q], x1 = s_v[q + SMDP_WAVE], x2 = s_v[q + 2 * SMDP_WAVE], x3 = s_v[q + 3 * SMDP_WAVE];
-          acc.add(x0);
-          acc.add(x1);
-          acc.add(x2);
-          acc.add(x3);
+          acc += (double)x0;
+          acc += (double)x1;
+          acc += (double)x2;
+          acc += (double)x3;
         }
-        for (; q < e; q += SMDP_WAVE) acc.add(s_v[q]);
-        acc = wave_csum_dpp(acc);
-        if (lane == 0) s_res[r] = acc.value();
+        for (; q < e; q += SMDP_WAVE) acc += (double)s_v[q];
+        acc = wave_sum_dpp(acc);
+        if (lane == 0) s_res[r] = (float)acc;
       } else if (task < nwave_rows + ngroup_tasks) {
         const int i = nwave_rows + (task - nwave_rows) * (SMDP_WAVE / kRowGroup) + lane / kRowGroup;
         const bool valid = i < nwave_rows + ngroup_rows;
         const int r = valid ? s_perm[i] : 0;
         const int s = valid ? s_row[r] : 0, e = valid ? s_row[r + 1] : 0;
-        CSum acc;
-        for (int q = s + (lane & (kRowGroup - 1)); q < e; q += kRowGroup) acc.add(s_v[q]);
-        acc = group8_csum(acc);
-        if (valid && (lane & (kRowGroup - 1)) == 4) s_res[r] = acc.value();
+        double acc = 0.0;
+        for (int q = s + (lane & (kRowGroup - 1)); q < e; q += kRowGroup) acc += (double)s_v[q];
+        acc = group8_sum_dpp(acc);
+        if (valid && (lane & (kRowGroup - 1)) == 4) s_res[r] = (float)acc;
       } else {
         const int i = nwave_rows + ngroup_rows + (task - nwave_rows - ngroup_tasks) * SMDP_WAVE + lane;
         if (i < nr) {
           const int r = s_perm[i];
           const int s = s_row[r], e = s_row[r + 1];
-          CSum acc;
-          for (int q = s; q < e; ++q) acc.add(s_v[q]);
-          s_res[r] = acc.value();
+          double acc = 0.0;
+          for (int q = s; q < e; ++q) acc += (double)s_v[q];
+          s_res[r] = (float)acc;
         }
       }
     }
@@ -497,7 +553,7 @@ int binned_ensure(smdp_graph* g, void** slot, BArgs* out) {
         const int32_t u = col[e];
         const int32_t c = u >> kSrcChunkLog;
         src[cs[(size_t)c]++] = (uint16_t)(u & (kSrcChunk - 1));
-        dst[(size_t)kFront + bs[(size_t)c]++] = wide[b] ? 0 : (uint16_t)(e - e0);
+        dst[(size_t)kFront + bs[(size_t)c]++] = wide[b] ? 0 : (uint16_t)(4 * (e - e0));
       }
     }
   });
@@ -555,7 +611,7 @@ int binned_ensure(smdp_graph* g, void** slot, BArgs* out) {
   }
   // reduce: items in row order (bins, and the pieces of each wide row),
   // claimed by the workgroups one at a time
-  std::vector<int4> r_item;
+  std::vector<int4> r_item, bins;  // pieces of wide rows, then bins of rows
   std::vector<int32_t> wfirst(1, 0), wrow;
   int32_t nparts = 0, npieces = 0;
   for (int64_t b = 0; b < B; ++b) {
@@ -570,8 +626,8 @@ int binned_ensure(smdp_graph* g, void** slot, BArgs* out) {
       wrow.push_back(brow[b]);
     } else {
       const int32_t nr = brow[b + 1] - brow[b];
-      r_item.push_back(make_int4(e0, e1, brow[b], nr));
-      r_item.push_back(make_int4(bcls[(size_t)(2 * b)], bcls[(size_t)(2 * b + 1)], nparts++, 0));
+      bins.push_back(make_int4(e0, e1, brow[b], nr));
+      bins.push_back(make_int4(bcls[(size_t)(2 * b)], bcls[(size_t)(2 * b + 1)], nparts++, 0));
     }
   }
 
@@ -587,6 +643,7 @@ int binned_ensure(smdp_graph* g, void** slot, BArgs* out) {
   step(upload(&p->rperm, rperm));
   step(upload(&p->s_item, s_item));
   step(upload(&p->s_group, s_group));
+  r_item.insert(r_item.end(), bins.begin(), bins.end());
   step(upload(&p->r_item, r_item));
   step(upload(&p->wfirst, wfirst));
   step(upload(&p->wrow, wrow));
@@ -615,6 +672,7 @@ int binned_ensure(smdp_graph* g, void** slot, BArgs* out) {
   a.nbins = (int32_t)B;
   a.nsgroups = (int32_t)(s_group.size() - 1);
   a.nitems = (int32_t)(r_item.size() / 2);
+  a.npieces = npieces;
   a.nwide = (int32_t)wrow.size();
   a.nparts = nparts;
   *slot = p;

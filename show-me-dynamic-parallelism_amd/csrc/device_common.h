@@ -305,6 +305,12 @@ __device__ __forceinline__ double dpp_d(double x) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
   return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
+// Sum of each aligned group of 8 lanes, read from lane 4 of the group.
+__device__ __forceinline__ double group8_sum_dpp(double x) {
+  x += dpp_d<kDppXor1>(x);
+  x += dpp_d<kDppXor2>(x);
+  return x + dpp_d<kDppShr4>(x);
+}
 __device__ __forceinline__ double wave_sum_dpp(double x) {
   x += dpp_d<kDppXor1>(x);
   x += dpp_d<kDppXor2>(x);

@@ -72,14 +72,14 @@ struct BArgs {
   const int32_t* __restrict__ cm;      // nchunks x (nbins+1): start of segment (c, b) in src; [c][nbins] = end of c
   const int32_t* __restrict__ bm;      // nchunks x nbins: start of segment (c, b) in vals and dst
   const uint16_t* __restrict__ src;    // chunk-major: source id minus its chunk's first id
-  const uint16_t* __restrict__ dst;    // bin-major: the arc's position in its bin, in in-CSR order
+  const uint16_t* __restrict__ dst;    // bin-major: 4 x the arc's position in its bin, in in-CSR order
   float* vals;                         // bin-major: the source's contribution, written by the scatter pass
   const uint16_t* __restrict__ rperm;  // per row: the rows of its bin by falling degree (index in the bin)
   const int32_t* __restrict__ s_item;  // scatter items: (chunk, first bin, end bin, first arc, end arc in src)
   const int32_t* __restrict__ s_group; // scatter workgroup g takes items s_group[g] .. s_group[g+1]-1
   const int4* __restrict__ r_item;     // reduce items, two int4 each: (beg, end, r0, nr), (nwave, ngroup, part, 0);
-                                       // nr < 0 marks a piece of a wide row, part indexes wpart, else bpart
-
+                                       // the pieces of wide rows (nr < 0, part indexes wpart) come first, then
+                                       // the bins of rows (part indexes bpart)
   const int32_t* __restrict__ wfirst;  // nwide+1: first piece of each wide row
   const int32_t* __restrict__ wrow;    // nwide: the wide rows
   float2* wpart;                       // per wide piece: (sum, error)
@@ -87,7 +87,8 @@ struct BArgs {
   int32_t nchunks;
   int32_t nbins;
   int32_t nsgroups;                    // scatter workgroups
-  int32_t nitems;                      // reduce items (claimed from RState::work_next)
+  int32_t nitems;                      // reduce items (bins are claimed from RState::work_next)
+  int32_t npieces;                     // of them, pieces of wide rows
   int32_t nwide;
   int32_t nparts;                      // bins of rows (entries of bpart)
 };
