@@ -36,8 +36,8 @@ namespace smdp {
 namespace {
 
 constexpr int kMpNT = 256;                // threads per workgroup
-// Merge items per thread: kMpBig where the tiles fill the device many times
-// over, kMpSmall where they would not (see items_per_thread).
+// Merge items per thread of a product: kMpBig where the tiles fill the device
+// many times over, kMpSmall where they would not (see items_per_thread).
 constexpr int kMpBig = 16;
 constexpr int kMpSmall = 4;
 
@@ -81,6 +81,18 @@ struct MArgs {
 // two kMpBig tiles per CU.
 int items_per_thread(int64_t total, int cus) {
   return total <= (int64_t)cus * kMpNT * kMpBig * 2 ? kMpSmall : kMpBig;
+}
+
+// The same for a PageRank iteration, which every workgroup ends with a fence
+// and a ticket, so fewer and larger tiles pay earlier.  Microseconds an
+// iteration with 4, 8, 16 and 32 items: 74K items 13.5, 13.9, 17.1, 23.2; 147K
+// 14.9, 14.6, 17.8, 24.2; 279K 18.7, 16.3, 17.7, 23.7; 557K 27.6, 21.6, 19.9,
+// 24.4; 1.11M 52.8, 34.7, 25.5, 27.2; 2.23M 99.7, 62.9, 37.8, 34.0; 4.46M 153,
+// 121, 79.7, 60.8.
+int items_per_thread_pr(int64_t total, int cus) {
+  if (total <= 550 * (int64_t)cus) return 4;
+  if (total <= 1600 * (int64_t)cus) return 8;
+  return total <= 5000 * (int64_t)cus ? 16 : 32;
 }
 
 // Number of row ends among the first d merge items: the smallest i with
@@ -347,10 +359,10 @@ __global__ void k_merge_fixup(MArgs a) {
 //
 // What bounds it below 2^20 arcs is the chain of one tile (row ends, columns,
 // gathers, walk, scan, epilogue) and the launch, not bytes: 262K arcs and 16K
-// rows take about 10 us an iteration.  The row-tile kernel it replaces took
-// 157 us there: 64 tiles of 256 rows on 64 of the 256 CUs, with each row of
-// 64 or more arcs summed by one wave after another.  A drop-in PageRank of
-// RMAT-14 went from 2.55 to 0.47 ms.
+// rows take 16 us an iteration.  The row-tile kernel it replaces took 157 us
+// there: 64 tiles of 256 rows on 64 of the 256 CUs, with each row of 64 or
+// more arcs summed by one wave after another.  A drop-in PageRank of RMAT-14
+// went from 2.55 to 0.43 ms.
 template <int kMpT>
 __global__ __launch_bounds__(kMpNT) void k_pr_merge(RArgs a, MArgs p, int k) {
   if (a.st->done) return;
@@ -548,7 +560,7 @@ static int ensure_merge(smdp_graph* g, void** slot, bool spmv, hipStream_t s, Me
   mp = new MergePlan();
   *slot = mp;
   const int64_t total = (int64_t)g->n + g->m;
-  mp->items = kMpNT * items_per_thread(total, g->ctx->cus);
+  mp->items = kMpNT * (spmv ? items_per_thread(total, g->ctx->cus) : items_per_thread_pr(total, g->ctx->cus));
   mp->ntiles = (int32_t)((total + mp->items - 1) / mp->items);
   const int64_t nt = std::max<int64_t>(1, mp->ntiles);
   SMDP_CHECK(alloc_once(&mp->tstart, nt + 1));
@@ -626,10 +638,13 @@ void merge_pagerank_pass(smdp_graph* g, void* slot, int grid, const RArgs& a, in
   const MArgs p = merge_args(g, mp);
   const dim3 gd(std::max(1, std::min(grid, mp->ntiles)));
   prof_mark(g->ctx, 0);
-  if (mp->items == kMpNT * kMpSmall)
-    hipLaunchKernelGGL(k_pr_merge<kMpSmall>, gd, dim3(kMpNT), 0, g->ctx->stream, a, p, k);
-  else
-    hipLaunchKernelGGL(k_pr_merge<kMpBig>, gd, dim3(kMpNT), 0, g->ctx->stream, a, p, k);
+  hipStream_t s = g->ctx->stream;
+  switch (mp->items / kMpNT) {
+    case 4: hipLaunchKernelGGL(k_pr_merge<4>, gd, dim3(kMpNT), 0, s, a, p, k); break;
+    case 8: hipLaunchKernelGGL(k_pr_merge<8>, gd, dim3(kMpNT), 0, s, a, p, k); break;
+    case 16: hipLaunchKernelGGL(k_pr_merge<16>, gd, dim3(kMpNT), 0, s, a, p, k); break;
+    default: hipLaunchKernelGGL(k_pr_merge<32>, gd, dim3(kMpNT), 0, s, a, p, k); break;
+  }
   prof_mark(g->ctx, 0);
   ++*launches;
 }

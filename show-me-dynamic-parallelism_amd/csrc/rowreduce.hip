@@ -604,11 +604,13 @@ static bool use_blocks(const smdp_params& p, int sol, int32_t) {
 }
 
 // The binned layout replaces every random gather of a PageRank iteration by
-// streamed runs; its one-time regrouping is worth it on graphs with at least
-// 2^20 arcs, where gathers miss L2.
+// streamed runs, which pays where the gathers miss L2.  Against merge-path
+// tiles, microseconds an iteration: RMAT-16 x 16 40 / 26, RMAT-17 x 16 48 /
+// 34, RMAT-18 x 16 (2^22 arcs) 62 / 61, RMAT-19 x 16 78 / 101.  Its plan, built
+// on the host by the first run, takes 19 ms for 2^22 arcs.
 static bool use_binned(const smdp_params& p, int sol, const smdp_graph* g) {
   if (sol != SMDP_SOL_TUNED) return false;
-  return p.layout == SMDP_LAYOUT_BINNED || (p.layout == SMDP_LAYOUT_AUTO && g->m >= (1 << 20));
+  return p.layout == SMDP_LAYOUT_BINNED || (p.layout == SMDP_LAYOUT_AUTO && g->m > (1 << 22));
 }
 
 template <bool PR>

@@ -74,3 +74,15 @@ def test_large_tiles(ctx):
         _check(ctx, smdp.invert(g))
     finally:
         ctx.set_params(smdp.APP_PAGERANK, **old.as_dict())
+
+
+# The largest matrix of each tile size (4, 8, 16 items a thread) on 256 CUs and the smallest of the next,
+# with a hub over many tiles, empty rows and a ragged end; and the last size before the binned layout.
+@pytest.mark.parametrize("total", [140800, 140801, 409600, 409601, 1280000, 1280001, 1 << 22])
+def test_tile_sizes_of_a_pass(ctx, total):
+    n = total // 9 + 1
+    lens = np.random.RandomState(total % 1000).randint(0, 9, n - 200)
+    lens[7] += total - n - lens.sum()
+    ig = _rows(lens, n, 11)
+    assert ig.n + ig.m == total and lens[7] > 4096
+    _check(ctx, ig)
