@@ -16,17 +16,21 @@
 //    later pass reads it (on the 4M-node Zipf tree 4.1M of the 4.2M vertices
 //    are leaves; level 4 holds 2.48M vertices of which 32.6K have children).
 //    The share's slot count is the sum of inner[u], each vertex's arcs to
-//    vertices that have arcs (counted once per graph); waves take positions
-//    in the reserved block from an LDS cursor.  An arc into the root, when
+//    vertices that have arcs (counted once per graph); the slots of u's
+//    children are consecutive, from first[u's slot] on.  An arc into the root, when
 //    the root has arcs, keeps its slot as a hole (-1); a forest has at most
 //    one.  The slots each level reserves are
 //    counted per level (rel), so a launch finds where its level ends from the
 //    one before without waiting for a last workgroup.
-//  * up (k_tree_up, one launch per level, deepest first): every vertex of
-//    level L pulls 1 + height[c] and 1 + desc[c] of its children (written by
-//    the down pass for leaves, by the launch for level L+1 otherwise) into LDS
+//  * up (k_tree_up, one launch per level, deepest first): a vertex's leaves
+//    are its arcs less inner[], and its other children are consecutive slots,
+//    whose heights and counts the launch for level L+1 left in their slots; so no
+//    leaf is read, and what is read is one run per workgroup.  Every vertex
+//    of level L pulls 1 + height and 1 + count of those children into LDS
 //    accumulators with integer atomics (max and add), in the same
-//    edge-balanced tiles, and stores its results.
+//    edge-balanced tiles, and stores its results, by vertex and by slot.  On
+//    the 4M-node tree (5 levels with children) a pass that pulled from every
+//    child took 118 us.
 // Integer max and add do not depend on order, so results are exact and the
 // same for every schedule.
 #include <hip/hip_runtime.h>
@@ -47,9 +51,11 @@ struct TArgs {
   const int32_t* __restrict__ col;
   const uint32_t* __restrict__ hasout;  // bit v set when v has children
   const int32_t* __restrict__ inner;    // inner[u]: arcs of u to vertices that have children
+  int32_t* first;   // per slot: first slot of its vertex's children; the up pass puts the vertex's descendants there
+                    // and its height into order (-1 in a hole)
   int32_t* order;   // reached vertices with children (and holes, -1) level by level
   int32_t* lo;      // lo[L]: first slot of level L (written by the launch for level L - 1)
-  int32_t* rel;     // rel[L]: slots reserved so far for level L + 1 (zeroed by the launch for level L - 1)
+  int32_t* rel;     // rel[L & 3]: slots reserved so far for level L + 1 (zeroed by the launch for level L - 1)
   int32_t* ctl;     // [1] number of levels, once a launch finds its level empty
   int32_t* height;
   int32_t* desc;
@@ -120,14 +126,14 @@ __global__ __launch_bounds__(SMDP_WG) void k_tree_down(TArgs a, int L) {
   __shared__ int s_start[SMDP_WG];
   __shared__ int s_off[SMDP_WG];
   __shared__ int s_scan[SMDP_WAVES_PER_WG];
+  __shared__ int s_slot[SMDP_WG];  // next slot for a child of the tile's vertex
   __shared__ int s_base;
-  __shared__ int s_cursor;
   // level L: from the end of level L - 1 for as many slots as level L - 1 reserved
   const int s = a.lo[L];
-  const int e = L == 0 ? 1 : s + a.rel[L - 1];
+  const int e = L == 0 ? 1 : s + a.rel[(L - 1) & 3];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.lo[L + 1] = e;  // for the launches after this one (none of this launch reads it)
-    a.rel[L + 1] = 0;
+    a.rel[(L + 1) & 3] = 0;
     if (e == s && a.ctl[1] == 0) {
       a.ctl[1] = L;  // level L is empty: levels 0 .. L-1
       atomicMax(&cnt_of(a.cnt)->rounds, (unsigned long long)L);
@@ -145,24 +151,26 @@ __global__ __launch_bounds__(SMDP_WG) void k_tree_down(TArgs a, int L) {
     }
     int total;
     (void)wg_exclusive_scan(part, s_scan, &total);
-    if (threadIdx.x == 0) {
-      s_base = total ? e + atomicAdd(&a.rel[L], total) : 0;
-      s_cursor = 0;
-    }
+    if (threadIdx.x == 0) s_base = total ? e + atomicAdd(&a.rel[L & 3], total) : 0;
     __syncthreads();
-    const int base = s_base;
+    int base = s_base;
     for (int t0 = b0; t0 < b1; t0 += SMDP_WG) {
       const int i = t0 + (int)threadIdx.x;
-      int u = -1, rs = 0, deg = 0;
+      int u = -1, rs = 0, deg = 0, inner = 0;
       if (i < b1) u = a.order[i];
       if (u >= 0) {
         rs = a.row[u];
         deg = a.row[u + 1] - rs;
+        inner = a.inner[u];
       }
-      int tot;
+      int tot, slots;
       const int ex = wg_exclusive_scan(deg, s_scan, &tot);
+      const int slot = base + wg_exclusive_scan(inner, s_scan, &slots);
+      base += slots;
+      if (i < b1) a.first[i] = slot;
       s_start[threadIdx.x] = rs;
       s_off[threadIdx.x] = ex;
+      s_slot[threadIdx.x] = slot;
       __syncthreads();
       for (int jb = 0; jb < tot; jb += kTreeIlp * SMDP_WG) {
         int j[kTreeIlp], own[kTreeIlp];
@@ -187,13 +195,7 @@ __global__ __launch_bounds__(SMDP_WG) void k_tree_down(TArgs a, int L) {
           }
           edges += ok;
           verts += child;
-          const uint64_t m = ballot(has);
-          if (m) {  // wave-uniform
-            int p = 0;
-            if (lane_id() == first_lane(m)) p = atomicAdd(&s_cursor, __popcll(m));
-            p = __shfl(p, first_lane(m));
-            if (has) a.order[base + p + mbcnt(m)] = child ? c[t] : -1;
-          }
+          if (has) a.order[atomicAdd(&s_slot[own[t]], 1)] = child ? c[t] : -1;
         }
       }
       __syncthreads();  // s_start / s_off are written again by the next tile
@@ -211,58 +213,56 @@ __global__ __launch_bounds__(SMDP_WG) void k_tree_down(TArgs a, int L) {
 }
 
 __global__ __launch_bounds__(SMDP_WG) void k_tree_up(TArgs a, int L) {
-  __shared__ int s_start[SMDP_WG];
   __shared__ int s_off[SMDP_WG];
   __shared__ int s_scan[SMDP_WAVES_PER_WG];
   __shared__ int s_h[SMDP_WG];
   __shared__ int s_d[SMDP_WG];
   const int s = a.lo[L], e = a.lo[L + 1];
   int b0, b1;
-  level_share(s, e, &b0, &b1);
+  level_share(s, e, &b0, &b1);  // the shares of the down pass: a tile's child slots are one run
   unsigned long long edges = 0;
   for (int t0 = b0; t0 < b1; t0 += SMDP_WG) {
     const int i = t0 + (int)threadIdx.x;
-    int u = -1, rs = 0, deg = 0;
+    int u = -1, inner = 0, leaves = 0;
     if (i < b1) u = a.order[i];
     if (u >= 0) {
-      rs = a.row[u];
-      deg = a.row[u + 1] - rs;
+      inner = a.inner[u];
+      leaves = a.row[u + 1] - a.row[u] - inner;
     }
+    const int first = a.first[t0];
     int tot;
-    const int ex = wg_exclusive_scan(deg, s_scan, &tot);
-    s_start[threadIdx.x] = rs;
+    const int ex = wg_exclusive_scan(inner, s_scan, &tot);
     s_off[threadIdx.x] = ex;
-    s_h[threadIdx.x] = 0;
-    s_d[threadIdx.x] = 0;
+    s_h[threadIdx.x] = leaves > 0;
+    s_d[threadIdx.x] = leaves;
     __syncthreads();
     for (int jb = 0; jb < tot; jb += kTreeIlp * SMDP_WG) {
-      int j[kTreeIlp], own[kTreeIlp], c[kTreeIlp];
+      int j[kTreeIlp], own[kTreeIlp], ch[kTreeIlp], cd[kTreeIlp];
 #pragma unroll
-      for (int t = 0; t < kTreeIlp; ++t) j[t] = min(jb + (int)threadIdx.x + t * SMDP_WG, tot - 1);
+      for (int t = 0; t < kTreeIlp; ++t) {
+        j[t] = min(jb + (int)threadIdx.x + t * SMDP_WG, tot - 1);
+        ch[t] = a.order[first + j[t]];
+        cd[t] = a.first[first + j[t]];
+      }
       tile_owners<kTreeIlp>(s_off, j, own);
 #pragma unroll
-      for (int t = 0; t < kTreeIlp; ++t) c[t] = stream_load(a.col + s_start[own[t]] + (j[t] - s_off[own[t]]));
-      int ch[kTreeIlp], cd[kTreeIlp];
-#pragma unroll
       for (int t = 0; t < kTreeIlp; ++t) {
-        // clamped gathers (the root's entries are valid); skipped below
-        ch[t] = a.height[c[t]];
-        cd[t] = a.desc[c[t]];
-      }
-#pragma unroll
-      for (int t = 0; t < kTreeIlp; ++t) {
-        const int jj = jb + (int)threadIdx.x + t * SMDP_WG;
-        if (jj < tot && c[t] != a.root) {
-          atomicMax(&s_h[own[t]], 1 + ch[t]);
+        if (jb + (int)threadIdx.x + t * SMDP_WG < tot) {
+          atomicMax(&s_h[own[t]], 1 + ch[t]);  // 0 for a hole
           atomicAdd(&s_d[own[t]], 1 + cd[t]);
           ++edges;
         }
       }
     }
     __syncthreads();
-    if (u >= 0) {
-      a.height[u] = s_h[threadIdx.x];
-      a.desc[u] = s_d[threadIdx.x];
+    if (i < b1) {
+      const int h = s_h[threadIdx.x], d = s_d[threadIdx.x];
+      if (u >= 0) {
+        a.height[u] = h;
+        a.desc[u] = d;
+      }
+      a.order[i] = u >= 0 ? h : -1;
+      a.first[i] = u >= 0 ? d : -1;
     }
     __syncthreads();  // the LDS arrays are written again by the next tile
   }
@@ -294,20 +294,21 @@ static int run_tree(smdp_graph* g, int32_t root, smdp_stats* st) {
                          ctx->stream, g->row, g->col, g->hasout, g->n, g->tree_inner);
     SMDP_HIP(hipGetLastError());
   }
-  // one buffer: level starts and per-level reservations (indices up to
-  // n + 2), the control line, and order[] (every reached vertex at most once
-  // plus at most one hole: n + 1 slots)
+  // one buffer: level starts (indices up to n + 2), the control line and the
+  // levels' reservations, and order[] and first[] (every reached vertex at
+  // most once plus at most one hole: n + 1 slots)
   const int64_t lo_len = (n + 3 + kTreeCtl - 1) / kTreeCtl * kTreeCtl;
-  SMDP_CHECK(alloc_once(&g->tree_lo, 2 * lo_len + kTreeCtl + n + 1));
+  SMDP_CHECK(alloc_once(&g->tree_lo, lo_len + 2 * kTreeCtl + 2 * (n + 1)));
   TArgs a;
   a.row = g->row;
   a.col = g->col;
   a.hasout = g->hasout;
   a.inner = g->tree_inner;
   a.lo = g->tree_lo;
-  a.rel = g->tree_lo + lo_len;
-  a.ctl = g->tree_lo + 2 * lo_len;
-  a.order = g->tree_lo + 2 * lo_len + kTreeCtl;
+  a.ctl = g->tree_lo + lo_len;
+  a.rel = a.ctl + kTreeCtl;
+  a.order = a.ctl + 2 * kTreeCtl;
+  a.first = a.order + (n + 1);
   a.height = g->dist;
   a.desc = g->stamp;
   a.cnt = g->cnt;
@@ -322,7 +323,7 @@ static int run_tree(smdp_graph* g, int32_t root, smdp_stats* st) {
   ++launches;
   // Down, in batches of levels, until a launch finds its level empty:
   // order[] holds at most n + 1 slots, so level n + 1 is empty at the latest
-  // (lo and rel are indexed up to n + 2).
+  // (lo is indexed up to n + 2).
   // (an empty level's launch costs ~4 us; a host check between batches about
   // 100 us, so the first batch covers the usual depths)
   int L = 0, levels = 0;
