@@ -1287,10 +1287,18 @@ static int ensure_buckets(smdp_graph* g, Relabel* rl, int delta) {
 // reached vertices' out-arcs to the counters, which are then already in the
 // context's pinned buffer (counters_staged).  The copy must have no negative
 // weight.
+// Workgroups per CU of a phase at most: half of a solve's phases hold little,
+// and a launch then costs by the workgroup.  With 8, 4, 3 and 2 (device time,
+// ms): RMAT-20 x 16 0.98, 0.88, 0.92, 1.04; RMAT-21 x 16 1.12, 1.08, 1.08, 1.21;
+// RMAT-22 x 16 1.60, 1.61, 1.59, 1.64; uniform 2^20 x 16 1.61, 1.35, 1.26, 1.23;
+// 2^21 x 8 2.38, 2.00, 1.96, 1.97.
+constexpr int kDeltaWgs = 3;
+
 int run_delta(smdp_graph* g, Relabel* rl, int32_t src, const smdp_params& p, int grid, float* ms_out,
               int* launches_out, bool* reached_counted) {
   *reached_counted = false;
   smdp_ctx* ctx = g->ctx;
+  grid = std::min(grid, kDeltaWgs * ctx->cus);
   if (rl->minw < 0 || (g->m > 0 && !g->w)) return SMDP_ERR_ARG;
   const int delta = p.delta > 0 ? p.delta : 64;
   SMDP_CHECK(ensure_buckets(g, rl, delta));
