@@ -276,11 +276,11 @@ __global__ __launch_bounds__(kRoundThreads) void k_rounds(RoundArgs a, int32_t i
       a.rlog[2 * r + 1] = (unsigned long long)A;
       a.rlog[2 * kRoundLogCap + r] = wall_clock64();
     }
-    if (L == 0) break;
-    if (r >= a.rmax) {
+    if (r >= a.rmax) {  // the last round, which finds no work, counts too
       end = kRoundsCapped;
       break;
     }
+    if (L == 0) break;
     if (b == 0 && tid == 0) {
       agent_store(&a.ctl->queued[((r + 2) & 3) * 16], (uint64_t)0);  // nobody uses it before round r + 1
       edges += A;

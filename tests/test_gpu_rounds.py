@@ -105,12 +105,14 @@ def test_negative_arcs_without_cycles(ctx):
 
 @pytest.mark.parametrize("bfs", [False, True])
 def test_round_cap(ctx, bfs):
-    """A path of 600 vertices takes 599 rounds (its last vertex has no arcs)."""
+    """A path of 600 vertices takes 599 rounds (its last vertex has no arcs) and
+    one that finds no work, which the cap counts as it does where the host
+    drives the rounds."""
     app = smdp.APP_BFS if bfs else smdp.APP_SSSP
     g = _path(600)
     old = ctx.get_params(app)
     try:
-        for cap, ok in ((598, False), (599, True), (600, True)):
+        for cap, ok in ((598, False), (599, False), (600, True), (601, True)):
             ctx.set_params(app, max_rounds=cap)
             run = ctx.bfs if bfs else ctx.sssp
             if ok:
