@@ -72,7 +72,8 @@ def sssp_section(ctx, g, dg, args, smdp, orc, np):
     ctx.set_profiling(True)
     pst = dg.sssp(src, sol)
     ctx.set_profiling(False)
-    bucketed = params.layout == smdp.LAYOUT_BUCKETS or (params.layout == smdp.LAYOUT_AUTO and g.m >= 1 << 20)
+    auto = params.layout == smdp.LAYOUT_AUTO
+    bucketed = params.layout == smdp.LAYOUT_BUCKETS or (auto and g.m >= 1 << 23)
     if bucketed:
         # one phase = k_delta_step (tiles) + k_delta_drain (grid chunks); a
         # relaxed arc moves 12 B (col, w, dist[v]), an arc read but left to the
@@ -90,7 +91,7 @@ def sssp_section(ctx, g, dg, args, smdp, orc, np):
         e1 = pst.edges_relaxed - pst.edges_phase2
         bytes1 = 12 * e1 + 20 * pst.vertices_expanded  # col + w + dist[v]; 2 offsets + dist[u] + queue in/out
         bytes2 = 12 * pst.edges_phase2
-        k1 = {"kernel": "k_expand_tile<false>", "bytes": bytes1, "ms": pst.ms_dominant,
+        k1 = {"kernel": "k_rounds<false>" if auto else "k_expand_tile<false>", "bytes": bytes1, "ms": pst.ms_dominant,
               "launches": pst.dominant_launches}
         k2 = {"kernel": "k_drain<false>", "bytes": bytes2, "ms": pst.ms_phase2, "launches": pst.phase2_launches}
         dom = k1 if k1["ms"] >= k2["ms"] else k2
@@ -241,7 +242,7 @@ def pagerank_section(ctx, g, args, smdp, orc, np):
     gteps = g.m * iters / (ms * 1e6)
     per_iter = 8 * g.m + 20 * g.n
     params = ctx.get_params(smdp.APP_PAGERANK)
-    binned = params.layout == smdp.LAYOUT_BINNED or (params.layout == smdp.LAYOUT_AUTO and g.m >= 1 << 20)
+    binned = params.layout == smdp.LAYOUT_BINNED or (params.layout == smdp.LAYOUT_AUTO and g.m > 1 << 22)
     # every launch after the stop rule fired returns at once: bytes of the
     # iterations run, over the summed duration of all launches.  The binned
     # iteration is two kernels (scatter, reduce); the roofline covers both.
@@ -252,7 +253,7 @@ def pagerank_section(ctx, g, args, smdp, orc, np):
         tr = [traffic_for("k_bin_scatter"), traffic_for("k_bin_reduce")]
         traffic = None if None in tr else tr[0] + tr[1]
     else:
-        kernel = "k_rows_tuned<true>"
+        kernel = "k_pr_merge"
         ms_k = pst.ms_dominant
         launches = pst.dominant_launches
         traffic = traffic_for(kernel)
@@ -311,15 +312,16 @@ def batched_section(ctx, args, smdp, orc, np):
             m_reached += x.m_reached
         t_plain = sum(plain)
     # an arc visit reads col and w (8 B) and the 64 distances of its target
-    # (one 256-B row): 264 B; the CSR bytes are shared by the 64 sources
+    # (one 256-B row): 264 B; the CSR bytes are shared by the 64 sources.  An
+    # arc skipped by its target's bound reads col, w and the bound: 12 B
     per_visit = 8 + 4 * 64
     ms_k = pst.ms_dominant
-    roof = _roof(per_visit * pst.edges_relaxed, ms_k)
+    roof = _roof(per_visit * pst.edges_relaxed + 12 * pst.arcs_skipped, ms_k)
     roof.update(kernel="k_ms_run (hipGraph replay)", launches=pst.dominant_launches,
                 avg_launch_us=round(ms_k * 1e3 / max(1, pst.dominant_launches), 3), traffic=traffic_for("k_ms_run"))
     entry = {"graph": f"rmat-{args.batch_scale} ef16 w[1,255] seed 4", "sources": 64,
              "ms_batched_median_of_10": round(ms_batch, 3), "ms_64_plain": round(t_plain, 3),
-             "speedup": round(t_plain / ms_batch, 2), "rounds": st.rounds, "arc_visits": st.edges_relaxed,
+             "speedup": round(t_plain / ms_batch, 2), "rounds": st.rounds, "arc_visits": st.edges_relaxed, "arcs_skipped": st.arcs_skipped,
              "gteps": round(m_reached / (ms_batch * 1e6), 3), "roofline": roof}
     if not args.skip_cpu:
         # the oracle's Dijkstra (the strongest sequential baseline), 16 of the
@@ -459,7 +461,7 @@ def bfs_section(ctx, smdp, orc, np):
             "rounds": int(st.rounds), "exact_vs_oracle": bool(np.array_equal(lv, ref)),
             "gteps": round(t.m / (ms * 1e6), 3),
             "roofline": dict(_roof(8 * st.edges_relaxed + 12 * t.n, ms),
-                             traffic_per_launch={"k_drain<true>": traffic_for("k_drain<true>")}),
+                             traffic_per_launch={"k_rounds<true>": traffic_for("k_rounds<true>")}),
             "cpu": _cpu_entry(t_cpu, t_par, nt, t.m, "one BFS from the root: FIFO (bfs_rec.cpp:102-121 restated, "
                               "orc_bfs_fifo) / level-synchronous (orc_bfs_par)")}
 

@@ -151,8 +151,9 @@ typedef struct {
   uint64_t edges_phase2;       /* arcs of edges_relaxed scanned by the phase-2 kernel */
   uint64_t atomics_tried;      /* SSSP/BFS: atomicMin issued after a plain read said "improves" */
   uint64_t atomics_won;        /* SSSP/BFS: atomicMin that lowered the distance */
-  uint64_t arcs_skipped;       /* bucketed SSSP: arcs read but left to the bucket's other pass (not relaxed,
-                                  not in edges_relaxed) */
+  uint64_t arcs_skipped;       /* bucketed SSSP: arcs read but left to the bucket's other pass; multi-source
+                                  SSSP: arcs read that a bound shows to lower no distance (not relaxed, not
+                                  in edges_relaxed) */
 } smdp_stats;
 
 /* PageRank options (the reference hard-codes them: DAMPING_FACTOR 0.5 and

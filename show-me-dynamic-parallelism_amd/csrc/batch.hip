@@ -484,7 +484,7 @@ __global__ __launch_bounds__(SMDP_WG) __attribute__((amdgpu_waves_per_eu(5, 5)))
   MsRefKeeper keeper;
   Sink out;
   out.init(s_out + (threadIdx.x / SMDP_WAVE) * kOutCap, nullptr, nullptr);  // the queue is set each round
-  unsigned long long edges = 0, verts = 0, wins = 0;
+  unsigned long long edges = 0, verts = 0, wins = 0, skipped = 0;
   uint32_t epoch = 0;
   int r = 0;
   bool capped = false;
@@ -536,6 +536,7 @@ __global__ __launch_bounds__(SMDP_WG) __attribute__((amdgpu_waves_per_eu(5, 5)))
     const int arcs = ms_relax_pass(a, qin, L, r + 1, s_pre, bound, out, wins, skips);
     if (lane_id() == 0) {
       edges += arcs;
+      skipped += skips;
       s_seen[threadIdx.x / SMDP_WAVE] = arcs;
       s_skip[threadIdx.x / SMDP_WAVE] = skips;
     }
@@ -549,6 +550,7 @@ __global__ __launch_bounds__(SMDP_WG) __attribute__((amdgpu_waves_per_eu(5, 5)))
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) flags[1 + group] = capped ? -1 : r;
   if (lane_id() != 0) wins = 0;
+  else if (skipped) atomicAdd(&cnt_of(a.cnt)->skipped, skipped);
   ms_counters(a, edges, verts, wins, 0, 0);
 }
 
@@ -1191,8 +1193,9 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
   if (st) {
     memset(st, 0, sizeof *st);
     st->ms_kernel = ms;
-    st->edges_relaxed = c.edges;
+    st->edges_relaxed = c.edges - c.skipped;
     st->edges_phase2 = c.edges2;
+    st->arcs_skipped = c.skipped;
     st->vertices_expanded = c.verts;
     st->rounds = rounds;
     st->atomics_won = c.atom_win;
