@@ -95,9 +95,9 @@ typedef struct {
   int32_t delta;            /* SSSP tuned, bucketed layout: bucket width, a power of two (0 = 64) */
   int32_t persistent;       /* SSSP tuned, bucketed layout: 0 = one launch per pass; 1 = every phase of the solve in
                                one launch whose workgroups are all resident, with a grid barrier between passes */
-  int32_t group_share;      /* small-graph batch (read from the SMDP_APP_MSSSP parameters): a graph with more arcs
-                               than group_share percent of one workgroup's fair share of the batch is solved by a
-                               group of workgroups (0 = 100; 10..1000) */
+  int32_t group_share;      /* small-graph batch (read from the SMDP_APP_MSSSP parameters): the share of arcs, in
+                               percent of one workgroup's fair share of the batch, that sizes the cluster or group
+                               of workgroups that solves a large graph (0 = 100; 10..1000) */
   int32_t settle;           /* SSSP tuned, bucketed layout: how a bucket's settle pass reaches the arcs that leave
                                the bucket, one of SMDP_SETTLE_* (0 = automatic) */
 } smdp_params;
