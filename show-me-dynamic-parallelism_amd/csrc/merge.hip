@@ -625,6 +625,9 @@ int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches) {
   return SMDP_OK;
 }
 
+// The last tile of the largest kind still ends within 32-bit positions.
+bool merge_pagerank_fits(int64_t n, int64_t m) { return n + m <= (int64_t)INT32_MAX - kMpNT * 32; }
+
 int merge_pagerank_ensure(smdp_graph* g, void** slot, RArgs* a) {
   MergePlan* mp = nullptr;
   SMDP_CHECK(ensure_merge(g, slot, false, g->ctx->stream, &mp));

@@ -279,6 +279,7 @@ int merge_spmv(smdp_graph* g, void** slot, hipStream_t s, int* launches);
 // PageRank iterations over g's in-CSR by merge-path tiles: the plan in *slot
 // (built on first use; sets the partials of *a that a pass fills), and one
 // iteration on at most `grid` workgroups.
+bool merge_pagerank_fits(int64_t n, int64_t m);
 int merge_pagerank_ensure(smdp_graph* g, void** slot, RArgs* a);
 void merge_pagerank_pass(smdp_graph* g, void* slot, int grid, const RArgs& a, int k, int* launches);
 void merge_free(void* plan);

@@ -775,8 +775,10 @@ int run_pagerank(smdp_graph* g, const smdp_pr_opts* o, int sol, smdp_stats* st) 
     }
   }
   const bool use_bins = binned && ba.vals != nullptr;
-  // tuned solution on the plain in-CSR: merge-path tiles
-  const bool use_merge = sol == SMDP_SOL_TUNED && !use_bins && !a.browp;
+  // tuned solution on the plain in-CSR: merge-path tiles, or a wave per row
+  // where rows and arcs together exceed the tiles' 32-bit positions
+  const bool use_merge = sol == SMDP_SOL_TUNED && !use_bins && !a.browp && merge_pagerank_fits(g->n, g->m);
+  const int rows_sol = sol == SMDP_SOL_TUNED ? SMDP_SOL_WAVE : sol;
   if (use_merge) SMDP_CHECK(merge_pagerank_ensure(g, &b->prmerge, &a));
   prof_reset(ctx);
   const int grid = grid_size(ctx, p);
@@ -804,7 +806,7 @@ int run_pagerank(smdp_graph* g, const smdp_pr_opts* o, int sol, smdp_stats* st) 
       a.y = g->rank[(k + 1) & 1];
       if (use_bins) binned_pass(ctx, s, a, ba, k, &launches);
       else if (use_merge) merge_pagerank_pass(g, b->prmerge, grid, a, k, &launches);
-      else launch_pass<true>(sol, grid, s, a, k, &launches, ctx);
+      else launch_pass<true>(rows_sol, grid, s, a, k, &launches, ctx);
     }
   };
   enqueue(kFeedFirst);
