@@ -462,12 +462,12 @@ void smdp_graph_destroy(smdp_graph* g) {
   if (!g) return;
   (void)hipSetDevice(g->ctx->device);
   if (g->arena) {
-    // these live in the context's arena
+    // these live in the context's arena (rqueue too, unless the arena had no room for it)
+    if (reinterpret_cast<int32_t*>(g->rqueue) == g->q[0]) g->rqueue = nullptr;
     g->row = g->col = g->w = g->dist = g->stamp = g->q[0] = g->q[1] = nullptr;
     g->ctl = nullptr;
     g->cnt = nullptr;
     g->hq = nullptr;
-    g->rqueue = nullptr;
   }
   void* bufs[] = {g->row,    g->col,      g->w,       g->dist,     g->stamp,  g->hasout, g->q[0],  g->q[1],
                   g->hq,     g->ctl,      g->cnt,     g->val,      g->x,      g->y,     g->outdeg,
