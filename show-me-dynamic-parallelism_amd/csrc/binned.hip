@@ -130,12 +130,14 @@ __global__ __launch_bounds__(kScatNT) void k_bin_scatter(RArgs a, BArgs b) {
     // arcs wrote at a 16-byte stride: 152 -> 106 us per RMAT-22 iteration).
     for (int k0 = wave; k0 < nblk; k0 += kQuads * kSW) {
       uint16_t sv[kQuads][4];
+      // no streaming hint: a load's 128 bytes straddle two lines (242.2 us an
+      // iteration with it, 239.6 without)
 #pragma unroll
       for (int u = 0; u < kQuads; ++u) {
         const int k = min(k0 + u * kSW, nblk - 1);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          sv[u][e] = __builtin_nontemporal_load(b.src + base + k * kScatterBlock + e * SMDP_WAVE + lane);
+          sv[u][e] = b.src[base + k * kScatterBlock + e * SMDP_WAVE + lane];
       }
 #pragma unroll
       for (int u = 0; u < kQuads; ++u) {
