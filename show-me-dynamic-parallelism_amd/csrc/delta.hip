@@ -530,7 +530,8 @@ __device__ __forceinline__ void relax_staged(const DArgs& a, DTile& t, const int
       int wk[kDIlp];
 #pragma unroll
       for (int q = 0; q < kDIlp; ++q) {
-        const int2v e = stream_load(a.rcw + k[q]);
+        // rows start anywhere in a line, so no streaming hint here and below (RMAT-22 2302 us a call with it, 2280 without)
+        const int2v e = a.rcw[k[q]];
         v[q] = e.x;  // the arc's source
         wk[q] = e.y;
       }
@@ -550,7 +551,7 @@ __device__ __forceinline__ void relax_staged(const DArgs& a, DTile& t, const int
     } else {
 #pragma unroll
       for (int q = 0; q < kDIlp; ++q) {
-        const int2v e = stream_load(a.cw + k[q]);
+        const int2v e = a.cw[k[q]];
         v[q] = e.x;
         alt[q] = s_du[own[q]] + e.y;
       }
@@ -682,7 +683,7 @@ __device__ __forceinline__ void pull_pass(const DArgs& a, const DPhase& d, DTile
       }
 #pragma unroll
       for (int q = 0; q < kDIlp; ++q) {
-        const int2v e = stream_load(a.rcw + s_base[o[q]] + f[q]);
+        const int2v e = a.rcw[s_base[o[q]] + f[q]];
         src[q] = e.x;
         wk[q] = e.y;
       }
@@ -858,7 +859,7 @@ __device__ __forceinline__ void wave_pass(const DArgs& a, const DPhase& d, int p
       }
 #pragma unroll
       for (int q = 0; q < kDIlp; ++q) {
-        const int2v e = stream_load(a.cw + s_base[o[q]] + f[q]);
+        const int2v e = a.cw[s_base[o[q]] + f[q]];
         vt[q] = e.x;
         alt[q] = s_du[o[q]] + e.y;
       }
