@@ -1086,8 +1086,9 @@ __global__ __launch_bounds__(kLayerThreads) void k_layer_short(LArgs a) {
       uint32_t pv = 0;
       if (ok) {
         const int4 e = s_ent[own];
-        v = stream_load(a.tcol + e.y + j);
-        if (a.prio) pv = stream_load(a.tprio + e.y + j);
+        // short rows share lines, so no streaming hint (RMAT-20 5643 us a call with it, 5573 without)
+        v = a.tcol[e.y + j];
+        if (a.prio) pv = a.tprio[e.y + j];
         const uint32_t pu = (uint32_t)e.z;
         if (pu < pv || (pu == pv && e.x < v)) {
           old = atomicSub(&a.pend[v], 1);
@@ -1167,8 +1168,8 @@ __global__ __launch_bounds__(SMDP_WG) void k_layer_drain(LArgs a) {
 #pragma unroll
       for (int t = 0; t < kLayerIlp; ++t) {
         const int k = b + (int)threadIdx.x + t * SMDP_WG;
-        v[t] = stream_load(a.tcol + min(k, e - 1));
-        pv[t] = a.prio ? stream_load(a.tprio + min(k, e - 1)) : 0u;
+        v[t] = a.tcol[min(k, e - 1)];
+        pv[t] = a.prio ? a.tprio[min(k, e - 1)] : 0u;
         uu[t] = ch.v;
         pu[t] = pu1;
         ok[t] = k < e && v[t] != ch.v;
