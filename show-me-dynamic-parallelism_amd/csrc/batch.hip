@@ -31,6 +31,7 @@
 #include "grid_barrier.h"
 #include "lds_sssp.h"
 #include "smdp_internal.h"
+#include "../host/batch_plan.h"
 
 namespace smdp {
 
@@ -593,27 +594,21 @@ struct GArgs {
   const int64_t* __restrict__ vbase; // per graph: first vertex slot in dist/stamp/queues
   const int32_t* __restrict__ nv;    // per graph: vertices
   const int32_t* __restrict__ src;   // per graph: source
-  const int32_t* __restrict__ order; // graphs without a group, by decreasing arcs (nsmall of them)
-  // Graphs with many more arcs than a workgroup's share are each solved by a
-  // group of workgroups: workgroup b < nplan belongs to group plan[b], whose
-  // graph is ggraph[j], first workgroup gbase[j] and size gsize[j].
-  const int32_t* __restrict__ plan;
-  const int32_t* __restrict__ ggraph;
-  const int32_t* __restrict__ gbase;
-  const int32_t* __restrict__ gsize;
-  int32_t* gctl;                     // per group one 32-word line: queue lengths [0..2], arrivals [3], epoch [4]
-  // LDS clusters, described by clusters[]: workgroup b works on citem[cfirst[b]
-  // .. cfirst[b + 1]) (cluster << 8 | rank, clusters rising) before its group.
-  const int32_t* __restrict__ cfirst;
-  const int32_t* __restrict__ citem;
-  const struct MgCluster* __restrict__ clusters;
+  const int32_t* __restrict__ order; // graphs without a team, by decreasing arcs (nsmall of them)
+  // Teams (host/batch_plan.h): workgroup b < nteamwg belongs to team team[b],
+  // whose workgroups are [tbase[t], tbase[t + 1]) and whose graphs are items
+  // [tfirst[t], tfirst[t + 1]).
+  const int32_t* __restrict__ team;
+  const int32_t* __restrict__ tbase;
+  const int32_t* __restrict__ tfirst;
+  const struct MgItem* __restrict__ items;
+  int32_t* gctl;                     // per item one 32-word line: queue lengths [0..2], arrivals [3], epoch [4]
   const uint8_t* __restrict__ lds;   // per graph: one workgroup can solve it in LDS
   uint64_t* cflags;                  // every cluster's barrier flags
-  int32_t ncwg;                      // workgroups with cluster items
+  int32_t nteamwg;
+  int32_t nitems;
   int32_t ncflags;                   // 64-bit words of cflags
-  int32_t nplan;
   int32_t nsmall;
-  int32_t ngroups;
   int32_t* dist;
   int32_t* stamp;
   int32_t* qa;
@@ -624,8 +619,9 @@ struct GArgs {
   int32_t ng;
 };
 
-// One LDS cluster: its graph and size, and what LdsGraph needs.
-struct MgCluster {
+// A graph that a team solves: in memory, or by a cluster with its distances in
+// LDS (block > 0) and what LdsGraph needs.
+struct MgItem {
   int32_t graph, k, block, pad0;
   uint32_t inv;
   int32_t pad;
@@ -636,21 +632,21 @@ struct MgCluster {
 };
 
 constexpr int kMgOut = 256;
-constexpr int kMgGroupLine = 32;      // ints per group control line
+constexpr int kMgGroupLine = 32;      // ints per item control line
 constexpr int kMgMaxGroup = 16;       // workgroups that solve one graph together, at most
 constexpr int kMgSpinLimit = 1 << 21; // polls before a group barrier gives up (about a second)
 
-__global__ __launch_bounds__(SMDP_WG) void k_mg_reset(int32_t* next, Counters* cnt, int32_t* gctl, int32_t ngroups,
+__global__ __launch_bounds__(SMDP_WG) void k_mg_reset(int32_t* next, Counters* cnt, int32_t* gctl, int32_t nitems,
                                                       uint64_t* cflags, int32_t ncflags) {
   for (int i = threadIdx.x; i < ncflags; i += blockDim.x) cflags[i] = 0;
   if (threadIdx.x == 0) *next = 0;
   unsigned long long* p = reinterpret_cast<unsigned long long*>(cnt);
   for (int i = threadIdx.x; i < (int)(kCntParts * sizeof(Counters) / 8); i += blockDim.x) p[i] = 0;
-  for (int i = threadIdx.x; i < ngroups * kMgGroupLine; i += blockDim.x) gctl[i] = 0;
+  for (int i = threadIdx.x; i < nitems * kMgGroupLine; i += blockDim.x) gctl[i] = 0;
 }
 
-// Barrier of the k workgroups of one group (all resident: they are the
-// first workgroups of the launch).  Arrivals only grow (epoch e is complete
+// Barrier of the k workgroups of one team in a solve in memory (all resident:
+// they are the first workgroups of the launch).  Arrivals only grow (epoch e is complete
 // at e * k); the last publishes the epoch.  Returns false in a workgroup that
 // gave up waiting.  What a group's workgroups exchange between rounds is
 // stored and read device-coherent (queue entries, the initial distances and
@@ -846,13 +842,13 @@ __device__ void mg_solve(const GArgs& a, int g, int rank, int k, int32_t* gq, Mg
 }
 
 // Messages from each workgroup of a cluster to each other one: the arcs from
-// its vertices to theirs (one workgroup per (cluster, sender)), the most a
-// round can send.
+// its vertices to theirs (one workgroup per (item, sender)), the most a round
+// can send.
 __global__ __launch_bounds__(kMgThreads) void k_mg_pairs(GArgs a, int64_t* count) {
   __shared__ int32_t s_cnt[kLdsMaxCluster];
-  const int it = a.citem[blockIdx.x];
-  const MgCluster cl = a.clusters[it >> 8];
-  const int rank = it & 255;
+  const MgItem cl = a.items[blockIdx.x / kLdsMaxCluster];
+  const int rank = blockIdx.x % kLdsMaxCluster;
+  if (cl.block == 0 || rank >= cl.k) return;
   if (threadIdx.x < kLdsMaxCluster) s_cnt[threadIdx.x] = 0;
   __syncthreads();
   const int n = a.nv[cl.graph];
@@ -866,7 +862,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_pairs(GArgs a, int64_t* count
 }
 
 template <bool CL>
-__device__ __forceinline__ void mg_lds(const GArgs& a, int g, const MgCluster* cl, int rank, const int64_t* moff,
+__device__ __forceinline__ void mg_lds(const GArgs& a, int g, const MgItem* cl, int rank, const int64_t* moff,
                                        uint64_t* msg, LdsShared& sh, unsigned long long& edges,
                                        unsigned long long& verts) {
   LdsGraph lg{};
@@ -909,23 +905,22 @@ __global__ __launch_bounds__(NT) void k_mg(GArgs a, const int64_t* moff, uint64_
   __shared__ int s_g;
   MgShared<NT>& sh = *reinterpret_cast<MgShared<NT>*>(raw);
   unsigned long long edges = 0, verts = 0;
-  // The clusters this workgroup belongs to, in the order every workgroup takes
-  // them (the first unfinished one then always has all its workgroups), and
-  // its group.  These workgroups come first: they are dispatched, and
-  // resident, before the others.
-  if (LDS && (int)blockIdx.x < a.ncwg) {
-    for (int i = a.cfirst[blockIdx.x]; i < a.cfirst[blockIdx.x + 1]; ++i) {
-      const int it = a.citem[i];
-      const MgCluster* cl = a.clusters + (it >> 8);
-      mg_lds<true>(a, cl->graph, cl, it & 255, moff, msg, *reinterpret_cast<LdsShared*>(raw), edges, verts);
+  // The graphs of this workgroup's team, in the order every member takes
+  // them.  These workgroups come first: they are dispatched, and resident,
+  // before the others.
+  if ((int)blockIdx.x < a.nteamwg) {
+    const int t = a.team[blockIdx.x];
+    const int rank = (int)blockIdx.x - a.tbase[t];
+    for (int i = a.tfirst[t]; i < a.tfirst[t + 1]; ++i) {
+      const MgItem* it = a.items + i;
+      if (LDS && it->block > 0)
+        mg_lds<true>(a, it->graph, it, rank, moff, msg, *reinterpret_cast<LdsShared*>(raw), edges, verts);
+      else
+        mg_solve<NT, true>(a, it->graph, rank, it->k, a.gctl + i * kMgGroupLine, sh, edges, verts);
+      __syncthreads();  // also after a barrier that gave up
     }
   }
-  if ((int)blockIdx.x < a.nplan) {
-    const int j = a.plan[blockIdx.x];
-    mg_solve<NT, true>(a, a.ggraph[j], (int)blockIdx.x - a.gbase[j], a.gsize[j], a.gctl + j * kMgGroupLine, sh, edges,
-                       verts);
-  }
-  // then graphs without either, one workgroup each, largest first
+  // then graphs without a team, one workgroup each, largest first
   for (;;) {
     if (threadIdx.x == 0) {
       const int t = atomicAdd(a.next, 1);
@@ -1230,15 +1225,11 @@ struct smdp_batch {
   int32_t* d_qb = nullptr;
   int32_t* d_next = nullptr;
   int32_t* d_status = nullptr;
-  int32_t* d_plan = nullptr;
-  int32_t* d_ggraph = nullptr;
-  int32_t* d_gbase = nullptr;
-  int32_t* d_gsize = nullptr;
+  int32_t* d_team = nullptr;
+  int32_t* d_tbase = nullptr;
+  int32_t* d_tfirst = nullptr;
   int32_t* d_gctl = nullptr;
-  int32_t ngroups = 0;
-  int32_t* d_cfirst = nullptr;
-  int32_t* d_citem = nullptr;
-  smdp::MgCluster* d_clusters = nullptr;
+  smdp::MgItem* d_items = nullptr;
   uint8_t* d_lds = nullptr;
   uint64_t* d_cflags = nullptr;
   int64_t* d_moff = nullptr;
@@ -1276,143 +1267,91 @@ static void batch_plan_free(smdp_batch* b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;
-  for (int32_t** q : {&b->d_order, &b->d_plan, &b->d_ggraph, &b->d_gbase, &b->d_gsize, &b->d_gctl, &b->d_cfirst, &b->d_citem}) {
+  for (int32_t** q : {&b->d_order, &b->d_team, &b->d_tbase, &b->d_tfirst, &b->d_gctl}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }
-  if (b->d_clusters) (void)hipFree(b->d_clusters);
+  if (b->d_items) (void)hipFree(b->d_items);
   if (b->d_lds) (void)hipFree(b->d_lds);
   if (b->d_cflags) (void)hipFree(b->d_cflags);
   if (b->d_moff) (void)hipFree(b->d_moff);
   if (b->d_msg) (void)hipFree(b->d_msg);
-  b->d_clusters = nullptr;
+  b->d_items = nullptr;
   b->d_lds = nullptr;
   b->d_cflags = nullptr;
   b->d_moff = nullptr;
   b->d_msg = nullptr;
 }
 
-// Clusters are worth their exchanges from 4 workgroups on (or where the
-// vertices need more than one), up to one per kClusterArcs arcs; a graph that
-// one workgroup holds is left to it below kClusterMin arcs.  Single graphs, k
-// workgroups, us: 32768 x 16 (1: 286, 2: 373, 4: 286, 8: 311), 32768 x 32
-// (390, 564, 349, 327), 65536 x 8 (2: 431, 4: 335, 8: 347, 16: 447), 65536 x 32
-// (2: 1000, 4: 561, 8: 462, 16: 515).
-constexpr int64_t kClusterArcs = int64_t(1) << 18;
-constexpr int64_t kClusterMin = int64_t(1) << 20;
-
-// Work plan of a batch for parameters p, and its hipGraph (reset + solve),
-// replacing the previous plan.  A workgroup's fair share is the batch's arcs
-// over the grid (p.wg_per_cu workgroups per CU, at most 2).
-// A graph that an LDS solve takes goes to one workgroup, or to a cluster of
-// them, ceil(m / share) within the limits above, when it has more than
-// kLdsVerts vertices or at least kClusterMin arcs.  Of the others, a graph of more than p.group_share percent
-// of one share is solved by a group of ceil(m / share) workgroups (at most
-// kMgMaxGroup).  The workgroups of clusters and groups are resident at once
-// and can belong to several clusters in turn; the rest of the graphs are
-// claimed one per workgroup, largest first.
+// Work plan of a batch for parameters p (host/batch_plan.h), and its hipGraph
+// (reset + solve), replacing the previous plan.  A workgroup's fair share is
+// the batch's arcs over the grid (p.wg_per_cu workgroups per CU, at most 2;
+// one where graphs are solved in LDS), of which p.group_share percent sizes
+// the teams.  The workgroups of teams are resident at once; the rest of the
+// graphs are claimed one per workgroup, largest first.
 // 256 graphs, 85M arcs: 6.8 ms with distances in memory and groups, 0.64 ms in
 // LDS with clusters (0.95 ms when a cluster's messages were placed by one LDS
-// atomic per receiver instead of one per lane).  Groups, 69M arcs: 20.9 ms with
-// none, 6.7 ms above two shares, 5.4 ms above one; up to 32 changed nothing.
+// atomic per receiver instead of one per lane).  In memory, 69M arcs: 20.9 ms
+// without teams, 6.7 ms for graphs above two shares, 5.4 ms above one; teams of
+// up to 32 changed nothing.
 static int batch_plan(smdp_batch* b, const smdp_params& p) {
   smdp_ctx* ctx = b->ctx;
   batch_plan_free(b);
   const int32_t ng = b->ng;
-  std::vector<int32_t> order(ng);
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->m[x] > b->m[y]; });
-  const bool lds = std::any_of(order.begin(), order.end(), [&](int32_t i) {
-    return b->fit[i] && b->nv[i] <= kLdsVerts * kLdsMaxCluster;
-  });
+  bool lds = false;
+  for (int32_t i = 0; i < ng; ++i) lds = lds || (b->fit[(size_t)i] && b->nv[i] <= kLdsVerts * kLdsMaxCluster);
   const int wgs = ctx->cus * (lds ? 1 : std::max(1, std::min(2, p.wg_per_cu)));
   int per_cu = 0;
   const void* kernel = lds ? reinterpret_cast<const void*>(k_mg<kMgThreads, true>)
                            : reinterpret_cast<const void*>(k_mg<kMgThreads, false>);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMgThreads, 0) != hipSuccess) per_cu = 0;
-  const int resident = std::min(wgs, per_cu * ctx->cus);
-  const double share = (double)b->etot / wgs * (p.group_share > 0 ? p.group_share : 100) / 100.0;
-  std::vector<int32_t> plan, ggraph, gbase, gsize, small;
-  std::vector<std::vector<int32_t>> items((size_t)std::max(1, resident));  // cluster items of each workgroup
-  std::vector<double> load(items.size(), 0.0);                             // and their arcs
-  std::vector<MgCluster> clusters;
-  std::vector<uint8_t> in_lds((size_t)ng, 0);
+  const BatchLimits lim{kLdsVerts, kLdsMaxCluster, kMgMaxGroup, std::min(wgs, per_cu * ctx->cus),
+                        (double)b->etot / wgs * (p.group_share > 0 ? p.group_share : 100) / 100.0};
+  const BatchPlan plan = plan_batch(b->nv, b->m, b->fit, lim);
+  const int32_t nteams = (int32_t)plan.base.size() - 1, nitems = (int32_t)plan.items.size();
+  const int32_t nteamwg = plan.workgroups();
+  std::vector<int32_t> team((size_t)nteamwg), tfirst((size_t)nteams + 1, 0);
+  for (int32_t t = 0; t < nteams; ++t)
+    std::fill(team.begin() + plan.base[(size_t)t], team.begin() + plan.base[(size_t)t + 1], t);
+  for (const BatchPlan::Item& it : plan.items) ++tfirst[(size_t)it.team + 1];
+  std::partial_sum(tfirst.begin(), tfirst.end(), tfirst.begin());
+  std::vector<MgItem> items((size_t)nitems);
+  std::vector<int32_t> at(tfirst.begin(), tfirst.end());
   int64_t nmoff = 0, nflags = 0;
-  for (int32_t gi : order) {
-    const int64_t n = b->nv[gi], m = b->m[gi];
-    if (b->fit[gi] && n <= (int64_t)kLdsVerts * kLdsMaxCluster) {
-      int64_t k = (n + kLdsVerts - 1) / kLdsVerts;
-      if (k > 1 || m >= kClusterMin)
-        k = std::max(k, std::min<int64_t>({(int64_t)kLdsMaxCluster, (int64_t)std::ceil(m / std::max(1.0, share)),
-                                           std::max<int64_t>(4, m / kClusterArcs)}));
-      const int64_t block = ((n + k - 1) / k + 63) / 64 * 64;
-      k = (n + block - 1) / block;
-      if (k >= 2 && k <= resident) {
-        // the least loaded workgroups take it
-        std::vector<int32_t> by(load.size());
-        std::iota(by.begin(), by.end(), 0);
-        std::partial_sort(by.begin(), by.begin() + k, by.end(),
-                          [&](int x, int y) { return load[x] != load[y] ? load[x] < load[y] : x < y; });
-        for (int j = 0; j < k; ++j) {
-          items[(size_t)by[(size_t)j]].push_back((int32_t)clusters.size() << 8 | j);
-          load[(size_t)by[(size_t)j]] += (double)m / k + kClusterArcs;
-        }
-        MgCluster c{};
-        c.graph = gi;
-        c.k = (int32_t)k;
-        c.block = (int32_t)block;
-        c.inv = (uint32_t)(((uint64_t(1) << 32) + block - 1) / block);
-        c.moff = nmoff;
-        c.flags = nflags;
-        nmoff += k * k;
-        nflags += 2 * k * k;
-        clusters.push_back(c);
-        continue;
-      }
-      if (n <= kLdsVerts) {
-        in_lds[gi] = 1;
-        small.push_back(gi);
-        continue;
-      }
+  for (const BatchPlan::Item& it : plan.items) {
+    MgItem c{};
+    c.graph = it.graph;
+    c.k = plan.team_size(it.team);
+    if (it.cluster) {
+      const int64_t block = cluster_block(b->nv[it.graph], c.k);
+      c.block = (int32_t)block;
+      c.inv = (uint32_t)(((uint64_t(1) << 32) + block - 1) / block);
+      c.moff = nmoff;
+      c.flags = nflags;
+      nmoff += (int64_t)c.k * c.k;
+      nflags += 2 * (int64_t)c.k * c.k;
     }
-    const int k = (int)std::min<int64_t>(kMgMaxGroup, (int64_t)std::ceil(m / std::max(1.0, share)));
-    if (k >= 2 && (int)plan.size() + k <= resident) {
-      ggraph.push_back(gi);
-      gbase.push_back((int32_t)plan.size());
-      gsize.push_back(k);
-      for (int j = 0; j < k; ++j) plan.push_back((int32_t)ggraph.size() - 1);
-    } else {
-      small.push_back(gi);
-    }
+    items[(size_t)at[(size_t)it.team]++] = c;
   }
-  std::vector<int32_t> cfirst(1, 0), citem;
-  int ncwg = 0;
-  for (size_t i = 0; i < items.size(); ++i) {
-    if (!items[i].empty()) ncwg = (int)i + 1;
-    citem.insert(citem.end(), items[i].begin(), items[i].end());
-    cfirst.push_back((int32_t)citem.size());
-  }
-  const int grid = std::max<int>(1, std::min<int>(wgs, std::max<int>(ncwg, (int)plan.size()) + (int)small.size()));
+  const int grid = std::max<int>(1, std::min<int>(wgs, nteamwg + (int)plan.single.size()));
   int rc = SMDP_OK;
   auto up32 = [&](int32_t** d, const int32_t* h, int64_t cnt) {
     if (rc != SMDP_OK) return;
-    if (hipMalloc((void**)d, sizeof(int32_t) * std::max<int64_t>(1, cnt)) != hipSuccess) rc = SMDP_ERR_NOMEM;
-    else if (h && cnt && hipMemcpy(*d, h, sizeof(int32_t) * cnt, hipMemcpyHostToDevice) != hipSuccess)
+    rc = alloc_once(d, std::max<int64_t>(1, cnt));
+    if (rc == SMDP_OK && h && cnt > 0 &&
+        hipMemcpy(*d, h, sizeof(int32_t) * (size_t)cnt, hipMemcpyHostToDevice) != hipSuccess)
       rc = SMDP_ERR_DEVICE;
   };
-  b->ngroups = (int32_t)ggraph.size();
-  up32(&b->d_order, small.data(), (int64_t)small.size());
-  up32(&b->d_plan, plan.data(), (int64_t)plan.size());
-  up32(&b->d_ggraph, ggraph.data(), (int64_t)ggraph.size());
-  up32(&b->d_gbase, gbase.data(), (int64_t)gbase.size());
-  up32(&b->d_gsize, gsize.data(), (int64_t)gsize.size());
-  up32(&b->d_gctl, nullptr, (int64_t)ggraph.size() * kMgGroupLine);
-  up32(&b->d_cfirst, cfirst.data(), (int64_t)cfirst.size());
-  up32(&b->d_citem, citem.data(), (int64_t)citem.size());
+  up32(&b->d_order, plan.single.data(), (int64_t)plan.single.size());
+  up32(&b->d_team, team.data(), nteamwg);
+  up32(&b->d_tbase, plan.base.data(), nteams + 1);
+  up32(&b->d_tfirst, tfirst.data(), nteams + 1);
+  up32(&b->d_gctl, nullptr, (int64_t)nitems * kMgGroupLine);
   if (rc != SMDP_OK) return rc;
   SMDP_CHECK(alloc_once(&b->d_lds, ng));
-  SMDP_HIP(hipMemcpy(b->d_lds, in_lds.data(), (size_t)ng, hipMemcpyHostToDevice));
-  SMDP_CHECK(alloc_once(&b->d_clusters, std::max<int64_t>(1, (int64_t)clusters.size())));
+  SMDP_HIP(hipMemcpy(b->d_lds, plan.lds.data(), (size_t)ng, hipMemcpyHostToDevice));
+  SMDP_CHECK(alloc_once(&b->d_items, std::max<int32_t>(1, nitems)));
+  if (nitems) SMDP_HIP(hipMemcpy(b->d_items, items.data(), sizeof(MgItem) * items.size(), hipMemcpyHostToDevice));
   SMDP_CHECK(alloc_once(&b->d_cflags, std::max<int64_t>(1, nflags)));
   SMDP_CHECK(alloc_once(&b->d_moff, std::max<int64_t>(1, nmoff)));
   GArgs& a = b->args;
@@ -1424,21 +1363,17 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
   a.nv = b->d_nv;
   a.src = b->d_src;
   a.order = b->d_order;
-  a.plan = b->d_plan;
-  a.ggraph = b->d_ggraph;
-  a.gbase = b->d_gbase;
-  a.gsize = b->d_gsize;
+  a.team = b->d_team;
+  a.tbase = b->d_tbase;
+  a.tfirst = b->d_tfirst;
+  a.items = b->d_items;
   a.gctl = b->d_gctl;
-  a.cfirst = b->d_cfirst;
-  a.citem = b->d_citem;
-  a.clusters = b->d_clusters;
   a.lds = b->d_lds;
   a.cflags = b->d_cflags;
-  a.ncwg = ncwg;
+  a.nteamwg = nteamwg;
+  a.nitems = nitems;
   a.ncflags = (int32_t)nflags;
-  a.nplan = (int32_t)plan.size();
-  a.nsmall = (int32_t)small.size();
-  a.ngroups = b->ngroups;
+  a.nsmall = (int32_t)plan.single.size();
   a.dist = b->d_dist;
   a.stamp = b->d_stamp;
   a.qa = b->d_qa;
@@ -1449,34 +1384,34 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
   a.ng = ng;
   b->grid = grid;
   hipStream_t s = ctx->stream;
-  if (!clusters.empty()) {
+  if (nmoff) {
     // message buffers: the arcs between each pair of a cluster's workgroups
-    SMDP_HIP(hipMemcpyAsync(b->d_clusters, clusters.data(), sizeof(MgCluster) * clusters.size(), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_mg_pairs, dim3((unsigned)citem.size()), dim3(kMgThreads), 0, s, b->args, b->d_moff);
+    hipLaunchKernelGGL(k_mg_pairs, dim3((unsigned)(nitems * kLdsMaxCluster)), dim3(kMgThreads), 0, s, b->args, b->d_moff);
     SMDP_HIP(hipGetLastError());
     std::vector<int64_t> moff((size_t)nmoff);
     SMDP_HIP(hipMemcpyAsync(moff.data(), b->d_moff, sizeof(int64_t) * moff.size(), hipMemcpyDeviceToHost, s));
     SMDP_HIP(hipStreamSynchronize(s));
     int64_t total = 0;
-    for (MgCluster& c : clusters) {
-      int64_t at = 0;
+    for (MgItem& c : items) {
+      if (!c.block) continue;
+      int64_t sum = 0;
       for (int64_t i = c.moff; i < c.moff + (int64_t)c.k * c.k; ++i) {
         const int64_t cnt = moff[(size_t)i];
-        moff[(size_t)i] = at;
-        at += cnt;
+        moff[(size_t)i] = sum;
+        sum += cnt;
       }
-      c.mtotal = at;
+      c.mtotal = sum;
       c.msg = total;
-      total += 2 * at;
+      total += 2 * sum;
     }
     SMDP_CHECK(alloc_once(&b->d_msg, std::max<int64_t>(1, total)));
     SMDP_HIP(hipMemcpy(b->d_moff, moff.data(), sizeof(int64_t) * moff.size(), hipMemcpyHostToDevice));
-    SMDP_HIP(hipMemcpy(b->d_clusters, clusters.data(), sizeof(MgCluster) * clusters.size(), hipMemcpyHostToDevice));
+    SMDP_HIP(hipMemcpy(b->d_items, items.data(), sizeof(MgItem) * items.size(), hipMemcpyHostToDevice));
   }
   // Capture reset + solve once; every run replays the graph.  No memset nodes:
   // counters are cleared by a kernel.
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return SMDP_ERR_DEVICE;
-  hipLaunchKernelGGL(k_mg_reset, dim3(1), dim3(256), 0, s, b->d_next, b->d_cnt, b->d_gctl, b->ngroups, b->d_cflags,
+  hipLaunchKernelGGL(k_mg_reset, dim3(1), dim3(256), 0, s, b->d_next, b->d_cnt, b->d_gctl, nitems, b->d_cflags,
                      (int32_t)nflags);
   hipLaunchKernelGGL(k_mg_status_clear, dim3(std::max(1, (ng + 255) / 256)), dim3(256), 0, s, b->d_status, ng);
   if (lds)
