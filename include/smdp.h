@@ -31,6 +31,13 @@
  *     at 1 (apps/graph-color/src/graph_color_wrapper.cu:118).
  *   - One context per host thread.  Calls on one context are serialised on
  *     the context's HIP stream.
+ *   - Contexts of one process on one GPU may run at the same time.  Launches
+ *     whose workgroups wait for one another (SSSP and BFS rounds in one launch,
+ *     multi-source SSSP, small-graph batches, colouring) take turns at the GPU's
+ *     CUs.  Another process that keeps the CUs for longer than about a second
+ *     makes such a launch give up: SSSP, BFS and multi-source SSSP then go on
+ *     with rounds that the host drives, a batch or a colouring returns
+ *     SMDP_ERR_DEVICE.
  */
 #ifndef SMDP_H
 #define SMDP_H

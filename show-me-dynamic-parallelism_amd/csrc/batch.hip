@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstring>
 #include <numeric>
+#include <optional>
 #include <vector>
 
 #include "device_common.h"
@@ -32,6 +33,7 @@
 #include "lds_sssp.h"
 #include "smdp_internal.h"
 #include "../host/batch_plan.h"
+#include "../host/resident_gate.h"
 
 namespace smdp {
 
@@ -1153,6 +1155,8 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
   prof_reset(ctx);
   uint64_t rounds = 0, launches = 0;
   bool host_rounds = !pl->exec;
+  std::optional<ResidentShare> cus;
+  if (!host_rounds) cus.emplace(ctx->device, pgrid, ctx->cus);
   SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
   if (!host_rounds) {
     SMDP_CHECK(prof_mark(ctx, 0));
@@ -1161,6 +1165,7 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
     launches += 5 * (uint64_t)groups;
     SMDP_HIP(hipMemcpyAsync(ctx->pinned, pl->flags, sizeof(int32_t) * (1 + groups), hipMemcpyDeviceToHost, s));
     SMDP_HIP(hipStreamSynchronize(s));
+    cus.reset();
     if (ctx->pinned[0]) {
       // a grid barrier gave up (the workgroups were not all resident): run
       // the same groups with host-driven rounds
@@ -1549,10 +1554,15 @@ int smdp_batch_run(smdp_batch* b, smdp_stats* st) {
   double t0 = now_ms();
   batch_drop_ahead(b);
   hipStream_t s = ctx->stream;
-  SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
-  SMDP_HIP(hipGraphLaunch(b->exec, s));
-  SMDP_HIP(hipEventRecord(ctx->ev_end, s));
-  SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  {
+    // workgroups of teams wait for one another
+    std::optional<ResidentShare> cus;
+    if (b->args.nteamwg) cus.emplace(ctx->device, b->grid, ctx->cus);
+    SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
+    SMDP_HIP(hipGraphLaunch(b->exec, s));
+    SMDP_HIP(hipEventRecord(ctx->ev_end, s));
+    SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  }
   float ms = 0;
   SMDP_HIP(hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end));
   std::vector<int32_t> status(b->ng);

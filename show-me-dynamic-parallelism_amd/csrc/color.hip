@@ -32,6 +32,7 @@
 #include "device_common.h"
 #include "grid_barrier.h"
 #include "smdp_internal.h"
+#include "../host/resident_gate.h"
 
 namespace smdp {
 
@@ -1371,6 +1372,7 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
   hipStream_t s = ctx->stream;
   prof_reset(ctx);
   int launches = 0;
+  ResidentShare cus(ctx->device, short_grid, ctx->cus);
   SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
   hipLaunchKernelGGL(k_layer_init, dim3(1), dim3(256), 0, s, g->ctl, g->cnt, a.rd);
   hipLaunchKernelGGL(k_layer_count, dim3(grid), dim3(SMDP_WG), 0, s, a);
@@ -1413,6 +1415,7 @@ static int run_color_layers(smdp_graph* g, int use_prio, smdp_stats* st) {
   }
   SMDP_HIP(hipEventRecord(ctx->ev_end, s));
   SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  cus.release();
   float ms = 0;
   SMDP_HIP(hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end));
   g->last_res = SMDP_RES_COLOR;

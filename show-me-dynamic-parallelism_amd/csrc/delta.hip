@@ -81,6 +81,7 @@
 #include "frontier.h"
 #include "grid_barrier.h"
 #include "smdp_internal.h"
+#include "../host/resident_gate.h"
 
 namespace smdp {
 
@@ -1370,6 +1371,7 @@ int run_delta(smdp_graph* g, Relabel* rl, int32_t src, const smdp_params& p, int
     int32_t* hf = ctx->pinned;
     bool gave_up = false;
     a.small_q = pgrid * SMDP_WG;
+    ResidentShare cus(ctx->device, pgrid, ctx->cus);
     for (;;) {
       SMDP_CHECK(prof_mark(ctx, 0));
       hipLaunchKernelGGL(k_delta_run, dim3(pgrid), dim3(SMDP_WG), 0, s, a, ph, ph + kRunPhases, bar, flags);

@@ -31,6 +31,7 @@
 #include "lds_sssp.h"
 #include "rounds.h"
 #include "smdp_internal.h"
+#include "../host/resident_gate.h"
 
 namespace smdp {
 
@@ -970,8 +971,14 @@ static int collect_rounds_log(smdp_ctx* ctx, int rounds) {
   return SMDP_OK;
 }
 
+// How long a solve waits for the CUs that other contexts' launches hold before
+// it goes to the host-driven rounds, which need none of their own: a few solves
+// of the kind (0.03 to 1 ms), and no longer than what it would then lose.
+constexpr double kRoundsWaitMs = 2.0;
+
 // Returns kRoundsRetry (and leaves the solve to the host-driven rounds) when
-// the workgroups were not all resident or there is no memory for the queues.
+// the workgroups were not all resident, other contexts hold the CUs, or there
+// is no memory for the queues.
 static int run_rounds(smdp_graph* g, int32_t src, bool bfs, const smdp_params& p, smdp_stats* st) {
   smdp_ctx* ctx = g->ctx;
   hipStream_t s = ctx->stream;
@@ -1000,6 +1007,8 @@ static int run_rounds(smdp_graph* g, int32_t src, bool bfs, const smdp_params& p
   // Workgroups: RMAT-16 x 17 took 334 us on 128, 320 on 192, 326 on 256; uniform
   // 33000 x 4 220 on 96 to 128, 235 on 192, 266 on 256.
   const int grid = std::max(1, std::min({kRoundWgs, ctx->cus * 3 / 4, std::max(32, g->m / 1024)}));
+  ResidentShare cus(ctx->device, grid, ctx->cus, kRoundsWaitMs);
+  if (!cus.held()) return kRoundsRetry;
   SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
   hipLaunchKernelGGL(k_rounds_init, dim3((unsigned)std::min<int64_t>(((int64_t)g->n + 255) / 256, 1024)), dim3(256), 0, s,
                      a, inf, src);
@@ -1011,6 +1020,7 @@ static int run_rounds(smdp_graph* g, int32_t src, bool bfs, const smdp_params& p
   SMDP_HIP(hipMemcpyAsync(ctx->pinned, g->cnt, kCntParts * sizeof(Counters), hipMemcpyDeviceToHost, s));
   SMDP_HIP(hipEventRecord(ctx->ev_end, s));
   SMDP_HIP(hipEventSynchronize(ctx->ev_end));
+  cus.release();
   const Counters* c = reinterpret_cast<const Counters*>(ctx->pinned);
   unsigned long long end = 0, rounds = 0;
   for (int i = 0; i < kCntParts; ++i) {
