@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 #include <optional>
 #include <vector>
@@ -1241,7 +1242,9 @@ struct smdp_batch {
   uint64_t* d_msg = nullptr;
   std::vector<uint8_t> fit;  // per graph: its weights suit an LDS solve
   // Results read ahead: graphs [ahead_lo, ahead_hi) of the last run in pinned
-  // memory (kAheadInts entries, allocated at the first use).
+  // memory (kAheadInts entries, allocated at the first use).  Several threads
+  // may read at once: ahead_mutex covers these fields.
+  std::mutex ahead_mutex;
   int32_t* ahead = nullptr;
   int32_t ahead_lo = 0, ahead_hi = 0;
   int32_t last_read = -2;      // the graph read last since the last run
@@ -1261,6 +1264,7 @@ constexpr int64_t kAheadFirst = int64_t(1) << 15;      // first piece: 128 KB
 
 // Every change of the results drops what was read ahead.
 static void batch_drop_ahead(smdp_batch* b) {
+  std::lock_guard<std::mutex> lock(b->ahead_mutex);
   b->ahead_lo = b->ahead_hi = 0;
   b->last_read = -2;
   b->ahead_ints = kAheadFirst;
@@ -1627,26 +1631,32 @@ int smdp_batch_read(smdp_batch* b, int32_t i, int32_t* dist) {
   // graph read in order on, results come over in pieces of several graphs that
   // double up to kAheadInts entries, and the next reads are copies on the
   // host: 256 graphs of 17 MB in 3.2 ms one by one.
-  const bool in_order = i == b->last_read + 1;
-  b->last_read = i;
-  if (i >= b->ahead_lo && i < b->ahead_hi) {
-    memcpy(dist, b->ahead + (b->vbase[i] - b->vbase[b->ahead_lo]), sizeof(int32_t) * (size_t)b->nv[i]);
-    return SMDP_OK;
-  }
-  if (in_order && i > 0 && b->nv[i] <= b->ahead_ints) {
-    if (!b->ahead && hipHostMalloc((void**)&b->ahead, sizeof(int32_t) * kAheadInts, hipHostMallocDefault) != hipSuccess)
-      b->ahead = nullptr;
-    if (b->ahead) {
-      int32_t hi = i + 1;
-      int64_t cnt = b->nv[i];
-      while (hi < b->ng && cnt + b->nv[hi] <= b->ahead_ints) cnt += b->nv[hi++];
-      b->ahead_lo = b->ahead_hi = 0;
-      SMDP_HIP(hipMemcpy(b->ahead, b->d_dist + b->vbase[i], sizeof(int32_t) * (size_t)cnt, hipMemcpyDeviceToHost));
-      b->ahead_lo = i;
-      b->ahead_hi = hi;
-      b->ahead_ints = std::min(b->ahead_ints * 2, kAheadInts);
-      memcpy(dist, b->ahead, sizeof(int32_t) * (size_t)b->nv[i]);
+  {
+    std::lock_guard<std::mutex> lock(b->ahead_mutex);
+    const bool in_order = i == b->last_read + 1;
+    b->last_read = i;
+    if (i >= b->ahead_lo && i < b->ahead_hi) {
+      memcpy(dist, b->ahead + (b->vbase[i] - b->vbase[b->ahead_lo]), sizeof(int32_t) * (size_t)b->nv[i]);
       return SMDP_OK;
+    }
+    if (in_order && i > 0 && b->nv[i] <= b->ahead_ints) {
+      if (!b->ahead &&
+          hipHostMalloc((void**)&b->ahead, sizeof(int32_t) * kAheadInts, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();  // read one by one
+        b->ahead = nullptr;
+      }
+      if (b->ahead) {
+        int32_t hi = i + 1;
+        int64_t cnt = b->nv[i];
+        while (hi < b->ng && cnt + b->nv[hi] <= b->ahead_ints) cnt += b->nv[hi++];
+        b->ahead_lo = b->ahead_hi = 0;
+        SMDP_HIP(hipMemcpy(b->ahead, b->d_dist + b->vbase[i], sizeof(int32_t) * (size_t)cnt, hipMemcpyDeviceToHost));
+        b->ahead_lo = i;
+        b->ahead_hi = hi;
+        b->ahead_ints = std::min(b->ahead_ints * 2, kAheadInts);
+        memcpy(dist, b->ahead, sizeof(int32_t) * (size_t)b->nv[i]);
+        return SMDP_OK;
+      }
     }
   }
   SMDP_HIP(hipMemcpy(dist, b->d_dist + b->vbase[i], sizeof(int32_t) * b->nv[i], hipMemcpyDeviceToHost));
