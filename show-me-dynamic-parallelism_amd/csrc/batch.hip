@@ -1303,18 +1303,21 @@ static void batch_plan_free(smdp_batch* b) {
 // atomic per receiver instead of one per lane).  In memory, 69M arcs: 20.9 ms
 // without teams, 6.7 ms for graphs above two shares, 5.4 ms above one; teams of
 // up to 32 changed nothing.
-static int batch_plan(smdp_batch* b, const smdp_params& p) {
+// Without memory for the clusters' messages, graphs that one workgroup does not
+// hold are solved in memory, which needs none.
+static int batch_plan(smdp_batch* b, const smdp_params& p, bool clusters = true) {
   smdp_ctx* ctx = b->ctx;
   batch_plan_free(b);
   const int32_t ng = b->ng;
+  const int max_cluster = clusters ? kLdsMaxCluster : 1;
   bool lds = false;
-  for (int32_t i = 0; i < ng; ++i) lds = lds || (b->fit[(size_t)i] && b->nv[i] <= kLdsVerts * kLdsMaxCluster);
+  for (int32_t i = 0; i < ng; ++i) lds = lds || (b->fit[(size_t)i] && b->nv[i] <= kLdsVerts * max_cluster);
   const int wgs = ctx->cus * (lds ? 1 : std::max(1, std::min(2, p.wg_per_cu)));
   int per_cu = 0;
   const void* kernel = lds ? reinterpret_cast<const void*>(k_mg<kMgThreads, true>)
                            : reinterpret_cast<const void*>(k_mg<kMgThreads, false>);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMgThreads, 0) != hipSuccess) per_cu = 0;
-  const BatchLimits lim{kLdsVerts, kLdsMaxCluster, kMgMaxGroup, std::min(wgs, per_cu * ctx->cus),
+  const BatchLimits lim{kLdsVerts, max_cluster, kMgMaxGroup, std::min(wgs, per_cu * ctx->cus),
                         (double)b->etot / wgs * (p.group_share > 0 ? p.group_share : 100) / 100.0};
   const BatchPlan plan = plan_batch(b->nv, b->m, b->fit, lim);
   const int32_t nteams = (int32_t)plan.base.size() - 1, nitems = (int32_t)plan.items.size();
@@ -1400,20 +1403,31 @@ static int batch_plan(smdp_batch* b, const smdp_params& p) {
     std::vector<int64_t> moff((size_t)nmoff);
     SMDP_HIP(hipMemcpyAsync(moff.data(), b->d_moff, sizeof(int64_t) * moff.size(), hipMemcpyDeviceToHost, s));
     SMDP_HIP(hipStreamSynchronize(s));
+    // A team's clusters use one buffer in turn: a workgroup begins the next when
+    // every member has left the last exchange of the one before, which has no
+    // messages.
     int64_t total = 0;
-    for (MgItem& c : items) {
-      if (!c.block) continue;
-      int64_t sum = 0;
-      for (int64_t i = c.moff; i < c.moff + (int64_t)c.k * c.k; ++i) {
-        const int64_t cnt = moff[(size_t)i];
-        moff[(size_t)i] = sum;
-        sum += cnt;
+    for (int32_t t = 0; t < nteams; ++t) {
+      int64_t most = 0;
+      for (int32_t it = tfirst[(size_t)t]; it < tfirst[(size_t)t + 1]; ++it) {
+        MgItem& c = items[(size_t)it];
+        if (!c.block) continue;
+        int64_t sum = 0;
+        for (int64_t i = c.moff; i < c.moff + (int64_t)c.k * c.k; ++i) {
+          const int64_t cnt = moff[(size_t)i];
+          moff[(size_t)i] = sum;
+          sum += cnt;
+        }
+        c.mtotal = sum;
+        c.msg = total;
+        most = std::max(most, sum);
       }
-      c.mtotal = sum;
-      c.msg = total;
-      total += 2 * sum;
+      total += 2 * most;
     }
-    SMDP_CHECK(alloc_once(&b->d_msg, std::max<int64_t>(1, total)));
+    if (alloc_once(&b->d_msg, std::max<int64_t>(1, total)) != SMDP_OK) {
+      (void)hipGetLastError();
+      return batch_plan(b, p, false);
+    }
     SMDP_HIP(hipMemcpy(b->d_moff, moff.data(), sizeof(int64_t) * moff.size(), hipMemcpyHostToDevice));
     SMDP_HIP(hipMemcpy(b->d_items, items.data(), sizeof(MgItem) * items.size(), hipMemcpyHostToDevice));
   }

@@ -1,0 +1,67 @@
+"""Calls that take extra device memory for speed, with the device nearly full:
+they go on without it and stay exact.  torch fills the device."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import orc
+import smdp
+from conftest import random_graph
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+@contextlib.contextmanager
+def device_left(mb):
+    """About mb MB of device memory are free inside (within 32 MB below)."""
+    def free():
+        return torch.cuda.mem_get_info(0)[0]
+
+    fill = []
+    try:
+        torch.cuda.empty_cache()
+        while free() > (mb + 1100) * MB:
+            fill.append(torch.empty(free() - (mb + 1024) * MB, dtype=torch.uint8, device="cuda:0"))
+        while free() > mb * MB:
+            fill.append(torch.empty(32 * MB, dtype=torch.uint8, device="cuda:0"))
+        print(f"device memory left: {free() // MB} MB", flush=True)
+        yield
+    finally:
+        fill.clear()
+        torch.cuda.empty_cache()
+
+
+def test_batch_without_memory_for_messages(ctx):
+    """15M arcs between the 16 workgroups of a cluster: 215 MB of messages
+    beside 126 MB for the batch itself."""
+    row, col, w = random_graph(500000, 15000000, 3, 1, 50)
+    g = smdp.HostGraph(row, col, w, 0)
+    ref = orc.dijkstra(row, col, w, 0)
+    with device_left(260):
+        with smdp.Batch(ctx, [g], np.zeros(1, np.int32)) as b:
+            for _ in range(2):
+                b.run()
+                assert np.array_equal(b.read(0), ref)
+    with smdp.Batch(ctx, [g], np.zeros(1, np.int32)) as b:
+        b.run()
+        assert np.array_equal(b.read(0), ref)
+
+
+def test_dropin_without_memory_for_round_queues(ctx):
+    """The queues of the rounds in one launch (32 bytes per vertex) beside a
+    graph of 8 million vertices."""
+    n = 8_000_000
+    row = np.minimum(np.arange(n + 1, dtype=np.int64) * 2, n - 1).astype(np.int32)
+    col = np.arange(1, n, dtype=np.int32)  # a binary heap: vertex v has 2v + 1 and 2v + 2
+    g = smdp.HostGraph(row, col, np.ones(n - 1, np.int32), 0)
+    want = np.floor(np.log2(np.arange(1, n + 1))).astype(np.int32)
+    with smdp.Context(0) as c, device_left(420):
+        for _ in range(2):
+            lv, _ = c.bfs(g, 0, smdp.SOL_TUNED)
+            assert np.array_equal(lv, want)
+    lv, st = ctx.bfs(g, 0, smdp.SOL_TUNED)
+    assert np.array_equal(lv, want) and st.kernel_launches == 2
