@@ -62,7 +62,8 @@ struct MArgs {
   const int32_t* __restrict__ w;
   int32_t* mdist;  // [n][64]
   int32_t* stamp;
-  int32_t* bound;  // [kMsGens][n] upper bound of a vertex's distances over the reference ones, INT32_MAX: none
+  int32_t* bound;  // [kMsGens][n] upper bound of a vertex's distances over the reference ones, INT32_MAX: none;
+                   // nullptr: no memory for them, and no arc is skipped
   MsRef* ref;
   int32_t* qoff;   // [n] arcs of the queue entries before this one in its workgroup's part
   int32_t* qm;     // [n] ms_bound of the queue entries
@@ -156,7 +157,8 @@ __global__ __launch_bounds__(SMDP_WG) void k_ms_init(MArgs a, int32_t n) {
   unsigned long long hub = 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     a.stamp[i] = -1;
-    for (int g = 0; g < kMsGens; ++g) a.bound[(int64_t)g * n + i] = INT32_MAX;
+    if (a.bound)
+      for (int g = 0; g < kMsGens; ++g) a.bound[(int64_t)g * n + i] = INT32_MAX;
     const unsigned long long deg = (unsigned long long)(uint32_t)(a.row[i + 1] - a.row[i]);
     hub = max(hub, deg << 32 | (uint32_t)~(uint32_t)i);
   }
@@ -486,6 +488,7 @@ __global__ __launch_bounds__(SMDP_WG) __attribute__((amdgpu_waves_per_eu(5, 5)))
   __shared__ int s_ok;
   const int G = gridDim.x;
   MsRefKeeper keeper;
+  keeper.done = a.bound == nullptr;
   Sink out;
   out.init(s_out + (threadIdx.x / SMDP_WAVE) * kOutCap, nullptr, nullptr);  // the queue is set each round
   unsigned long long edges = 0, verts = 0, wins = 0, skipped = 0;
@@ -966,9 +969,7 @@ struct MsPlan {
   uint32_t* bar = nullptr;    // kBarLines * 32 barrier words
   int32_t* bound = nullptr;   // [kMsGens][n] MArgs::bound
   smdp::MsRef* ref = nullptr;
-  int32_t* qoff = nullptr;    // [n], [n], [kMsGrid]: of k_ms_run's passes
-  int32_t* qm = nullptr;
-  int32_t* tot = nullptr;
+  int32_t* tot = nullptr;     // [kMsGrid] of k_ms_run's passes
   int32_t* flags = nullptr;   // [0] a barrier gave up; [1 + j] rounds of group j (-1: round cap)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -988,7 +989,7 @@ void msplan_free(smdp_graph* g) {
   MsPlan* pl = static_cast<MsPlan*>(g->msplan);
   if (!pl) return;
   pl->drop_graph();
-  void* ptrs[] = {pl->d_srcs, pl->mres, pl->bar, pl->bound, pl->ref, pl->qoff, pl->qm, pl->tot, pl->flags};
+  void* ptrs[] = {pl->d_srcs, pl->mres, pl->bar, pl->bound, pl->ref, pl->tot, pl->flags};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   delete pl;
@@ -1012,8 +1013,9 @@ static MArgs ms_args(smdp_graph* g, const MsPlan* pl, const smdp_params& p) {
   a.stamp = g->stamp;
   a.bound = pl->bound;
   a.ref = pl->ref;
-  a.qoff = pl->qoff;
-  a.qm = pl->qm;
+  // the grid queue (n entries of 8 bytes and more) serves the host-driven rounds only
+  a.qoff = reinterpret_cast<int32_t*>(g->hq);
+  a.qm = a.qoff + g->n;
   a.tot = pl->tot;
   a.q0 = g->q[0];
   a.q1 = g->q[1];
@@ -1118,12 +1120,10 @@ int run_multi_source(smdp_graph* g, const int32_t* srcs, int32_t k, int32_t* hos
       SMDP_CHECK(alloc_once(&pl->flags, 1 + groups));
     }
     SMDP_CHECK(alloc_once(&pl->bar, (int64_t)kBarLines * 32));
-    SMDP_CHECK(alloc_once(&pl->bound, (int64_t)kMsGens * n));
     SMDP_CHECK(alloc_once(&pl->ref, 1));
-    SMDP_CHECK(alloc_once(&pl->qoff, n));
-    SMDP_CHECK(alloc_once(&pl->qm, n));
     SMDP_CHECK(alloc_once(&pl->tot, kMsGrid));
     SMDP_CHECK(ensure(&pl->mres, &pl->mres_cap, (int64_t)k * n));
+    if (alloc_once(&pl->bound, (int64_t)kMsGens * n) != SMDP_OK) (void)hipGetLastError();  // without bounds
     pl->k = k;
     pl->groups = groups;
     pl->grid = pgrid;
