@@ -33,7 +33,13 @@
 // and lays their arcs end to end: a bit per arc marks where a vertex's arcs
 // begin, so an arc finds its vertex by counting the marks before it (a binary
 // search over offsets was 10 LDS reads per arc).  Vertices of kLdsHeavy arcs
-// or more become chunks that all waves share after a barrier.
+// or more become chunks that all waves share after a barrier; those that find
+// no room in a round's list stay active for the next round, which takes only
+// the smallest distance, so that it settles a vertex.  (Expanded by the wave
+// that found them, they left 15 waves idle: complete graph of 600 vertices 204
+// us, now 118; star of 500000 leaves on a cluster of 16 2634, now 448; hub of 4
+// million arcs 20.9 ms, now 2.8.)  Graphs of few scan blocks share vertices
+// from kLdsHeavyFew arcs on: 255 vertices of 255 arcs 160 us, now 51.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -49,8 +55,12 @@ constexpr int kLdsVerts = 32768;  // vertices of one workgroup: 128 KB of distan
 constexpr int kLdsBlock = 256;    // vertices a wave scans at once
 constexpr int kLdsIlp = 4;        // arcs per lane and step
 constexpr int kLdsStep = kLdsIlp * SMDP_WAVE;
-constexpr int kLdsHeavy = 256;    // arcs from which a vertex is cut into chunks of kLdsStep arcs for all waves
-constexpr int kLdsChunks = 512;   // such chunks per round (later vertices are expanded by the wave that found them)
+constexpr int kLdsHeavy = 256;    // arcs from which a vertex is cut into chunks for all waves
+constexpr int kLdsHeavyFew = 64;  // the same where the scan blocks are too few for the waves: kLdsFew vertices
+constexpr int kLdsFew = 4 * kLdsBlock;
+constexpr int kLdsChunks = 512;   // such chunks per round
+constexpr int kLdsPieces = 128;   // chunks of one vertex, about, at most: of kLdsStep arcs below 32768 arcs, longer above
+constexpr int kLdsChunkBits = 17; // of a chunk's arcs
 constexpr int kLdsSeg = 2048;     // arcs whose begin bits a wave holds at once
 constexpr int kLdsList = SMDP_WAVE + kLdsBlock;  // selected vertices a wave holds
 constexpr int kLdsMaxCluster = 16;
@@ -58,6 +68,7 @@ constexpr int kLdsSpinLimit = 1 << 21;  // polls before a cluster barrier gives 
 constexpr float kLdsWindow = 7.0f;
 constexpr int32_t kLdsWeightLimit = 1 << 30;
 static_assert(kLdsVerts % kLdsBlock == 0 && kLdsVerts <= 65536, "whole blocks, 16-bit local ids");
+static_assert(kLdsVerts <= 1 << (32 - kLdsChunkBits), "a chunk's vertex and arcs share a word");
 static_assert(kLdsSeg % kLdsStep == 0 && kLdsSeg / 32 == SMDP_WAVE, "one mark word per lane, whole steps");
 
 struct LdsGraph {
@@ -81,7 +92,7 @@ struct LdsShared {
   int2 ent[kLdsWaves][SMDP_WAVE];        // per entry with arcs: (4 * (first arc - its offset), word)
   uint32_t mark[kLdsWaves][kLdsSeg / 32];
   uint16_t list[kLdsWaves][kLdsList];
-  int2 chunk[kLdsChunks];                // (4 * first arc, vertex << 16 | arcs)
+  int2 chunk[kLdsChunks];                // (4 * first arc, vertex << kLdsChunkBits | arcs)
   // Round r uses slot r % 3: written during it, read after its last barrier.
   // Fast waves may be a round ahead of the last reader, never two, so slot
   // (r + 1) % 3 is cleared as round r starts.
@@ -243,19 +254,27 @@ struct LdsSolver {
       // claims the vertex: lowered from here on it is active again
       x = __hip_atomic_fetch_and(&sh.x[u], ~1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    c.verts += cnt;
-    if (deg >= kLdsHeavy) {
-      const int nch = (deg + kLdsStep - 1) / kLdsStep;
+    bool back = false;
+    if (deg >= (nl <= kLdsFew ? kLdsHeavyFew : kLdsHeavy)) {
+      const int steps = (deg + kLdsStep - 1) / kLdsStep;
+      constexpr int kMost = ((1 << kLdsChunkBits) - 1) / kLdsStep;
+      const int each = steps <= kLdsPieces ? 1 : min((steps + kLdsPieces - 1) / kLdsPieces, kMost);
+      const int nch = each == 1 ? steps : (steps + each - 1) / each, len = each * kLdsStep;
       const int at = __hip_atomic_fetch_add(&sh.nchunk[slot], nch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (at + nch <= kLdsChunks) {
         for (int i = 0; i < nch; ++i)
-          sh.chunk[at + i] = make_int2(4 * (s + i * kLdsStep), (int)((uint32_t)u << 16) | min(kLdsStep, deg - i * kLdsStep));
-        deg = 0;
+          sh.chunk[at + i] =
+              make_int2(4 * (s + i * len), (int)((uint32_t)u << kLdsChunkBits) | min(len, deg - i * len));
       } else {
-        // no room: the slots below the limit stay empty
-        for (int i = at; i < kLdsChunks; ++i) sh.chunk[i] = make_int2(4 * s, (int)((uint32_t)u << 16));
+        // no room: active again, and the slots below the limit stay empty
+        for (int i = at; i < kLdsChunks; ++i) sh.chunk[i] = make_int2(4 * s, 0);
+        __hip_atomic_fetch_or(&sh.x[u], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        low = min(low, x | 1u);
+        back = true;
       }
+      deg = 0;
     }
+    c.verts += cnt - __popcll(__builtin_amdgcn_ballot_w64(back));
     const int incl = wave_scan_dpp(deg);
     const int off = incl - deg;
     const int T = __builtin_amdgcn_readlane(incl, SMDP_WAVE - 1);
@@ -332,19 +351,21 @@ struct LdsSolver {
   __device__ __forceinline__ void chunk_pass(int nch) {
     for (int h = wave; h < nch; h += kLdsWaves) {
       const int2 ch = sh.chunk[h];
-      const int len = __builtin_amdgcn_readfirstlane(ch.y & 0xFFFF);
+      const int len = __builtin_amdgcn_readfirstlane(ch.y & ((1 << kLdsChunkBits) - 1));
       if (!len) continue;
-      const uint32_t x = sh.x[(uint32_t)ch.y >> 16] | 1u;
+      const uint32_t x = sh.x[(uint32_t)ch.y >> kLdsChunkBits] | 1u;
       c.edges += len;
-      uint32_t q[kLdsIlp], from[kLdsIlp];
-      uint64_t ok[kLdsIlp];
+      for (int o = 0; o < len; o += kLdsStep) {
+        uint32_t q[kLdsIlp], from[kLdsIlp];
+        uint64_t ok[kLdsIlp];
 #pragma unroll
-      for (int t = 0; t < kLdsIlp; ++t) {
-        ok[t] = low_lanes(len - t * SMDP_WAVE);
-        q[t] = (uint32_t)ch.x + 4 * (uint32_t)min(t * SMDP_WAVE + lane, len - 1);
-        from[t] = x;
+        for (int t = 0; t < kLdsIlp; ++t) {
+          ok[t] = low_lanes(len - o - t * SMDP_WAVE);
+          q[t] = (uint32_t)ch.x + 4 * (uint32_t)min(o + t * SMDP_WAVE + lane, len - 1);
+          from[t] = x;
+        }
+        step(q, from, ok);
       }
-      step(q, from, ok);
     }
   }
 
@@ -458,9 +479,10 @@ struct LdsSolver {
     low = UINT32_MAX;
     int r = 0;
     for (;; ++r) {
-      // rounds with work number at most n, and a cluster's round may find
-      // only candidates that lowered nothing after one with work
-      if (r > 2 * g.n + 2) return kLdsRoundCap;
+      // rounds that settle a vertex number at most n; after each there may be
+      // one that overflowed the list of chunks, or in a cluster one that found
+      // only candidates that lowered nothing
+      if (r > (CL ? 4 : 2) * g.n + 2) return kLdsRoundCap;
       slot = r % 3;
       if (tid == 0) {
         const int next = (r + 1) % 3;
@@ -471,9 +493,9 @@ struct LdsSolver {
       publish_min();
       if (CL) __builtin_amdgcn_s_waitcnt(0);  // this wave's messages are stored
       __syncthreads();
-      const int nch = min(sh.nchunk[slot], kLdsChunks);
-      if (nch) {
-        chunk_pass(nch);
+      const int listed = sh.nchunk[slot];
+      if (listed) {
+        chunk_pass(min(listed, kLdsChunks));
         publish_min();
         if (CL) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -485,7 +507,7 @@ struct LdsSolver {
         if (mn < 0) return kLdsTimeout;
       }
       if (mn == INT32_MAX) break;
-      thr = min(mn + win, SMDP_SSSP_INF);
+      thr = min(mn + (listed > kLdsChunks ? 1 : win), SMDP_SSSP_INF);
     }
     for (int i = tid; i < nl; i += kLdsThreads) {
       const uint32_t x = sh.x[i];
