@@ -32,6 +32,7 @@ constexpr int kRoundWgs = 256;       // most workgroups (one per CU)
 constexpr int kRoundThreads = 1024;
 constexpr int kRoundOut = 8192;      // entries a workgroup keeps before they go to the queue
 constexpr int kRoundIlp = 2;         // arcs per thread and step
+constexpr int kTriedBits = 11;       // of the slots for candidates that a workgroup has tried
 
 // A workgroup's part of a queue: arcs before it and first entry in the high
 // and low half of at, entries in count.  Found with the queue's counters, it
@@ -130,12 +131,41 @@ struct RoundShared {
   unsigned long long base; // what the next queue held before them
   int count;               // the entries among them
   int ok;
+  uint64_t tried[1 << kTriedBits];  // vertex << 32 | candidate, at the vertex's tried_slot
   int v[kRoundOut], start[kRoundOut], before[kRoundOut];  // what the workgroup queued
 };
+
+__device__ __forceinline__ uint32_t tried_slot(int v) { return (uint32_t)v * 2654435761u >> (32 - kTriedBits); }
 
 struct RoundCount {
   uint32_t tries = 0, wins = 0, pushes = 0;
 };
+
+// A round's arcs read their targets before any of its atomics lands, so where
+// many lead to one vertex nearly all of them tried to lower it, one after
+// another: 200000 arcs into one vertex took BFS 1107 us and SSSP 603, into 64
+// vertices 468 and 293.  So of the lanes of a wave that want to lower the same
+// vertex only one with the lowest candidate stays, and every workgroup keeps
+// what it has tried: 59 and 76 us, 152 and 260.  (A vertex in RoundShared::tried
+// is only skipped for candidates that are no lower than one whose atomic was
+// issued, in this round or before.)
+// The first lanes' targets are looked at as long as kSameTarget lanes or more
+// share them: once, where they do not.  A round of fewer than kCrowdedArcs arcs
+// does without, since it costs 0.15 us of the 5 that such a round takes.
+constexpr int kSameTarget = 4;
+constexpr int kCrowdedArcs = 8192;
+__device__ __forceinline__ bool lowest_of_target(bool want, int v, int alt) {
+  for (uint64_t m = ballot(want); m;) {
+    const int target = __builtin_amdgcn_readlane(v, first_lane(m));
+    const bool same = want && v == target;
+    const uint64_t s = ballot(same);
+    if (__popcll(s) < kSameTarget) break;
+    m &= ~s;
+    const int lowest = __builtin_amdgcn_readlane(wave_min_dpp(same ? alt : INT32_MAX), SMDP_WAVE - 1);
+    if (same) want = lane_id() == first_lane(ballot(same && alt == lowest));
+  }
+  return want;
+}
 
 // Relaxes the window's arcs jb + K * thread + k below jend, K per thread.
 // Wave-uniform.  A thread's arcs follow one another, so one search finds them
@@ -144,7 +174,7 @@ struct RoundCount {
 // 334 (four arcs kRoundThreads apart, each with its search: 406, 113, 382).
 template <bool BFS, int K>
 __device__ __forceinline__ void round_arcs(const RoundArgs& a, RoundShared& sh, int jb, int jend, int top, int r,
-                                           RoundCount& n) {
+                                           bool crowded, RoundCount& n) {
   const int lane = lane_id();
   int j[K], own[K], v[K], alt[K], seen[K];
   const int j0 = jb + (int)threadIdx.x * K;
@@ -171,10 +201,27 @@ __device__ __forceinline__ void round_arcs(const RoundArgs& a, RoundShared& sh, 
   for (int k = 0; k < K; ++k) seen[k] = agent_load(a.dist + v[k]);
   // Only the atomic is under a condition: loads in a branch were waited for
   // there, slot after slot.  A lane without a candidate loads vertex 0's words.
-  int old[K], stamp[K], st[K], deg[K];
+  int old[K], stamp[K], st[K], deg[K], wants[K];
+  uint64_t tried[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const bool want = j0 + k < jend && alt[k] < seen[k];
+    wants[k] = j0 + k < jend && alt[k] < seen[k] ? 1 : 0;
+    tried[k] = ~0ull;
+  }
+  if (crowded) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      wants[k] = lowest_of_target(wants[k] != 0, v[k], alt[k]) ? 1 : 0;
+      tried[k] = __hip_atomic_load(&sh.tried[tried_slot(v[k])], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint64_t t = tried[k];
+    const bool want = wants[k] && ((int)(t >> 32) != v[k] || (int)(uint32_t)t > alt[k]);
+    if (want && crowded)
+      __hip_atomic_store(&sh.tried[tried_slot(v[k])], (uint64_t)(uint32_t)v[k] << 32 | (uint32_t)alt[k],
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     old[k] = INT32_MIN;
     if (want) old[k] = atomicMin(&a.dist[v[k]], alt[k]);
     v[k] = want ? v[k] : 0;
@@ -251,6 +298,7 @@ __global__ __launch_bounds__(kRoundThreads) void k_rounds(RoundArgs a, int32_t i
   const int lane = lane_id(), tid = threadIdx.x, b = blockIdx.x, G = gridDim.x;
   RoundCount n;
   unsigned long long edges = 0, verts = 0;
+  for (int i = tid; i < 1 << kTriedBits; i += kRoundThreads) sh.tried[i] = ~0ull;
   if (tid == 0) {
     sh.out = 0;
     sh.nent[0] = sh.nent[1] = 0;
@@ -346,10 +394,10 @@ __global__ __launch_bounds__(kRoundThreads) void k_rounds(RoundArgs a, int32_t i
           }
           room -= min(jend - jb, kRoundIlp * kRoundThreads);
           if (jend - jb > kRoundThreads) {
-            round_arcs<BFS, kRoundIlp>(a, sh, jb, jend, top, r, n);
+            round_arcs<BFS, kRoundIlp>(a, sh, jb, jend, top, r, A >= kCrowdedArcs, n);
             jb += kRoundIlp * kRoundThreads;
           } else {
-            round_arcs<BFS, 1>(a, sh, jb, jend, top, r, n);
+            round_arcs<BFS, 1>(a, sh, jb, jend, top, r, A >= kCrowdedArcs, n);
             jb += kRoundThreads;
           }
         }
