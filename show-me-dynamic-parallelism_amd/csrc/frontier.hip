@@ -619,9 +619,12 @@ __global__ __launch_bounds__(kLdsThreads) void k_lds_solve(LdsGraph g, Counters*
   if (threadIdx.x < 4) s_tot[threadIdx.x] = 0;
   unsigned long long* c = reinterpret_cast<unsigned long long*>(cnt);
   for (int i = threadIdx.x; i < (int)(kCntParts * sizeof(Counters) / 8); i += kLdsThreads) c[i] = 0;
+  if (g.rlog)
+    for (int i = threadIdx.x; i < 3 * kRoundLogCap; i += kLdsThreads) g.rlog[i] = 0;
+  __syncthreads();
   LdsCount k;
   LdsSolver<BFS, false> s(sh, g, k, 0, 1);
-  const int rounds = s.solve();
+  const int end = s.solve();
   __syncthreads();
   const unsigned long long v[4] = {k.edges, k.verts, k.wins, wave_sum(k.reached)};
   if (lane_id() == 0)
@@ -633,8 +636,8 @@ __global__ __launch_bounds__(kLdsThreads) void k_lds_solve(LdsGraph g, Counters*
     cnt->push[0] = s_tot[1] ? s_tot[1] - 1 : 0;  // every expanded vertex but the source was activated
     cnt->atom_try = cnt->atom_win = s_tot[2];
     cnt->reached = s_tot[3];
-    cnt->rounds = rounds > 0 ? rounds : 0;
-    cnt->done = rounds < 0 ? (unsigned long long)-rounds : 0;
+    cnt->rounds = s.rounds;
+    cnt->done = end < 0 ? (unsigned long long)-end : 0;
   }
 }
 
@@ -901,6 +904,25 @@ static bool use_lds(const smdp_params& p, const smdp_graph* g, bool bfs) {
          p.max_rounds >= 2 * g->n + 2;
 }
 
+// Reads the per-round log of k_rounds or k_lds_solve: queue lengths, arcs and clocks.
+static int collect_rounds_log(smdp_ctx* ctx, int rounds) {
+  const int k = std::min(rounds, kRoundLogCap - 1);
+  std::vector<unsigned long long> h(3 * (size_t)kRoundLogCap);
+  SMDP_HIP(hipMemcpy(h.data(), ctx->rlog, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost));
+  int khz = 0;
+  SMDP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+  ctx->log_qlen.assign(k, 0);
+  ctx->log_arcs.assign(k, 0);
+  ctx->log_ms.assign(k, 0.0);
+  for (int i = 0; i < k; ++i) {
+    ctx->log_qlen[i] = (int64_t)h[2 * i];
+    ctx->log_arcs[i] = (int64_t)h[2 * i + 1];
+    const unsigned long long* clock = h.data() + 2 * kRoundLogCap + i;
+    if (khz > 0) ctx->log_ms[i] = (double)(clock[1] - clock[0]) / khz;
+  }
+  return SMDP_OK;
+}
+
 // Returns kLdsWeight (and leaves the solve to the rounds) when a weight is out
 // of the LDS solve's range.
 static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
@@ -914,6 +936,7 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
   a.n = g->n;
   a.src = src;
   a.out = g->dist;
+  a.rlog = ctx->profiling ? ctx->rlog : nullptr;
   prof_reset(ctx);
   SMDP_HIP(hipEventRecord(ctx->ev_begin, s));
   SMDP_CHECK(prof_mark(ctx, 0));
@@ -924,14 +947,15 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
   SMDP_HIP(hipMemcpyAsync(ctx->pinned, g->cnt, kCntParts * sizeof(Counters), hipMemcpyDeviceToHost, s));
   SMDP_HIP(hipEventRecord(ctx->ev_end, s));
   SMDP_HIP(hipEventSynchronize(ctx->ev_end));
-  const int failed = (int)reinterpret_cast<const Counters*>(ctx->pinned)->done;
+  const Counters* c = reinterpret_cast<const Counters*>(ctx->pinned);
+  const int failed = (int)c->done, rounds = (int)c->rounds;
   if (failed == -kLdsWeight) return kLdsWeight;
   if (failed) return SMDP_ERR_OVERFLOW;
   float ms = 0;
   SMDP_HIP(hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end));
+  if (a.rlog) SMDP_CHECK(collect_rounds_log(ctx, rounds));
   ctx->counters_staged = st != nullptr;
-  return finish_frontier(g, g->row, bfs ? SMDP_BFS_UNDEF : SMDP_SSSP_INF, bfs, false, ms, 1,
-                         ctx->profiling ? 0 : -1, false, st, true);
+  return finish_frontier(g, g->row, bfs ? SMDP_BFS_UNDEF : SMDP_SSSP_INF, bfs, false, ms, 1, -1, false, st, true);
 }
 
 // Graphs whose rounds run in one launch (rounds.h), beyond those of use_lds.
@@ -950,25 +974,6 @@ static bool use_rounds(const smdp_params& p, const smdp_graph* g, bool bfs) {
   if (p.layout != SMDP_LAYOUT_AUTO) return false;
   if (g->hasout_mem) return g->n <= kRoundFixedN;  // the fixed array holds no larger queues
   return g->n <= kRoundMaxN && g->m <= (bfs ? kRoundMaxArcs : g->transient ? kRoundMaxArcsDropin : kRoundMaxArcsSssp);
-}
-
-// Reads the per-round log of k_rounds: queue lengths, arcs and clocks.
-static int collect_rounds_log(smdp_ctx* ctx, int rounds) {
-  const int k = std::min(rounds, kRoundLogCap - 1);
-  std::vector<unsigned long long> h(3 * (size_t)kRoundLogCap);
-  SMDP_HIP(hipMemcpy(h.data(), ctx->rlog, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost));
-  int khz = 0;
-  SMDP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
-  ctx->log_qlen.assign(k, 0);
-  ctx->log_arcs.assign(k, 0);
-  ctx->log_ms.assign(k, 0.0);
-  for (int i = 0; i < k; ++i) {
-    ctx->log_qlen[i] = (int64_t)h[2 * i];
-    ctx->log_arcs[i] = (int64_t)h[2 * i + 1];
-    const unsigned long long* clock = h.data() + 2 * kRoundLogCap + i;
-    if (khz > 0) ctx->log_ms[i] = (double)(clock[1] - clock[0]) / khz;
-  }
-  return SMDP_OK;
 }
 
 // How long a solve waits for the CUs that other contexts' launches hold before

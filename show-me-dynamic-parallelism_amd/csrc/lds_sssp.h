@@ -85,6 +85,8 @@ struct LdsGraph {
   const int64_t* moff;              // [k][k]: first message of the pair (sender, receiver), parity 0
   int64_t mtotal;                   // messages of one parity
   uint64_t* flags;                  // [2][k][k]: epoch << 55 | messages << 31 | smallest distance
+  // profiling: per counted round (vertices, arcs), then the rounds' starting clocks and the end's (zeroed), or nullptr
+  unsigned long long* rlog;
 };
 
 struct LdsShared {
@@ -98,6 +100,7 @@ struct LdsShared {
   // (r + 1) % 3 is cleared as round r starts.
   int32_t smin[3];                       // smallest active distance left
   int32_t nchunk[3];
+  int32_t work[3];                       // one workgroup: a wave relaxed arcs of its own vertices
   int32_t bad[3];                        // a weight outside [0, 2^30) was read
   int32_t mn;                            // cluster: smallest distance anywhere
   int32_t mcnt[kLdsMaxCluster];          // cluster: messages queued for each workgroup this round
@@ -159,6 +162,7 @@ struct LdsSolver {
   int rest;       // per lane: smallest word left active, rotated (see round_pass)
   uint32_t low;   // per lane: smallest candidate word that lowered a vertex
   int slot = 0;   // round % 3
+  int rounds = 0; // one workgroup: rounds that relaxed an arc, and the first
   int parity = 0;
 
   __device__ __forceinline__ LdsSolver(LdsShared& s, const LdsGraph& gg, LdsCount& cc, int rank_, int k_)
@@ -457,6 +461,20 @@ struct LdsSolver {
     return gmin;
   }
 
+  // Profiling: the wave's part of the last counted round (one without arcs
+  // joins the one before).
+  __device__ __forceinline__ void log_round(uint32_t verts0, unsigned long long edges0) {
+    if (rounds > kRoundLogCap || lane != 0) return;
+    const unsigned long long by[2] = {c.verts - verts0, c.edges - edges0};
+    for (int i = 0; i < 2; ++i)
+      if (by[i])
+        __hip_atomic_fetch_add(&g.rlog[2 * (rounds - 1) + i], by[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void log_clock() {
+    if (rounds < kRoundLogCap && threadIdx.x == 0 && !g.rlog[2 * kRoundLogCap + rounds])
+      g.rlog[2 * kRoundLogCap + rounds] = wall_clock64();
+  }
+
   // The solve; returns the rounds run or a result below 0.
   __device__ __forceinline__ int solve() {
     const int tid = threadIdx.x;
@@ -471,6 +489,7 @@ struct LdsSolver {
     if (tid < 3) {
       sh.smin[tid] = INT32_MAX;
       sh.nchunk[tid] = 0;
+      sh.work[tid] = 0;
       sh.bad[tid] = 0;
     }
     const int win = window(sh.got);
@@ -491,8 +510,13 @@ struct LdsSolver {
         const int next = (r + 1) % 3;
         sh.smin[next] = INT32_MAX;
         sh.nchunk[next] = 0;
+        sh.work[next] = 0;
       }
+      const uint32_t verts0 = c.verts;
+      const unsigned long long edges0 = c.edges;
+      if (!CL && g.rlog) log_clock();
       round_pass(thr);
+      if (!CL && c.edges != edges0) sh.work[slot] = 1;
       publish_min();
       if (CL) __builtin_amdgcn_s_waitcnt(0);  // this wave's messages are stored
       __syncthreads();
@@ -503,6 +527,11 @@ struct LdsSolver {
         if (CL) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
       }
+      if (!CL) {
+        // (vertices without arcs are not queued in rounds of other kinds, and make no round here)
+        if (r == 0 || listed || sh.work[slot]) ++rounds;
+        if (g.rlog) log_round(verts0, edges0);
+      }
       int mn = sh.smin[slot];
       if (!BFS && !CL && sh.bad[slot]) return kLdsWeight;  // (clusters are given weights in range)
       if (CL) {
@@ -512,6 +541,7 @@ struct LdsSolver {
       if (mn == INT32_MAX) break;
       thr = min(mn + (listed > kLdsChunks ? 1 : win), SMDP_SSSP_INF);
     }
+    if (!CL && g.rlog) log_clock();
     for (int i = tid; i < nl; i += kLdsThreads) {
       const uint32_t x = sh.x[i];
       g.out[lo + i] = x == inf ? (BFS ? SMDP_BFS_UNDEF : SMDP_SSSP_INF) : (int)(x >> 1);
