@@ -128,7 +128,8 @@ typedef struct {
                                   falling in-degree (built once per resident graph; results are reported in the
                                   caller's numbering).  Automatic picks it for BFS on resident graphs of more than
                                   2^25 arcs (or 2^23 vertices); smaller ones are solved on the graph as given, in one
-                                  launch. */
+                                  launch.  A call on host or device arrays has no copy to run on: for it this layout
+                                  and BUCKETS are AUTO. */
 #define SMDP_LAYOUT_BUCKETS 4  /* SSSP tuned: bucketed rounds (delta-stepping) on the renumbered copy.  Vertices are
                                   taken in order of distance buckets of width delta; within a bucket, arcs that stay in
                                   the bucket are relaxed until no distance in it changes, then every other arc of the

@@ -889,6 +889,16 @@ static int finish_frontier(smdp_graph* g, const int32_t* row, int32_t inf, bool 
   return SMDP_OK;
 }
 
+// A graph uploaded or handed over for one call has no renumbered copy, so the
+// layouts that name one mean nothing there: parameters that were set or tuned
+// for a resident graph of the same context do not take the faster solves from
+// the others (drop-in SSSP of uniform 16384 x 8 under BUCKETS: @A@ us with the
+// host-driven rounds, 276 now).
+static bool auto_layout(const smdp_params& p, const smdp_graph* g) {
+  return p.layout == SMDP_LAYOUT_AUTO ||
+         (g->transient && (p.layout == SMDP_LAYOUT_HOT || p.layout == SMDP_LAYOUT_BUCKETS));
+}
+
 // Graphs that one workgroup solves in LDS: all distances fit, and the arcs,
 // read by one CU, cost less than the launches of the rounds they replace.
 // Measured (device time, rounds against LDS): SSSP uniform 1024 x 8 180 / 39
@@ -900,7 +910,7 @@ static int finish_frontier(smdp_graph* g, const int32_t* row, int32_t inf, bool 
 constexpr int32_t kLdsMaxArcs = 3 << 17;
 constexpr int32_t kLdsMaxArcsBfs = 3 << 16;
 static bool use_lds(const smdp_params& p, const smdp_graph* g, bool bfs) {
-  return p.layout == SMDP_LAYOUT_AUTO && g->n <= kLdsVerts && g->m <= (bfs ? kLdsMaxArcsBfs : kLdsMaxArcs) &&
+  return auto_layout(p, g) && g->n <= kLdsVerts && g->m <= (bfs ? kLdsMaxArcsBfs : kLdsMaxArcs) &&
          p.max_rounds >= 2 * g->n + 2;
 }
 
@@ -971,7 +981,7 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
 // not needed either.  Drop-in SSSP of 2^22 arcs and more keeps the rounds that
 // the host drives, whose launches its statistics report.
 static bool use_rounds(const smdp_params& p, const smdp_graph* g, bool bfs) {
-  if (p.layout != SMDP_LAYOUT_AUTO) return false;
+  if (!auto_layout(p, g)) return false;
   if (g->hasout_mem) return g->n <= kRoundFixedN;  // the fixed array holds no larger queues
   return g->n <= kRoundMaxN && g->m <= (bfs ? kRoundMaxArcs : g->transient ? kRoundMaxArcsDropin : kRoundMaxArcsSssp);
 }
