@@ -891,9 +891,9 @@ static int finish_frontier(smdp_graph* g, const int32_t* row, int32_t inf, bool 
 
 // A graph uploaded or handed over for one call has no renumbered copy, so the
 // layouts that name one mean nothing there: parameters that were set or tuned
-// for a resident graph of the same context do not take the faster solves from
-// the others (drop-in SSSP of uniform 16384 x 8 under BUCKETS: @A@ us with the
-// host-driven rounds, 276 now).
+// for a resident graph of the same context keep no other call from the faster
+// solves (drop-in SSSP of uniform 16384 x 8 under BUCKETS: 517 us a call with
+// the host-driven rounds, 276 now).
 static bool auto_layout(const smdp_params& p, const smdp_graph* g) {
   return p.layout == SMDP_LAYOUT_AUTO ||
          (g->transient && (p.layout == SMDP_LAYOUT_HOT || p.layout == SMDP_LAYOUT_BUCKETS));
