@@ -292,9 +292,14 @@ int  smdp_batch_autotune(smdp_batch* b, smdp_params* chosen);
 
 /* ---- autotuner --------------------------------------------------------------*/
 /* Times candidate parameter sets of SMDP_SOL_TUNED for `app` on the resident
- * graph and installs the fastest in the context.  cache_path (may be NULL) is a
- * JSON file keyed by GPU arch and the graph's degree histogram; a hit skips the
- * search.  For SSSP/BFS `src` is the probe source. */
+ * graph and installs the fastest in the context; the context's own parameters
+ * (for SSSP with the automatic layout) stay unless another set is faster by
+ * more than 2 %.  cache_path (may be NULL) is a JSON file keyed by GPU arch, the
+ * graph's degree histogram and the kernel that the automatic layout runs; a hit
+ * skips the search.  For SSSP/BFS `src` is the probe source.  An SSSP graph of at
+ * most 32768 vertices and 393216 arcs is solved in LDS without parameters and
+ * needs no tuning: its search chooses a layout (BUCKETS or HOT) for larger
+ * resident graphs, which the small graph then uses too. */
 int smdp_autotune(smdp_graph* gr, int app, int32_t src, const char* cache_path,
                   smdp_params* chosen);
 

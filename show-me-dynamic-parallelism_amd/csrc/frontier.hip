@@ -986,6 +986,12 @@ static bool use_rounds(const smdp_params& p, const smdp_graph* g, bool bfs) {
   return g->n <= kRoundMaxN && g->m <= (bfs ? kRoundMaxArcs : g->transient ? kRoundMaxArcsDropin : kRoundMaxArcsSssp);
 }
 
+// The route of a tuned solve with weights in range and memory for its queues.
+FrontierRoute frontier_route(const smdp_params& p, const smdp_graph* g, bool bfs) {
+  if (use_lds(p, g, bfs)) return FrontierRoute::kLds;
+  return use_rounds(p, g, bfs) ? FrontierRoute::kRounds : FrontierRoute::kHost;
+}
+
 // How long a solve waits for the CUs that other contexts' launches hold before
 // it goes to the host-driven rounds, which need none of their own: a few solves
 // of the kind (0.03 to 1 ms), and no longer than what it would then lose.

@@ -613,6 +613,11 @@ static bool use_binned(const smdp_params& p, int sol, const smdp_graph* g) {
   return p.layout == SMDP_LAYOUT_BINNED || (p.layout == SMDP_LAYOUT_AUTO && g->m > (1 << 22));
 }
 
+// A tuned PageRank on merge tiles.
+bool pagerank_by_merge(const smdp_params& p, const smdp_graph* g) {
+  return !use_binned(p, SMDP_SOL_TUNED, g) && !use_blocks(p, SMDP_SOL_TUNED, g->n) && merge_pagerank_fits(g->n, g->m);
+}
+
 template <bool PR>
 static void launch_pass(int sol, int grid, hipStream_t s, const RArgs& a, int k, int* launches, smdp_ctx* ctx) {
   dim3 g(grid), b(SMDP_WG);

@@ -35,6 +35,10 @@ constexpr int32_t kRoundMaxArcsDropin = (1 << 22) - 1;
 // Entries of one queue: the vertices with arcs, and a source without.
 inline int64_t round_queue_cap(int64_t n, int64_t m) { return std::min(n, m + 1); }
 
+// What a tuned SSSP or BFS runs as: one workgroup in LDS, every round in one
+// launch, or rounds (or bucketed phases) that the host drives.
+enum class FrontierRoute { kHost, kLds, kRounds };
+
 struct Ctl {
   int32_t qlen;        // frontier entries of this round
   int32_t hlen;        // grid-queue entries pushed during this round
