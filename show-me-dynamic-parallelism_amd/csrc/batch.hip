@@ -1347,25 +1347,33 @@ static int batch_plan(smdp_batch* b, const smdp_params& p, bool clusters = true)
   }
   const int grid = std::max<int>(1, std::min<int>(wgs, nteamwg + (int)plan.single.size()));
   int rc = SMDP_OK;
+  // (an allocation or copy takes about 10 us, a whole call on one small graph
+  // 350: a plan without teams has none of theirs)
   auto up32 = [&](int32_t** d, const int32_t* h, int64_t cnt) {
-    if (rc != SMDP_OK) return;
-    rc = alloc_once(d, std::max<int64_t>(1, cnt));
-    if (rc == SMDP_OK && h && cnt > 0 &&
+    if (rc != SMDP_OK || cnt == 0) return;
+    rc = alloc_once(d, cnt);
+    if (rc == SMDP_OK && h &&
         hipMemcpy(*d, h, sizeof(int32_t) * (size_t)cnt, hipMemcpyHostToDevice) != hipSuccess)
       rc = SMDP_ERR_DEVICE;
   };
   up32(&b->d_order, plan.single.data(), (int64_t)plan.single.size());
   up32(&b->d_team, team.data(), nteamwg);
-  up32(&b->d_tbase, plan.base.data(), nteams + 1);
-  up32(&b->d_tfirst, tfirst.data(), nteams + 1);
+  up32(&b->d_tbase, plan.base.data(), nteams ? nteams + 1 : 0);
+  up32(&b->d_tfirst, tfirst.data(), nteams ? nteams + 1 : 0);
   up32(&b->d_gctl, nullptr, (int64_t)nitems * kMgGroupLine);
   if (rc != SMDP_OK) return rc;
-  SMDP_CHECK(alloc_once(&b->d_lds, ng));
-  SMDP_HIP(hipMemcpy(b->d_lds, plan.lds.data(), (size_t)ng, hipMemcpyHostToDevice));
-  SMDP_CHECK(alloc_once(&b->d_items, std::max<int32_t>(1, nitems)));
-  if (nitems) SMDP_HIP(hipMemcpy(b->d_items, items.data(), sizeof(MgItem) * items.size(), hipMemcpyHostToDevice));
-  SMDP_CHECK(alloc_once(&b->d_cflags, std::max<int64_t>(1, nflags)));
-  SMDP_CHECK(alloc_once(&b->d_moff, std::max<int64_t>(1, nmoff)));
+  if (lds) {
+    SMDP_CHECK(alloc_once(&b->d_lds, ng));
+    SMDP_HIP(hipMemcpy(b->d_lds, plan.lds.data(), (size_t)ng, hipMemcpyHostToDevice));
+  }
+  if (nitems) {
+    SMDP_CHECK(alloc_once(&b->d_items, nitems));
+    SMDP_HIP(hipMemcpy(b->d_items, items.data(), sizeof(MgItem) * items.size(), hipMemcpyHostToDevice));
+  }
+  if (nmoff) {
+    SMDP_CHECK(alloc_once(&b->d_cflags, nflags));
+    SMDP_CHECK(alloc_once(&b->d_moff, nmoff));
+  }
   GArgs& a = b->args;
   a.row = b->d_row;
   a.col = b->d_col;
