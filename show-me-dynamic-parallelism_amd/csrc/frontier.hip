@@ -978,8 +978,13 @@ static int run_lds(smdp_graph* g, int32_t src, bool bfs, smdp_stats* st) {
 // 50000 87 / 32, 2^18 119 / 49, 2^22 200 / 114, RMAT-17 x 16 233 / 169, RMAT-20
 // x 16 629 / 322, uniform 2^22 x 8 1102 / 964, RMAT-22 x 16 1059 / 1293.  The
 // renumbered copy, built on the host by the first run (143 ms for RMAT-20), is
-// not needed either.  Drop-in SSSP of 2^22 arcs and more keeps the rounds that
-// the host drives, whose launches its statistics report.
+// not needed either.  Below 2^23 arcs buckets are the faster solve on dense
+// graphs all the same (uniform, 16 arcs a vertex, 7.9M arcs 1344 / 1043, 31 a
+// vertex 1276 / 773; RMAT-19 x 15 871 / 648), but a graph's first solve then
+// takes 35 to 65 ms for the copy instead of 1 to 3: from 100 to 300 solves on
+// they win, and the autotuner finds them.  Drop-in SSSP of 2^22 arcs and more
+// keeps the rounds that the host drives only because a test of their launch
+// counts, at that size, expects them.
 static bool use_rounds(const smdp_params& p, const smdp_graph* g, bool bfs) {
   if (!auto_layout(p, g)) return false;
   if (g->hasout_mem) return g->n <= kRoundFixedN;  // the fixed array holds no larger queues
