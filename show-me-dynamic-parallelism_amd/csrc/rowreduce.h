@@ -158,17 +158,21 @@ __device__ __forceinline__ CSum wg_csum(CSum v, float2* lds) {
 template <bool PR>
 __device__ __forceinline__ CSum wave_row(const RArgs& a, int s, int e) {
   CSum acc;
-  int k = s + lane_id();
+  const int32_t* col = a.col + s;
+  const float* val = PR ? nullptr : a.val + s;
+  // unsigned offsets: a row may end at arc 2^31 - 1, and steps go past its end
+  const uint32_t len = (uint32_t)(e - s);
+  uint32_t k = (uint32_t)lane_id();
   // four steps' loads are issued before their terms are added (same order)
-  for (; k + 3 * SMDP_WAVE < e; k += 4 * SMDP_WAVE) {
+  for (; k + 3 * SMDP_WAVE < len; k += 4 * SMDP_WAVE) {
     int c[4];
     float g[4], va[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) c[t] = stream_load(a.col + k + t * SMDP_WAVE);
+    for (int t = 0; t < 4; ++t) c[t] = stream_load(col + k + t * SMDP_WAVE);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       g[t] = a.x[c[t]];
-      va[t] = PR ? 0.f : stream_load(a.val + k + t * SMDP_WAVE);
+      va[t] = PR ? 0.f : stream_load(val + k + t * SMDP_WAVE);
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -176,7 +180,7 @@ __device__ __forceinline__ CSum wave_row(const RArgs& a, int s, int e) {
       else acc.add_prod(va[t], g[t]);
     }
   }
-  for (; k < e; k += SMDP_WAVE) add_term<PR>(a, acc, k);
+  for (; k < len; k += SMDP_WAVE) add_term<PR>(a, acc, s + (int)k);
   acc = wave_csum(acc);
   CSum out;
   out.s = __shfl(acc.s, 0);
@@ -188,17 +192,20 @@ __device__ __forceinline__ CSum wave_row(const RArgs& a, int s, int e) {
 template <bool PR>
 __device__ __forceinline__ CSum wg_row(const RArgs& a, int s, int e, float2* lds) {
   CSum acc;
-  int k = s + (int)threadIdx.x;
+  const int32_t* col = a.col + s;
+  const float* val = PR ? nullptr : a.val + s;
+  const uint32_t len = (uint32_t)(e - s);  // as in wave_row
+  uint32_t k = threadIdx.x;
   // four independent gathers per step, added in arc order
-  for (; k + 3 * SMDP_WG < e; k += 4 * SMDP_WG) {
+  for (; k + 3 * SMDP_WG < len; k += 4 * SMDP_WG) {
     int c[4];
     float g[4], va[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) c[t] = stream_load(a.col + k + t * SMDP_WG);
+    for (int t = 0; t < 4; ++t) c[t] = stream_load(col + k + t * SMDP_WG);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       g[t] = a.x[c[t]];
-      va[t] = PR ? 0.f : stream_load(a.val + k + t * SMDP_WG);
+      va[t] = PR ? 0.f : stream_load(val + k + t * SMDP_WG);
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -206,7 +213,7 @@ __device__ __forceinline__ CSum wg_row(const RArgs& a, int s, int e, float2* lds
       else acc.add_prod(va[t], g[t]);
     }
   }
-  for (; k < e; k += SMDP_WG) add_term<PR>(a, acc, k);
+  for (; k < len; k += SMDP_WG) add_term<PR>(a, acc, s + (int)k);
   return wg_csum(acc, lds);
 }
 
