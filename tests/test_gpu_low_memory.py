@@ -1,6 +1,7 @@
 """Calls that take extra device memory for speed, with the device nearly full:
-they go on without it and stay exact.  torch fills the device."""
+they go on without it and stay exact."""
 import contextlib
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -8,31 +9,39 @@ import pytest
 import orc
 import smdp
 from conftest import random_graph
+from test_zz_no_alloc import hip
 
-torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 MB = 1 << 20
 
 
+def _free():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
 @contextlib.contextmanager
 def device_left(mb):
     """About mb MB of device memory are free inside (within 16 MB below)."""
-    def free():
-        return torch.cuda.mem_get_info(0)[0]
-
     fill = []
+
+    def take(nbytes):
+        p = C.c_void_p()
+        assert hip().hipMalloc(C.byref(p), C.c_size_t(nbytes)) == 0
+        fill.append(p)
+
     try:
-        torch.cuda.empty_cache()
-        while free() > (mb + 1100) * MB:
-            fill.append(torch.empty(free() - (mb + 1024) * MB, dtype=torch.uint8, device="cuda:0"))
-        while free() > mb * MB:
-            fill.append(torch.empty(16 * MB, dtype=torch.uint8, device="cuda:0"))
-        print(f"device memory left: {free() // MB} MB", flush=True)
+        while _free() > (mb + 1100) * MB:
+            take(_free() - (mb + 1024) * MB)
+        while _free() > mb * MB:
+            take(16 * MB)
+        print(f"device memory left: {_free() // MB} MB", flush=True)
         yield
     finally:
-        fill.clear()
-        torch.cuda.empty_cache()
+        for p in fill:
+            hip().hipFree(p)
 
 
 def test_batch_without_memory_for_messages(ctx):
@@ -82,9 +91,9 @@ def test_multi_source_without_memory_for_bounds(ctx):
         return st
 
     with smdp.Graph(ctx, g) as dg:
-        before = torch.cuda.mem_get_info(0)[0]
+        before = _free()
         solve(dg)
-        used = before - torch.cuda.mem_get_info(0)[0]
+        used = before - _free()
     print(f"multi-source: {used // MB} MB", flush=True)
     with smdp.Graph(ctx, g) as dg:
         with device_left(used // MB - 6):
