@@ -21,9 +21,10 @@
 //    Rows of at least kBinWide arcs have a bin of their own, cut into pieces;
 //    the last workgroup merges each wide row's piece sums in order.
 // Per arc and iteration the passes move 2 + 4 bytes (scatter) and 4 + 2 bytes
-// (reduce).  Results do not depend on the schedule: every light row is summed
-// in in-CSR arc order by one thread, every heavy row by one wave in a fixed
-// lane order, and every partial is combined in a fixed order.
+// (reduce).  Results do not depend on the schedule: rows of fewer than 8 arcs
+// are summed in in-CSR arc order by one thread, rows of 8 to 63 by 8 lanes and
+// longer ones by a wave, each in a fixed lane order, and every partial is
+// combined in a fixed order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -28,7 +28,7 @@
 
 namespace smdp {
 
-constexpr int kRoundWgs = 256;       // most workgroups (one per CU)
+constexpr int kRoundWgs = 256;       // most workgroups (a launch has at most three quarters of the CUs)
 constexpr int kRoundThreads = 1024;
 constexpr int kRoundOut = 8192;      // entries a workgroup keeps before they go to the queue
 constexpr int kRoundIlp = 2;         // arcs per thread and step
