@@ -1293,10 +1293,14 @@ static void batch_plan_free(smdp_batch* b) {
 }
 
 // Work plan of a batch for parameters p (host/batch_plan.h), and its hipGraph
-// (reset + solve), replacing the previous plan.  A workgroup's fair share is
-// the batch's arcs over the grid (p.wg_per_cu workgroups per CU, at most 2;
-// one where graphs are solved in LDS), of which p.group_share percent sizes
-// the teams.  The workgroups of teams are resident at once; the rest of the
+// (reset + solve), replacing the previous plan.  The launch has a workgroup per
+// graph, at least one per CU, and at most p.wg_per_cu (1 or 2) per CU, or one
+// where graphs are solved in LDS.  p.group_share percent of a workgroup's fair
+// share of the batch's arcs sizes the teams.
+// (Teams that fill two workgroups per CU are slower, in memory: 30 graphs of
+// 32000 arcs 0.66 ms, one per CU 0.39, 0.39 without teams; of 512000 arcs 2.4,
+// 1.8 and 6.6 ms; 400 of 32000 arcs, teams of two for some, 1.41, 1.07 without.)
+// The workgroups of teams are resident at once; the rest of the
 // graphs are claimed one per workgroup, largest first.
 // 256 graphs, 85M arcs: 6.8 ms with distances in memory and groups, 0.64 ms in
 // LDS with clusters (0.95 ms when a cluster's messages were placed by one LDS
@@ -1312,12 +1316,12 @@ static int batch_plan(smdp_batch* b, const smdp_params& p, bool clusters = true)
   const int max_cluster = clusters ? kLdsMaxCluster : 1;
   bool lds = false;
   for (int32_t i = 0; i < ng; ++i) lds = lds || (b->fit[(size_t)i] && b->nv[i] <= kLdsVerts * max_cluster);
-  const int wgs = ctx->cus * (lds ? 1 : std::max(1, std::min(2, p.wg_per_cu)));
+  const int wgs = std::max(ctx->cus, std::min(ng, ctx->cus * (lds ? 1 : std::max(1, std::min(2, p.wg_per_cu)))));
   int per_cu = 0;
   const void* kernel = lds ? reinterpret_cast<const void*>(k_mg<kMgThreads, true>)
                            : reinterpret_cast<const void*>(k_mg<kMgThreads, false>);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMgThreads, 0) != hipSuccess) per_cu = 0;
-  const BatchLimits lim{kLdsVerts, max_cluster, kMgMaxGroup, std::min(wgs, per_cu * ctx->cus),
+  const BatchLimits lim{kLdsVerts, max_cluster, kMgMaxGroup, std::min(wgs, per_cu * ctx->cus), wgs,
                         (double)b->etot / wgs * (p.group_share > 0 ? p.group_share : 100) / 100.0};
   const BatchPlan plan = plan_batch(b->nv, b->m, b->fit, lim);
   const int32_t nteams = (int32_t)plan.base.size() - 1, nitems = (int32_t)plan.items.size();

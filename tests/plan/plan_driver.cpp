@@ -20,7 +20,7 @@ int main() {
     m[i] = arcs;
     fit[i] = (uint8_t)f;
   }
-  const smdp::BatchPlan p = smdp::plan_batch(nv, m, fit, smdp::BatchLimits{32768, cluster, 16, resident, share});
+  const smdp::BatchPlan p = smdp::plan_batch(nv, m, fit, smdp::BatchLimits{32768, cluster, 16, resident, resident, share});
   printf("base");
   for (int32_t b : p.base) printf(" %d", b);
   printf("\n");

@@ -79,3 +79,20 @@ def test_edges_of_one_workgroup(driver):
         assert (len(single) == 1) == (k == 0) and (k == 0 or base[1] == k), n
     _, items, single = _plan(driver, [(16 * V + 1, 10, True), (10, 0, True)], share=10)
     assert not items and sorted(single) == [(0, 0), (1, 1)]
+
+
+@pytest.mark.parametrize("count,resident,team", [(400, 512, 0), (512, 512, 0), (600, 512, 0), (255, 256, 0), (128, 256, 0),
+                                                 (127, 256, 2), (100, 256, 2), (30, 256, 8), (4, 256, 16)])
+def test_equal_graphs_in_memory_do_not_ask_for_more_workgroups_than_there_are(driver, count, resident, team):
+    base, items, single = _plan(driver, [(4000, 32000, False)] * count, resident)
+    if team:
+        assert len(items) == count and set(np.diff(base)) == {team}
+    else:
+        assert not items and len(single) == count
+    _, items, _ = _plan(driver, [(1000, 1 << 14, False)] * count, resident)
+    assert not items  # too small for a team
+
+
+def test_graphs_above_the_mean_get_teams_in_memory(driver):
+    base, items, single = _plan(driver, [(90000, 900000, False)] * 3 + [(2000, 20000, False)] * 250)
+    assert sorted(g for g, _, _ in items) == [0, 1, 2] and set(np.diff(base)) == {16} and len(single) == 250
