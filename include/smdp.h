@@ -120,7 +120,9 @@ typedef struct {
 #define SMDP_SETTLE_PULL 2
 
 /* Arc layouts of the tuned SpMV/PageRank solution (smdp_params.layout). */
-#define SMDP_LAYOUT_AUTO    0  /* PageRank: BINNED when the graph has more than 2^22 arcs, else CSR; SpMV: CSR */
+#define SMDP_LAYOUT_AUTO    0  /* PageRank: BINNED when the graph has more than 2^22 arcs, or stays on the
+                                  device with more than 2^21 arcs and 2^14 rows and arcs per CU, else CSR;
+                                  SpMV: CSR */
 #define SMDP_LAYOUT_CSR     1  /* gather from the in-CSR as given */
 #define SMDP_LAYOUT_BINNED  2  /* PageRank only: arcs regrouped once per graph by (source chunk, row bin); each
                                   iteration is two streaming passes through LDS instead of random gathers */

@@ -606,11 +606,20 @@ static bool use_blocks(const smdp_params& p, int sol, int32_t) {
 // The binned layout replaces every random gather of a PageRank iteration by
 // streamed runs, which pays where the gathers miss L2.  Against merge-path
 // tiles, microseconds an iteration: RMAT-16 x 16 40 / 26, RMAT-17 x 16 48 /
-// 34, RMAT-18 x 16 (2^22 arcs) 62 / 61, RMAT-19 x 16 78 / 101.  Its plan, built
-// on the host by the first run, takes 19 ms for 2^22 arcs.
+// 34, RMAT-18 x 16 (2^22 arcs) 61 / 62, RMAT-19 x 16 78 / 101.  Its plan, built
+// on the host by the first run, takes 19 ms for 2^22 arcs, so one solve of a
+// drop-in call takes it only above 2^22 arcs.  A graph that stays takes it from
+// where the largest merge tiles, two to a CU, no longer run all at once: 12
+// iterations of 2^20 vertices, uniform, 3.0M arcs (4.05M items) 759 us binned /
+// 612 by tiles, 3.5M 787 / 891, 4.2M 814 / 913; of 2^21 vertices 2.0M arcs 841 /
+// 675, 2.5M 848 / 938, 4.2M 899 / 1109; RMAT-19 x 8 748 / 805.  Graphs with few
+// arcs stay on tiles: 2^22 vertices 1.2M arcs 1116 / 989, 2.0M 1105 / 1091, 3.0M
+// 1100 / 1214.
 static bool use_binned(const smdp_params& p, int sol, const smdp_graph* g) {
   if (sol != SMDP_SOL_TUNED) return false;
-  return p.layout == SMDP_LAYOUT_BINNED || (p.layout == SMDP_LAYOUT_AUTO && g->m > (1 << 22));
+  if (p.layout != SMDP_LAYOUT_AUTO) return p.layout == SMDP_LAYOUT_BINNED;
+  const int64_t at_once = (int64_t)g->ctx->cus << 14;  // merge items of two tiles per CU
+  return g->m > (1 << 22) || (!g->transient && g->m > (1 << 21) && (int64_t)g->n + g->m > at_once);
 }
 
 // A tuned PageRank on merge tiles.
@@ -904,6 +913,7 @@ int smdp_pagerank_f32(smdp_ctx* ctx, const smdp_csr* in_csr, const int32_t* outd
   smdp_csr c = *in_csr;
   c.w = nullptr;
   SMDP_CHECK(smdp_graph_create(ctx, &c, &g));
+  g->transient = true;
   int rc = smdp_graph_set_outdeg(g, outdeg);
   if (rc == SMDP_OK) rc = run_pagerank(g, opt, solution, st);
   if (rc == SMDP_OK) rc = smdp_graph_read(g, SMDP_RES_RANK, rank, g->n);
