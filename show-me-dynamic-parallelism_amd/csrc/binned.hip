@@ -232,9 +232,9 @@ __device__ __forceinline__ void bin_load(const RArgs& a, const BArgs& b, const i
 // before it are summed, so the memory has work during the sums.  Rows are
 // summed in FP64 (two instructions per arc, where a compensated FP32 sum
 // takes seven), and only a wave that holds an end of the bin tests its arcs
-// one by one.  On RMAT-22 (67M arcs) a pass went from 136 to 126 us: 4 TB/s
-// over the 500 MB of arcs and rows it moves; without the sums it takes 113,
-// without LDS stores as well 112.  Two workgroups per CU need at most 128
+// one by one.  On RMAT-22 (67M arcs) a pass went from 136 to 126 us, and by
+// another 13 when the last bins were no longer loaded twice: 4 TB/s over the
+// 458 MB of arcs and rows it moves.  Two workgroups per CU need at most 128
 // registers (one took 157 us): hence the scalar descriptors and the 32-bit
 // offsets.
 __global__ __launch_bounds__(kBinNT, 4) void k_bin_reduce(RArgs a, BArgs b, int k) {
@@ -336,12 +336,12 @@ __global__ __launch_bounds__(kBinNT, 4) void k_bin_reduce(RArgs a, BArgs b, int 
     __syncthreads();
     it = it1;
     it1 = __builtin_amdgcn_readfirstlane(s_next);
-    // after the last bin its own loads are made again (a load under a condition
-    // kept the registers of both sides)
-    if (it < nitems) {
-      d0 = e0;
-      d1 = e1;
-    }
+    // After the last bin the loads are those of an empty one, all lanes at one
+    // place (a load under a condition kept the registers of both sides).  With
+    // the last bin's own loads made again a graph of one bin a workgroup read
+    // its arcs twice: 18 iterations of RMAT-19 x 9 took 1142 us, now 998.
+    d0 = it < nitems ? e0 : make_int4(beg, beg, r0, 1);
+    if (it < nitems) d1 = e1;
     // for the epilogue of this bin, and the next one's loads
     float rold[kRowsPerThread];
     int od[kRowsPerThread];

@@ -606,15 +606,15 @@ static bool use_blocks(const smdp_params& p, int sol, int32_t) {
 // The binned layout replaces every random gather of a PageRank iteration by
 // streamed runs, which pays where the gathers miss L2.  Against merge-path
 // tiles, microseconds an iteration: RMAT-16 x 16 40 / 26, RMAT-17 x 16 48 /
-// 34, RMAT-18 x 16 (2^22 arcs) 61 / 62, RMAT-19 x 16 78 / 101.  Its plan, built
+// 34, RMAT-18 x 16 (2^22 arcs) 55 / 62, RMAT-19 x 16 62 / 101.  Its plan, built
 // on the host by the first run, takes 19 ms for 2^22 arcs, so one solve of a
 // drop-in call takes it only above 2^22 arcs.  A graph that stays takes it from
 // where the largest merge tiles, two to a CU, no longer run all at once: 12
-// iterations of 2^20 vertices, uniform, 3.0M arcs (4.05M items) 759 us binned /
-// 612 by tiles, 3.5M 787 / 891, 4.2M 814 / 913; of 2^21 vertices 2.0M arcs 841 /
-// 675, 2.5M 848 / 938, 4.2M 899 / 1109; RMAT-19 x 8 748 / 805.  Graphs with few
-// arcs stay on tiles: 2^22 vertices 1.2M arcs 1116 / 989, 2.0M 1105 / 1091, 3.0M
-// 1100 / 1214.
+// iterations of 2^20 vertices, uniform, 3.0M arcs (4.05M items) 678 us binned /
+// 609 by tiles, 3.5M 677 / 883, 4.2M 692 / 901; of 2^21 vertices 2.0M arcs 789 /
+// 676, 2.5M 806 / 929, 4.2M 842 / 1111; RMAT-19 x 8 662 / 804.  Graphs with few
+// arcs stay on tiles: 2^22 vertices 1.2M arcs 1092 / 986, 2.0M 1077 / 1090, 3.0M
+// 1087 / 1214.
 static bool use_binned(const smdp_params& p, int sol, const smdp_graph* g) {
   if (sol != SMDP_SOL_TUNED) return false;
   if (p.layout != SMDP_LAYOUT_AUTO) return p.layout == SMDP_LAYOUT_BINNED;
