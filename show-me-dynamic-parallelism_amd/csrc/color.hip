@@ -1108,19 +1108,18 @@ __global__ __launch_bounds__(kLayerThreads) void k_layer_short(LArgs a) {
       if (lane == 0) pushes += __popcll(m);
       if (won) {
         a.color[v] = r + 2;
-        if (at < a.seg_cap) store_entry(out + at, v, st, en - st, pv);
-      }
-      // What the segment has no place for, with one atomic a wave: a hub may
-      // release most of the graph at once (a star of 10^6 leaves with random
-      // priorities, its hub among the first: 11.4 ms a call with an atomic for
-      // each vertex, 1.0 so).
-      const bool over = won && at >= a.seg_cap;
-      const uint64_t om = ballot(over);
-      if (om) {
-        int o = 0;
-        if (lane == 0) o = atomicAdd(&cout->qlen, __popcll(om));
-        o = __builtin_amdgcn_readfirstlane(o) + mbcnt(om);
-        if (over) qover[o] = v;
+        if (at < a.seg_cap) {
+          store_entry(out + at, v, st, en - st, pv);
+        } else {
+          // What the segment has no place for, with one atomic for the lanes
+          // here: a hub may release most of the graph at once (a star of 10^6
+          // leaves with random priorities, its hub among the first: 11.4 ms a
+          // call with an atomic for each vertex, 1.0 so).
+          const uint64_t om = ballot(true);
+          int o = 0;
+          if (lane == first_lane(om)) o = atomicAdd(&cout->qlen, __popcll(om));
+          qover[__builtin_amdgcn_readfirstlane(o) + mbcnt(om)] = v;
+        }
       }
     }
     ++r;
